@@ -406,6 +406,72 @@ void solve_columns(dm_ctx* ctx, const dm_solve_opts& o, const dm_rwg& r, DevOp* 
   }
 }
 
+// Dense LU of z's complex128 matrix and the solution of the nrhs columns of Bd
+// (device, internal basis order, n x nrhs) into host X (caller order).  Up to
+// kLuRhs right-hand sides are carried through the factorization as further
+// columns; more take a forward substitution of their own per block.
+constexpr i64 kLuRhs = 1024;
+void solve_direct(dm_ctx* ctx, const dm_rwg& r, const dm_zmat* z, const double* Bd, i64 nrhs, bool conj_out,
+                  double* X, i64 ldx, bool name_pivot, double t0, dm_solve_stats& st, double& worst) {
+  hipStream_t s = ctx->stream;
+  const i64 n = z->n, ld = z->ld, R0 = std::min(nrhs, kLuRhs);
+  DBuf<double> A, x, xe, tmp, nr;
+  DBuf<int> ipiv, status;
+  DBuf<char> ws;
+  A.alloc((size_t)2 * ld * (n + R0));
+  HIP_OK(hipMemcpyAsync(A.p, z->z64.p, (size_t)16 * ld * n, hipMemcpyDeviceToDevice, s));
+  double* Y = A.p + (size_t)2 * ld * n;
+  auto put_rhs = [&](i64 j0, i64 R) {
+    if (R > 0)
+      HIP_OK(hipMemcpy2DAsync(Y, 16 * ld, Bd + 2 * n * j0, 16 * n, 16 * n, R, hipMemcpyDeviceToDevice, s));
+  };
+  put_rhs(0, R0);
+  ipiv.alloc(n);
+  status.alloc(1);
+  HIP_OK(hipMemsetAsync(status.p, 0, sizeof(int), s));
+  dml::lu_factor(n, ld, A.p, R0, ipiv.p, status.p, s);
+  int sv = 0;
+  HIP_OK(hipMemcpyAsync(&sv, status.p, sizeof(int), hipMemcpyDeviceToHost, s));
+  HIP_OK(hipStreamSynchronize(s));
+  DM_REQUIRE(sv == 0, DM_ERR_ARGUMENT,
+             "dense LU: matrix is singular" + (name_pivot ? " (zero pivot " + std::to_string(sv) + ")" : std::string()));
+  st.precond_time_s = now() - t0;
+  if (nrhs <= 0) return;
+  x.alloc((size_t)2 * n * R0);
+  xe.alloc((size_t)2 * n * R0);
+  OpZ64 op(z);
+  const i64 RB = std::min(R0, kMfmaMaxRhs);
+  tmp.alloc((size_t)2 * n * RB);
+  ws.alloc(std::max<size_t>(op.batch_ws((int)RB), 1));
+  nr.alloc(2 * RB);
+  std::vector<double> h(2 * RB);
+  for (i64 j0 = 0; j0 < nrhs; j0 += kLuRhs) {
+    const i64 R = std::min(kLuRhs, nrhs - j0);
+    if (j0) {
+      put_rhs(j0, R);
+      dml::lu_forward(n, ld, A.p, ipiv.p, Y, ld, R, s);
+    }
+    dml::lu_back(n, ld, A.p, Y, ld, x.p, n, R, s);
+    launch_permute_cols(n, R, r.d_ext.p, x.p, n, xe.p, n, 0, conj_out, s);
+    HIP_OK(hipMemcpy2DAsync(X + 2 * ldx * j0, 16 * ldx, xe.p, 16 * n, 16 * n, R, hipMemcpyDeviceToHost, s));
+    // relative true residuals of the block, column by column
+    for (i64 q = 0; q < R; q += RB) {
+      const int w = (int)std::min(RB, R - q);
+      const double* b = Bd + 2 * n * (j0 + q);
+      op.apply_batch(x.p + 2 * n * q, tmp.p, w, ws.p, s);
+      dml::axpby(n * w, 1, 0, b, -1, 0, tmp.p, s);
+      dmb::norm2(n, w, tmp.p, nullptr, nr.p, s);
+      dmb::norm2(n, w, b, nullptr, nr.p + RB, s);
+      HIP_OK(hipMemcpyAsync(h.data(), nr.p, sizeof(double) * 2 * RB, hipMemcpyDeviceToHost, s));
+      HIP_OK(hipStreamSynchronize(s));
+      for (int c = 0; c < w; ++c) {
+        const double rr = h[c], bb = h[RB + c];
+        worst = std::max(worst, bb == 0 ? (rr == 0 ? 0.0 : INFINITY) : std::sqrt(rr / bb));
+      }
+    }
+  }
+}
+
 void validate_opts(const dm_solve_opts& o) {
   DM_REQUIRE(std::isfinite(o.tol) && o.tol > 0, DM_ERR_ARGUMENT, "GMRES tol must be finite and positive");
   DM_REQUIRE(o.maxiter >= 1 && o.maxiter <= 1000, DM_ERR_ARGUMENT, "maxiter must be in [1, 1000]");
@@ -1380,30 +1446,7 @@ int dm_solve_scattering_pw(dm_ctx* ctx, const dm_rwg* rwg_c, double k_re, double
     double worst = 0;
     bool all_ok = true;
     if (o.method == DM_METHOD_LU) {
-      DBuf<double> A;
-      DBuf<int> ipiv, status;
-      A.alloc((size_t)2 * z->ld * n);
-      HIP_OK(hipMemcpyAsync(A.p, z->z64.p, A.bytes(), hipMemcpyDeviceToDevice, s));
-      ipiv.alloc(n);
-      status.alloc(1);
-      HIP_OK(hipMemsetAsync(status.p, 0, sizeof(int), s));
-      dml::lu_factor(n, z->ld, A.p, ipiv.p, status.p, s);
-      int sv = 0;
-      HIP_OK(hipMemcpyAsync(&sv, status.p, sizeof(int), hipMemcpyDeviceToHost, s));
-      HIP_OK(hipStreamSynchronize(s));
-      DM_REQUIRE(sv == 0, DM_ERR_ARGUMENT, "dense LU: matrix is singular");
-      st.precond_time_s = now() - t1;
-      DBuf<double> tmp, hb;
-      tmp.alloc(2 * n);
-      hb.alloc(4);
-      for (i64 j = 0; j < nrhs; ++j) {
-        double* bj = V.p + 2 * n * j;
-        HIP_OK(hipMemcpyAsync(x.p, bj, 16 * n, hipMemcpyDeviceToDevice, s));
-        dml::lu_solve(n, z->ld, A.p, ipiv.p, x.p, n, 1, s);
-        worst = std::max(worst, true_residual(*A64, n, bj, x.p, tmp.p, hb.p, s));
-        launch_permute(n, r.d_ext.p, x.p, xe.p, 0, s);
-        HIP_OK(hipMemcpyAsync(X + 2 * n * j, xe.p, 16 * n, hipMemcpyDeviceToHost, s));
-      }
+      solve_direct(ctx, r, z.get(), V.p, nrhs, false, X, n, false, t1, st, worst);
     } else {
       auto M = build_precond(z.get(), pick_form(z.get(), o.method == DM_METHOD_MIXED, batched), o, s);
       HIP_OK(hipStreamSynchronize(s));
@@ -1450,42 +1493,18 @@ int dm_solve(dm_ctx* ctx, const dm_zmat* z, const double* B, int64_t ldb, int64_
     hipStream_t s = ctx->stream;
     const dm_rwg& r = *z->rwg;
     dm_solve_stats st{};
-    DBuf<double> be, b, x, tmp, hb;
-    be.alloc(2 * n);
-    b.alloc(2 * n);
-    x.alloc(2 * n);
-    tmp.alloc(2 * n);
-    hb.alloc(4);
     double t0 = now();
     if (o.method == DM_METHOD_LU) {
       DM_REQUIRE(z->forms & DM_Z64, DM_ERR_ARGUMENT, "dense LU needs the complex128 matrix");
-      DBuf<double> A, bb;
-      DBuf<int> ipiv, status;
-      A.alloc((size_t)2 * z->ld * n);
-      HIP_OK(hipMemcpyAsync(A.p, z->z64.p, A.bytes(), hipMemcpyDeviceToDevice, s));
-      ipiv.alloc(n);
-      status.alloc(1);
-      HIP_OK(hipMemsetAsync(status.p, 0, sizeof(int), s));
-      dml::lu_factor(n, z->ld, A.p, ipiv.p, status.p, s);
-      int sv = 0;
-      HIP_OK(hipMemcpyAsync(&sv, status.p, sizeof(int), hipMemcpyDeviceToHost, s));
-      HIP_OK(hipStreamSynchronize(s));
-      DM_REQUIRE(sv == 0, DM_ERR_ARGUMENT, "dense LU: matrix is singular (zero pivot " + std::to_string(sv) + ")");
-      st.precond_time_s = now() - t0;
-      OpZ64 A64(z);
-      double worst = 0;
-      for (i64 j = 0; j < nrhs; ++j) {
-        HIP_OK(hipMemcpyAsync(be.p, B + 2 * ldb * j, 16 * n, hipMemcpyHostToDevice, s));
-        if (o.adjoint) dml::conj(n, be.p, s);
-        launch_permute(n, r.d_ext.p, be.p, b.p, 1, s);
-        HIP_OK(hipMemcpyAsync(x.p, b.p, 16 * n, hipMemcpyDeviceToDevice, s));
-        dml::lu_solve(n, z->ld, A.p, ipiv.p, x.p, n, 1, s);
-        worst = std::max(worst, true_residual(A64, n, b.p, x.p, tmp.p, hb.p, s));
-        launch_permute(n, r.d_ext.p, x.p, be.p, 0, s);
-        if (o.adjoint) dml::conj(n, be.p, s);
-        HIP_OK(hipMemcpyAsync(X + 2 * ldx * j, be.p, 16 * n, hipMemcpyDeviceToHost, s));
+      DBuf<double> Bx, Bd;
+      Bx.alloc((size_t)2 * n * nrhs);
+      Bd.alloc((size_t)2 * n * nrhs);
+      if (nrhs > 0) {
+        HIP_OK(hipMemcpy2DAsync(Bx.p, 16 * n, B, 16 * ldb, 16 * n, nrhs, hipMemcpyHostToDevice, s));
+        launch_permute_cols(n, nrhs, r.d_ext.p, Bx.p, n, Bd.p, n, 1, o.adjoint != 0, s);
       }
-      HIP_OK(hipStreamSynchronize(s));
+      double worst = 0;
+      solve_direct(ctx, r, z, Bd.p, nrhs, o.adjoint != 0, X, ldx, true, t0, st, worst);
       st.solved = 1;
       st.residual = worst;
       st.solve_time_s = now() - t0 - st.precond_time_s;
@@ -1506,7 +1525,8 @@ int dm_solve(dm_ctx* ctx, const dm_zmat* z, const double* B, int64_t ldb, int64_
     if (f32) A32 = make_op(z, o.method == DM_METHOD_MIXED ? op_form(z, batched) : f32);
     bool all_ok = true;
     double worst = 0;
-    DBuf<double> Bd;
+    DBuf<double> be, Bd;
+    be.alloc(2 * n);
     Bd.alloc((size_t)2 * n * std::max<i64>(nrhs, 1));
     for (i64 j = 0; j < nrhs; ++j) {
       HIP_OK(hipMemcpyAsync(be.p, B + 2 * ldb * j, 16 * n, hipMemcpyHostToDevice, s));

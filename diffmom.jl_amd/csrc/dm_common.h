@@ -410,4 +410,8 @@ void launch_gemv_z32(i64 n, i64 ld, const float* z, const double* x, double* y, 
 
 // small vector kernels
 void launch_permute(i64 n, const int* idx, const double* src, double* dst, int gather, hipStream_t s);
+// the same for ncols columns (leading dimensions lds, ldd) in one launch,
+// optionally conjugated
+void launch_permute_cols(i64 n, i64 ncols, const int* idx, const double* src, i64 lds, double* dst, i64 ldd,
+                         int gather, bool conj, hipStream_t s);
 void launch_cast_c128_to_c64_matrix(i64 n, i64 ld, const double* src, float* dst, hipStream_t s);

@@ -22,8 +22,14 @@ void block_inverse(int bs, int nb, double* blocks, int* status, hipStream_t s);
 void block_apply(i64 n, int bs, int nb, const double* inv, const double* x, double* y, hipStream_t s);
 void diag_inv(i64 n, const ZRef& z, double* d, hipStream_t s);
 void diag_apply(i64 n, const double* d, const double* x, double* y, hipStream_t s);
-void lu_factor(i64 n, i64 ld, double* A, int* ipiv, int* status, hipStream_t s);
-void lu_solve(i64 n, i64 ld, const double* A, const int* ipiv, double* B, i64 ldb, int nrhs, hipStream_t s);
+// Dense LU (k_lu.hip).  lu_factor: A holds n + nrhs columns (leading dimension
+// ld); the first n become the factors (ipiv: 0-based exchanges in order,
+// *status: 1 + the first column without a pivot), the others L^-1 P B.
+// lu_forward makes further right-hand sides L^-1 P B; lu_back solves U X = Y
+// (Y is overwritten).
+void lu_factor(i64 n, i64 ld, double* A, i64 nrhs, int* ipiv, int* status, hipStream_t s);
+void lu_forward(i64 n, i64 ld, const double* A, const int* ipiv, double* B, i64 ldb, i64 nrhs, hipStream_t s);
+void lu_back(i64 n, i64 ld, const double* A, double* Y, i64 ldy, double* X, i64 ldx, i64 nrhs, hipStream_t s);
 // entries of one stored form; rows / columns of out in caller order via iofe
 void unpermute(i64 n, const ZRef& z, i64 c0, i64 nc, const int* iofe, double* out, hipStream_t s);
 void entries(const ZRef& z, i64 count, const int* iofe, const i64* m, const i64* n, double* out, hipStream_t s);
