@@ -188,8 +188,9 @@ struct SpaiPattern {
   double mean_radius = 0;  // mean over columns of the radius J_j covers
   i64 capped = 0;          // columns whose cap left bases within the cutoff out
   i64 nnz = 0;
-  std::vector<int> jptr, jidx, iptr, iidx;   // per column: support J_j, rows I_j
-  std::vector<int> rowptr, colidx, map;      // CSR of M and CSR position -> CSC position
+  int max_cols = 0;        // widest support
+  // per column: support J_j (jptr, jidx), rows I_j (iptr, iidx); CSR of M
+  // (rowptr, colidx) and CSR position -> CSC position (map)
   DBuf<int> d_jptr, d_jidx, d_iptr, d_iidx, d_rowptr, d_colidx, d_map;
 };
 
@@ -335,6 +336,10 @@ std::shared_ptr<const SpaiPattern> spai_pattern(dm_rwg& r, double cutJ, int maxJ
 
 namespace dmp {
 int spai_max_cols();
+// The pattern's device arrays and figures for the n centres (internal order);
+// false where the host form has to build it (k_pattern.hip).
+bool spai_pattern_device(i64 n, const double* centres, double mean_len, double cutJ, int maxJ, SpaiPattern& P,
+                         hipStream_t s);
 // maxJ: widest column support of the pattern (<= spai_max_cols())
 void spai_build(i64 n, const ZRef& z, int maxJ, const int* jptr, const int* jidx, const int* iptr, const int* iidx,
                 double* vals, int* status, hipStream_t s);

@@ -400,14 +400,14 @@ void finalize_rwg(dm_rwg& r) {
 // within 1.6 x the radius actually covered by J_j (at most 512 nearest).
 // Centres are the midpoints of the two triangle centroids
 // (rwg_centers, src/solver/NearFieldPreconditioner.jl:247-257).
+// The device form (k_pattern.hip) builds the same lists; this one serves meshes
+// it refuses (more than 1024 bases at practically one distance, ...).
 // The hash grid's cells are sized to the radius the maxJ nearest bases cover
 // on a surface of this mesh's mean edge (~2.7 mean edges for 80), not to the
 // cutoff, so a cutoff of a wavelength does not make every column scan the
 // whole mesh; a column whose J or I radius reaches past the scanned cells is
 // scanned again over a wider block of cells.
-std::shared_ptr<const SpaiPattern> spai_pattern(dm_rwg& r, double cutJ, int maxJ) {
-  std::lock_guard<std::mutex> lk(r.tab_mu);
-  if (r.spai && r.spai->cutJ == cutJ) return r.spai;
+static std::shared_ptr<SpaiPattern> spai_pattern_host(dm_rwg& r, double cutJ, int maxJ) {
   auto P = std::make_shared<SpaiPattern>();
   P->cutJ = cutJ;
   i64 n = r.n;
@@ -423,8 +423,8 @@ std::shared_ptr<const SpaiPattern> spai_pattern(dm_rwg& r, double cutJ, int maxJ
                                (long)std::floor((c[3 * i + 2] - lo[2]) / cell)};
   };
   for (i64 i = 0; i < n; ++i) grid[key(i)].push_back((int)i);
-  P->jptr.assign(n + 1, 0);
-  P->iptr.assign(n + 1, 0);
+  std::vector<int> jptr(n + 1, 0), jidx, iptr(n + 1, 0), iidx;  // per column: support J_j, rows I_j
+  std::vector<int> rowptr, colidx, map;  // CSR of M and CSR position -> CSC position
   std::vector<std::pair<double, int>> cand;
   double rsum = 0;
   i64 capped = 0;
@@ -478,37 +478,48 @@ std::shared_ptr<const SpaiPattern> spai_pattern(dm_rwg& r, double cutJ, int maxJ
     }
     std::sort(J.begin(), J.end());
     std::sort(I.begin(), I.end());
-    P->jidx.insert(P->jidx.end(), J.begin(), J.end());
-    P->iidx.insert(P->iidx.end(), I.begin(), I.end());
-    P->jptr[j + 1] = (int)P->jidx.size();
-    P->iptr[j + 1] = (int)P->iidx.size();
+    jidx.insert(jidx.end(), J.begin(), J.end());
+    iidx.insert(iidx.end(), I.begin(), I.end());
+    jptr[j + 1] = (int)jidx.size();
+    iptr[j + 1] = (int)iidx.size();
+    P->max_cols = std::max(P->max_cols, (int)J.size());
   }
   P->mean_radius = rsum / (double)std::max<i64>(n, 1);
   P->capped = capped;
-  P->nnz = (i64)P->jidx.size();
+  P->nnz = (i64)jidx.size();
   // CSR of M by transposing the CSC support lists
-  P->rowptr.assign(n + 1, 0);
-  for (int rr : P->jidx) P->rowptr[rr + 1]++;
-  for (i64 i = 0; i < n; ++i) P->rowptr[i + 1] += P->rowptr[i];
-  P->colidx.resize(P->nnz);
-  P->map.resize(P->nnz);
-  std::vector<int> fill(P->rowptr.begin(), P->rowptr.end() - 1);
+  rowptr.assign(n + 1, 0);
+  for (int rr : jidx) rowptr[rr + 1]++;
+  for (i64 i = 0; i < n; ++i) rowptr[i + 1] += rowptr[i];
+  colidx.resize(P->nnz);
+  map.resize(P->nnz);
+  std::vector<int> fill(rowptr.begin(), rowptr.end() - 1);
   for (i64 j = 0; j < n; ++j)
-    for (int p = P->jptr[j]; p < P->jptr[j + 1]; ++p) {
-      int rr = P->jidx[p];
+    for (int p = jptr[j]; p < jptr[j + 1]; ++p) {
+      int rr = jidx[p];
       int q = fill[rr]++;
-      P->colidx[q] = (int)j;
-      P->map[q] = p;
+      colidx[q] = (int)j;
+      map[q] = p;
     }
   hipStream_t s = r.ctx->stream;
-  P->d_jptr.upload(P->jptr, s);
-  P->d_jidx.upload(P->jidx, s);
-  P->d_iptr.upload(P->iptr, s);
-  P->d_iidx.upload(P->iidx, s);
-  P->d_rowptr.upload(P->rowptr, s);
-  P->d_colidx.upload(P->colidx, s);
-  P->d_map.upload(P->map, s);
+  P->d_jptr.upload(jptr, s);
+  P->d_jidx.upload(jidx, s);
+  P->d_iptr.upload(iptr, s);
+  P->d_iidx.upload(iidx, s);
+  P->d_rowptr.upload(rowptr, s);
+  P->d_colidx.upload(colidx, s);
+  P->d_map.upload(map, s);
   HIP_OK(hipStreamSynchronize(s));
+  return P;
+}
+
+std::shared_ptr<const SpaiPattern> spai_pattern(dm_rwg& r, double cutJ, int maxJ) {
+  std::lock_guard<std::mutex> lk(r.tab_mu);
+  if (r.spai && r.spai->cutJ == cutJ) return r.spai;
+  auto P = std::make_shared<SpaiPattern>();
+  P->cutJ = cutJ;
+  if (!dmp::spai_pattern_device(r.n, r.cen_i.data(), r.mean_len, cutJ, maxJ, *P, r.ctx->stream))
+    P = spai_pattern_host(r, cutJ, maxJ);
   r.spai = P;
   return P;
 }
