@@ -2,7 +2,7 @@
 // preconditioner's message-passing network (layout and equations in k_mpnn.h).
 //
 // Training products with the samples' matrices A = Z S are small (n up to a
-// few thousand): a row per thread for A y, a wave per row for A^H q.
+// few thousand): 16 rows per workgroup for A y, four rows per wave for A^H q.
 //
 // Layers run 64 nodes per workgroup: the layer's two 64 x 64 weight matrices
 // (bfloat16 in memory, widened to FP32 in LDS, rows padded to 65 floats), the
@@ -391,70 +391,100 @@ __global__ void k_add(i64 n, const double2* __restrict__ a, const double2* __res
   if (i < n) out[i] = make_double2(a[i].x + b[i].x, a[i].y + b[i].y);
 }
 
-// out[:, c] = A x[:, c] for c < k: one row per thread, the row's k sums in
-// FP64; A is read down its columns, which a wave reads as consecutive rows.
+// out[:, c] = A x[:, c] for c < k, FP64 sums: 16 rows per workgroup, its 16
+// waves and the four 16-lane groups of a wave over the columns j of A (64 at a
+// time, 128 contiguous bytes of A per group), the 64 partial sums of a row
+// added in a fixed order.  Bound by FP64 issue and L2 latency: 25 us for n =
+// 1278, k = 6 (a row per thread left all but five CUs idle: 1.13 ms).
+constexpr int AC_ROWS = 16, AC_WAVES = 16;
 template <int KMAX, class TX>
-__global__ __launch_bounds__(256) void k_acols(i64 n, int k, const float2* __restrict__ A, const TX* __restrict__ x,
-                                               double2* __restrict__ out) {
-  const i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x;
-  if (i >= n) return;
+__global__ __launch_bounds__(64 * AC_WAVES) void k_acols(i64 n, int k, const float2* __restrict__ A,
+                                                         const TX* __restrict__ x, double2* __restrict__ out) {
+  __shared__ double2 part[AC_WAVES][KMAX][AC_ROWS];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane & (AC_ROWS - 1);
+  const i64 i0 = blockIdx.x * (i64)AC_ROWS, i = min(i0 + row, n - 1);
   double ar[KMAX], ai[KMAX];
 #pragma unroll
   for (int c = 0; c < KMAX; ++c) ar[c] = ai[c] = 0.0;
-  for (i64 j = 0; j < n; ++j) {
+#pragma unroll 2
+  for (i64 j = 4 * wave + lane / AC_ROWS; j < n; j += 4 * AC_WAVES) {
     const float2 af = A[i + j * n];
     const double zr = af.x, zi = af.y;
+    TX xv[KMAX];
+#pragma unroll
+    for (int c = 0; c < KMAX; ++c) xv[c] = x[j + min(c, k - 1) * n];  // clamped: no load behind a branch
 #pragma unroll
     for (int c = 0; c < KMAX; ++c) {
-      if (c < k) {
-        const TX xv = x[j + c * n];
-        const double xr = xv.x, xi = xv.y;
-        ar[c] += zr * xr - zi * xi;
-        ai[c] += zr * xi + zi * xr;
-      }
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < KMAX; ++c)
-    if (c < k) out[i + c * n] = make_double2(ar[c], ai[c]);
-}
-
-// out[:, c] = A^H x[:, c] for c < k: one wave per output row i (column i of
-// A, read contiguously by the lanes), FP64 lane sums reduced across the wave.
-template <int KMAX>
-__global__ __launch_bounds__(256) void k_acols_adj(i64 n, int k, const float2* __restrict__ A,
-                                                   const float2* __restrict__ x, double2* __restrict__ out) {
-  const i64 i = blockIdx.x * (i64)(blockDim.x >> 6) + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (i >= n) return;
-  double ar[KMAX], ai[KMAX];
-#pragma unroll
-  for (int c = 0; c < KMAX; ++c) ar[c] = ai[c] = 0.0;
-  const float2* col = A + i * n;
-  for (i64 j = lane; j < n; j += 64) {
-    const float2 af = col[j];
-    const double zr = af.x, zi = -(double)af.y;
-#pragma unroll
-    for (int c = 0; c < KMAX; ++c) {
-      if (c < k) {
-        const float2 xv = x[j + c * n];
-        ar[c] += zr * xv.x - zi * xv.y;
-        ai[c] += zr * xv.y + zi * xv.x;
-      }
+      const double xr = xv[c].x, xi = xv[c].y;
+      ar[c] += zr * xr - zi * xi;
+      ai[c] += zr * xi + zi * xr;
     }
   }
 #pragma unroll
   for (int c = 0; c < KMAX; ++c) {
-    for (int o = 32; o > 0; o >>= 1) {
+#pragma unroll
+    for (int o = 16; o < 64; o <<= 1) {
       ar[c] += __shfl_xor(ar[c], o, 64);
       ai[c] += __shfl_xor(ai[c], o, 64);
     }
+    if (lane < AC_ROWS) part[wave][c][row] = make_double2(ar[c], ai[c]);
   }
-  if (lane == 0) {
+  __syncthreads();
+  if (threadIdx.x < KMAX * AC_ROWS) {
+    const int c = threadIdx.x / AC_ROWS, q = threadIdx.x % AC_ROWS;
+    double sr = 0, si = 0;
 #pragma unroll
-    for (int c = 0; c < KMAX; ++c)
-      if (c < k) out[i + c * n] = make_double2(ar[c], ai[c]);
+    for (int w = 0; w < AC_WAVES; ++w) {
+      sr += part[w][c][q].x;
+      si += part[w][c][q].y;
+    }
+    if (c < k && i0 + q < n) out[i0 + q + c * n] = make_double2(sr, si);
   }
+}
+
+// out[:, c] = A^H x[:, c] for c < k, FP64 lane sums: four output rows (columns
+// of A, read contiguously by the lanes) per wave, which share the reads of x;
+// the wave's 2 x 4 KMAX = 64 sums are reduced by one transposing butterfly
+// (each step halves the values a lane holds), lane l ends with sum l.
+template <int KMAX>
+__global__ __launch_bounds__(256) void k_acols_adj(i64 n, int k, const float2* __restrict__ A,
+                                                   const float2* __restrict__ x, double2* __restrict__ out) {
+  constexpr int AR = 4;
+  static_assert(2 * AR * KMAX == 64, "one sum per lane");
+  const i64 i0 = (blockIdx.x * (i64)4 + (threadIdx.x >> 6)) * AR;
+  const int lane = threadIdx.x & 63;
+  if (i0 >= n) return;
+  double v[64];  // [row][c][re, im]
+#pragma unroll
+  for (int q = 0; q < 64; ++q) v[q] = 0.0;
+  for (i64 j = lane; j < n; j += 64) {
+    float2 af[AR], xv[KMAX];
+#pragma unroll
+    for (int r = 0; r < AR; ++r) af[r] = A[j + min(i0 + r, n - 1) * n];
+#pragma unroll
+    for (int c = 0; c < KMAX; ++c) xv[c] = x[j + min(c, k - 1) * n];
+#pragma unroll
+    for (int r = 0; r < AR; ++r) {
+      const double zr = af[r].x, zi = -(double)af[r].y;
+#pragma unroll
+      for (int c = 0; c < KMAX; ++c) {
+        v[2 * (r * KMAX + c)] += zr * xv[c].x - zi * xv[c].y;
+        v[2 * (r * KMAX + c) + 1] += zr * xv[c].y + zi * xv[c].x;
+      }
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const bool hi = (lane & o) != 0;
+#pragma unroll
+    for (int q = 0; q < o; ++q) {
+      const double send = hi ? v[q] : v[q + o], keep = hi ? v[q + o] : v[q];
+      v[q] = keep + __shfl_xor(send, o, 64);
+    }
+  }
+  const double im = __shfl_xor(v[0], 1, 64);
+  const int r = lane / (2 * KMAX), c = lane % (2 * KMAX) / 2;
+  if ((lane & 1) == 0 && c < k && i0 + r < n) out[i0 + r + c * n] = make_double2(v[0], im);
 }
 
 __global__ void k_gather_c64(i64 n, const double2* __restrict__ a, const int* __restrict__ iofe,
@@ -505,7 +535,7 @@ template <class TX>
 void acols(i64 n, int k, const float* A, const TX* x, double* out, hipStream_t s) {
   for (int c0 = 0; c0 < k; c0 += ZC_K) {
     const int kk = std::min(ZC_K, k - c0);
-    k_acols<ZC_K, TX><<<nb256(n), 256, 0, s>>>(n, kk, reinterpret_cast<const float2*>(A), x + (i64)c0 * n,
+    k_acols<ZC_K, TX><<<(unsigned)((n + AC_ROWS - 1) / AC_ROWS), 64 * AC_WAVES, 0, s>>>(n, kk, reinterpret_cast<const float2*>(A), x + (i64)c0 * n,
                                                reinterpret_cast<double2*>(out) + (i64)c0 * n);
   }
 }
@@ -513,7 +543,7 @@ void acols(i64 n, int k, const float* A, const TX* x, double* out, hipStream_t s
 void acols_adj(i64 n, int k, const float* A, const float2* x, double* out, hipStream_t s) {
   for (int c0 = 0; c0 < k; c0 += ZC_K) {
     const int kk = std::min(ZC_K, k - c0);
-    k_acols_adj<ZC_K><<<(unsigned)((n + 3) / 4), 256, 0, s>>>(n, kk, reinterpret_cast<const float2*>(A),
+    k_acols_adj<ZC_K><<<(unsigned)((n + 15) / 16), 256, 0, s>>>(n, kk, reinterpret_cast<const float2*>(A),
                                                               x + (i64)c0 * n,
                                                               reinterpret_cast<double2*>(out) + (i64)c0 * n);
   }
