@@ -5,9 +5,9 @@
 // few thousand): 16 rows per workgroup for A y, four rows per wave for A^H q.
 //
 // Layers run 64 nodes per workgroup: the layer's two 64 x 64 weight matrices
-// (bfloat16 in memory, widened to FP32 in LDS, rows padded to 65 floats), the
-// nodes' hidden states and their aggregated neighbour messages are staged in
-// LDS; each of the 256 threads produces 16 outputs of one node.  Weight
+// (bfloat16 in memory, widened to FP32 in LDS), the nodes' hidden states and
+// their aggregated neighbour messages are staged in LDS; each of the 256
+// threads produces four outputs of four nodes.  Weight
 // gradients are sums of per-node outer products, reduced per workgroup into
 // FP32 partials and across workgroups in FP64 (fixed order).
 #include <hip/hip_runtime.h>
@@ -115,61 +115,88 @@ __global__ void k_encode(i64 n, const float* __restrict__ u, const uint16_t* __r
   h[idx] = acc;
 }
 
-// h_out = h + tanh(W_s h + W_n m + b), m_i = dinv_i sum_q sgn_iq h_{nbr_iq}
+// The two 64 x 64 matrices of a layer, widened to FP32, transposed to
+// [input][output] rows of TP floats (16-byte reads of four outputs).
+constexpr int TP = H + 4;
+__device__ inline void stage_weights(const uint16_t* __restrict__ prm, float (*ws)[TP], float (*wn)[TP], bool transpose) {
+  for (int e = threadIdx.x; e < H * H; e += 256) {
+    const int o = e / H, k = e % H;
+    const float a = bf(prm[e]), b = bf(prm[H * H + e]);
+    if (transpose) {
+      ws[k][o] = a;
+      wn[k][o] = b;
+    } else {
+      ws[o][k] = a;
+      wn[o][k] = b;
+    }
+  }
+}
+
+// h_out = h + tanh(W_s h + W_n m + b), m_i = dinv_i sum_q sgn_iq h_{nbr_iq}.
+// Each thread forms 4 nodes x 4 outputs from 16-byte LDS reads (four of the
+// weights' outputs, one value of each node: 10 reads for 32 FMAs), so the FMAs
+// and not the LDS pipe bound it: 30 us for 46 000 nodes (a node x 16 outputs
+// per thread read LDS once per FMA, and the missing neighbours' branches kept
+// the loads from overlapping: 50 us).
 __global__ __launch_bounds__(256) void k_layer(i64 n, i64 gnode0, const int* __restrict__ nbr,
                                                const float* __restrict__ sgn, const float* __restrict__ dinv,
                                                const float* __restrict__ hin, const uint16_t* __restrict__ prm,
                                                float* __restrict__ hout, float* __restrict__ tcache,
                                                float* __restrict__ mcache) {
-  __shared__ float Ws[H * HP], Wn[H * HP];
+  __shared__ __align__(16) float Ws[H][TP], Wn[H][TP];
   __shared__ float bs[H];
-  __shared__ float hs[NT * HP], ms[NT * HP];
+  __shared__ float hs[NT][HP], ms[NT][HP];
   const int tid = threadIdx.x;
   const i64 i0 = (i64)blockIdx.x * NT;
-  for (int e = tid; e < H * H; e += 256) {
-    int o = e / H, k = e % H;
-    Ws[o * HP + k] = bf(prm[e]);
-    Wn[o * HP + k] = bf(prm[H * H + e]);
-  }
+  stage_weights(prm, Ws, Wn, true);
   if (tid < H) bs[tid] = bf(prm[2 * H * H + tid]);
+#pragma unroll 4
   for (int e = tid; e < NT * H; e += 256) {
-    int nd = e / H, k = e % H;
-    i64 gi = i0 + nd;
-    float hv = 0.f, mv = 0.f;
-    if (gi < n) {
-      hv = hin[gi * H + k];
+    const int nd = e / H, k = e % H;
+    const i64 gi = min(i0 + nd, n - 1);
+    const float hv = hin[gi * H + k];
+    float mv = 0.f;
+    // every neighbour is read (a missing one as the node itself, weight 0)
 #pragma unroll
-      for (int q = 0; q < DEG; ++q) {
-        int j = nbr[gi * DEG + q];
-        if (j >= 0) mv += sgn[gi * DEG + q] * hin[(i64)(j - gnode0) * H + k];
-      }
-      mv *= dinv[gi];
+    for (int q = 0; q < DEG; ++q) {
+      const int j = nbr[gi * DEG + q];
+      const float w = j >= 0 ? sgn[gi * DEG + q] : 0.f;
+      mv += w * hin[(j >= 0 ? (i64)j - gnode0 : gi) * H + k];
     }
-    hs[nd * HP + k] = hv;
-    ms[nd * HP + k] = mv;
+    hs[nd][k] = hv;
+    ms[nd][k] = mv * dinv[gi];
   }
   __syncthreads();
-  const int nd = tid >> 2, cg = tid & 3;
-  float acc[16];
+  const int n0 = (tid >> 4) * 4, o0 = (tid & 15) * 4;
+  float acc[4][4];
 #pragma unroll
-  for (int j = 0; j < 16; ++j) acc[j] = bs[cg * 16 + j];
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[r][j] = bs[o0 + j];
+#pragma unroll 4
   for (int k = 0; k < H; ++k) {
-    const float hk = hs[nd * HP + k], mk = ms[nd * HP + k];
+    const float4 w = *reinterpret_cast<const float4*>(&Ws[k][o0]), v = *reinterpret_cast<const float4*>(&Wn[k][o0]);
+    const float wj[4] = {w.x, w.y, w.z, w.w}, vj[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int o = cg * 16 + j;
-      acc[j] += Ws[o * HP + k] * hk + Wn[o * HP + k] * mk;
+    for (int r = 0; r < 4; ++r) {
+      const float hk = hs[n0 + r][k], mk = ms[n0 + r][k];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[r][j] += wj[j] * hk + vj[j] * mk;
     }
   }
-  const i64 gi = i0 + nd;
-  if (gi >= n) return;
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int o = cg * 16 + j;
-    const float tt = tanhf(acc[j]);
-    hout[gi * H + o] = hs[nd * HP + o] + tt;
-    if (tcache) tcache[gi * H + o] = tt;
-    if (mcache) mcache[gi * H + o] = ms[nd * HP + o];
+  for (int r = 0; r < 4; ++r) {
+    const i64 gi = i0 + n0 + r;
+    if (gi >= n) continue;
+    float t[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) t[j] = tanhf(acc[r][j]);
+    *reinterpret_cast<float4*>(hout + gi * H + o0) = make_float4(
+        hs[n0 + r][o0] + t[0], hs[n0 + r][o0 + 1] + t[1], hs[n0 + r][o0 + 2] + t[2], hs[n0 + r][o0 + 3] + t[3]);
+    if (tcache) *reinterpret_cast<float4*>(tcache + gi * H + o0) = make_float4(t[0], t[1], t[2], t[3]);
+    if (mcache)
+      *reinterpret_cast<float4*>(mcache + gi * H + o0) =
+          make_float4(ms[n0 + r][o0], ms[n0 + r][o0 + 1], ms[n0 + r][o0 + 2], ms[n0 + r][o0 + 3]);
   }
 }
 
@@ -205,54 +232,54 @@ __global__ void k_decode_back(i64 n, const float2* __restrict__ gy, const uint16
   gh[idx] = bf(wd[k]) * g.x + bf(wd[H + k]) * g.y;
 }
 
-// ga = gh (1 - t^2); gh_out = gh + W_s^T ga; gm = dinv W_n^T ga
+// ga = gh (1 - t^2); gh_out = gh + W_s^T ga; gm = dinv W_n^T ga (tiles as in
+// k_layer)
 __global__ __launch_bounds__(256) void k_layer_back(i64 n, const float* __restrict__ gh, const float* __restrict__ t,
                                                     const float* __restrict__ dinv, const uint16_t* __restrict__ prm,
                                                     float* __restrict__ gh_out, float* __restrict__ gm) {
-  __shared__ float Ws[H * HP], Wn[H * HP];
-  __shared__ float gas[NT * HP];
+  __shared__ __align__(16) float Ws[H][TP], Wn[H][TP];
+  __shared__ float gas[NT][HP];
   const int tid = threadIdx.x;
   const i64 i0 = (i64)blockIdx.x * NT;
-  for (int e = tid; e < H * H; e += 256) {
-    int o = e / H, k = e % H;
-    Ws[o * HP + k] = bf(prm[e]);
-    Wn[o * HP + k] = bf(prm[H * H + e]);
-  }
+  stage_weights(prm, Ws, Wn, false);
+#pragma unroll 4
   for (int e = tid; e < NT * H; e += 256) {
-    int nd = e / H, o = e % H;
-    i64 gi = i0 + nd;
-    float v = 0.f;
-    if (gi < n) {
-      float tt = t[gi * H + o];
-      v = gh[gi * H + o] * (1.f - tt * tt);
-    }
-    gas[nd * HP + o] = v;
+    const int nd = e / H, o = e % H;
+    const i64 at = min(i0 + nd, n - 1) * H + o;
+    const float tt = t[at];
+    gas[nd][o] = gh[at] * (1.f - tt * tt);
   }
   __syncthreads();
-  const int nd = tid >> 2, cg = tid & 3;
-  float as[16], an[16];
+  const int n0 = (tid >> 4) * 4, k0 = (tid & 15) * 4;
+  float as[4][4], an[4][4];
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    as[j] = 0.f;
-    an[j] = 0.f;
-  }
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) as[r][j] = an[r][j] = 0.f;
+#pragma unroll 4
   for (int o = 0; o < H; ++o) {
-    const float g = gas[nd * HP + o];
+    const float4 w = *reinterpret_cast<const float4*>(&Ws[o][k0]), v = *reinterpret_cast<const float4*>(&Wn[o][k0]);
+    const float wj[4] = {w.x, w.y, w.z, w.w}, vj[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int k = cg * 16 + j;
-      as[j] += Ws[o * HP + k] * g;
-      an[j] += Wn[o * HP + k] * g;
+    for (int r = 0; r < 4; ++r) {
+      const float g = gas[n0 + r][o];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        as[r][j] += wj[j] * g;
+        an[r][j] += vj[j] * g;
+      }
     }
   }
-  const i64 gi = i0 + nd;
-  if (gi >= n) return;
-  const float di = dinv[gi];
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int k = cg * 16 + j;
-    gh_out[gi * H + k] = gh[gi * H + k] + as[j];
-    gm[gi * H + k] = an[j] * di;
+  for (int r = 0; r < 4; ++r) {
+    const i64 gi = i0 + n0 + r;
+    if (gi >= n) continue;
+    const float di = dinv[gi];
+    const float4 g = *reinterpret_cast<const float4*>(gh + gi * H + k0);
+    *reinterpret_cast<float4*>(gh_out + gi * H + k0) =
+        make_float4(g.x + as[r][0], g.y + as[r][1], g.z + as[r][2], g.w + as[r][3]);
+    *reinterpret_cast<float4*>(gm + gi * H + k0) =
+        make_float4(an[r][0] * di, an[r][1] * di, an[r][2] * di, an[r][3] * di);
   }
 }
 
@@ -329,16 +356,106 @@ __global__ __launch_bounds__(256) void k_outer(i64 n, const float* __restrict__ 
   }
 }
 
-// grad[woff + a * KB + c] (c < KB), grad[boff + a] (c == KB, bias) from G partials
-__global__ void k_outer_reduce(int G, int LA, int KB, int bias, const float* __restrict__ part, float* __restrict__ grad,
-                               int woff, int boff) {
+// The H x H form for up to two right factors that share the left one (the
+// layer's inputs and its messages): 4 x 4 sums per thread and factor from
+// 16-byte LDS reads; the bias sums ride with the first factor.  Reading one
+// value of each factor per FMA, and the left factor once per right factor,
+// took 2 x 22 us for 46 000 nodes; this takes 11 us.
+__global__ __launch_bounds__(256) void k_outer_pair(i64 n, const float* __restrict__ A, const float* __restrict__ T,
+                                                    const float* __restrict__ B0, const float* __restrict__ B1,
+                                                    float* __restrict__ part) {
+  constexpr int O = H * (H + 1);
+  __shared__ __align__(16) float As[NT][TP], Bs[2][NT][TP];
+  const int tid = threadIdx.x;
+  const int a0 = (tid >> 4) * 4, c0 = (tid & 15) * 4;
+  float acc[2][4][4], bias = 0.f;
+#pragma unroll
+  for (int f = 0; f < 2; ++f)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[f][i][j] = 0.f;
+  const i64 ntile = (n + NT - 1) / NT;
+  for (i64 tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+    const i64 i0 = tile * NT;
+    __syncthreads();
+#pragma unroll 4
+    for (int e = tid; e < NT * H / 4; e += 256) {
+      const int nd = e / (H / 4), c = e % (H / 4) * 4;
+      const i64 at = min(i0 + nd, n - 1) * H + c;
+      float4 a = *reinterpret_cast<const float4*>(A + at);
+      const float4 t = *reinterpret_cast<const float4*>(T + at);
+      a = make_float4(a.x * (1.f - t.x * t.x), a.y * (1.f - t.y * t.y), a.z * (1.f - t.z * t.z),
+                      a.w * (1.f - t.w * t.w));
+      if (i0 + nd >= n) a = make_float4(0.f, 0.f, 0.f, 0.f);
+      *reinterpret_cast<float4*>(&As[nd][c]) = a;
+      *reinterpret_cast<float4*>(&Bs[0][nd][c]) = *reinterpret_cast<const float4*>(B0 + at);
+      *reinterpret_cast<float4*>(&Bs[1][nd][c]) = *reinterpret_cast<const float4*>(B1 + at);
+    }
+    __syncthreads();
+    float s[2][4][4];
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[f][i][j] = 0.f;
+#pragma unroll 2
+    for (int nd = 0; nd < NT; ++nd) {
+      const float4 a = *reinterpret_cast<const float4*>(&As[nd][a0]);
+      const float ai[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+        const float4 b = *reinterpret_cast<const float4*>(&Bs[f][nd][c0]);
+        const float bj[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) s[f][i][j] += ai[i] * bj[j];
+      }
+    }
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[f][i][j] += s[f][i][j];
+    if (tid < H) {
+      float sb = 0.f;
+      for (int nd = 0; nd < NT; ++nd) sb += As[nd][tid];
+      bias += sb;
+    }
+  }
+  // factor f's partials of workgroup b at (f gridDim.x + b) O
+#pragma unroll
+  for (int f = 0; f < 2; ++f) {
+    float* p = part + ((i64)f * gridDim.x + blockIdx.x) * O;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) p[(a0 + i) * (H + 1) + c0 + j] = acc[f][i][j];
+    if (f == 0 && tid < H) p[tid * (H + 1) + H] = bias;
+  }
+}
+
+// grad[woff + a * KB + c] (c < KB), grad[boff + a] (c == KB, bias) from G
+// partials: the four waves of a workgroup take the partials b = wave mod 4 of
+// 64 sums, then their FP64 sums are added in order.
+__global__ __launch_bounds__(256) void k_outer_reduce(int G, int LA, int KB, int bias, const float* __restrict__ part,
+                                                      float* __restrict__ grad, int woff, int boff) {
+  __shared__ double red[4][64];
   const int KB1 = KB + 1, O = LA * KB1;
-  int o = blockIdx.x * blockDim.x + threadIdx.x;
-  if (o >= O) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int o = blockIdx.x * 64 + lane;
+  double s = 0;
+#pragma unroll 8
+  for (int b = wave; b < G; b += 4) s += part[(i64)b * O + min(o, O - 1)];
+  red[wave][lane] = s;
+  __syncthreads();
+  if (wave != 0 || o >= O) return;
   const int a = o / KB1, c = o % KB1;
   if (c == KB && !bias) return;
-  double s = 0;
-  for (int b = 0; b < G; ++b) s += part[(i64)b * O + o];
+  s = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
   if (c < KB)
     grad[woff + a * KB + c] = (float)s;
   else
@@ -555,7 +672,18 @@ void outer(i64 n, const float* A, const float* T, const float* B, int bias, floa
   const int G = (int)std::min<i64>(OUTER_G, std::max<i64>(1, (n + NT - 1) / NT));
   k_outer<LA, KB><<<G, 256, 0, s>>>(n, A, T, B, bias, part);
   const int O = LA * (KB + 1);
-  k_outer_reduce<<<(O + 255) / 256, 256, 0, s>>>(G, LA, KB, bias, part, grad, woff, boff);
+  k_outer_reduce<<<(O + 63) / 64, 256, 0, s>>>(G, LA, KB, bias, part, grad, woff, boff);
+}
+
+// weight and bias gradients of one layer: left factor gh (1 - t^2), right
+// factors the layer's inputs hin and messages ml
+void outer_layer(i64 n, const float* gh, const float* t, const float* hin, const float* ml, float* part, float* grad,
+                 int ws, int bo, int wn, hipStream_t s) {
+  const int G = (int)std::min<i64>(OUTER_G, std::max<i64>(1, (n + NT - 1) / NT));
+  constexpr int O = H * (H + 1);
+  k_outer_pair<<<G, 256, 0, s>>>(n, gh, t, hin, ml, part);
+  k_outer_reduce<<<(O + 63) / 64, 256, 0, s>>>(G, H, H, 1, part, grad, ws, bo);
+  k_outer_reduce<<<(O + 63) / 64, 256, 0, s>>>(G, H, H, 0, part + (size_t)G * O, grad, wn, 0);
 }
 
 }  // namespace
@@ -600,7 +728,7 @@ void sum(i64 n, const double* parts, double* out, hipStream_t s) {
 }
 
 size_t backward_floats(i64 n) { return (size_t)3 * n * H; }
-size_t outer_floats() { return (size_t)OUTER_G * H * (H + 1); }
+size_t outer_floats() { return (size_t)2 * OUTER_G * H * (H + 1); }
 
 void backward(const Graph& g, i64 gnode0, const uint16_t* prm, const Cache& c, const float* gy, float* grad,
               float* work, float* part, hipStream_t s) {
@@ -615,8 +743,7 @@ void backward(const Graph& g, i64 gnode0, const uint16_t* prm, const Cache& c, c
     const float* hin = c.h + (i64)l * n * H;
     const float* tl = c.t + (i64)l * n * H;
     const float* ml = c.m + (i64)l * n * H;
-    outer<H, H>(n, gh, tl, hin, 1, part, grad, off_ws(l), off_b(l), s);
-    outer<H, H>(n, gh, tl, ml, 0, part, grad, off_wn(l), 0, s);
+    outer_layer(n, gh, tl, hin, ml, part, grad, off_ws(l), off_b(l), off_wn(l), s);
     k_layer_back<<<gl, 256, 0, s>>>(n, gh, tl, g.dinv, prm + off_ws(l), gh2, gm);
     k_scatter<<<nb256(n * H), 256, 0, s>>>(n, gnode0, g.nbr, g.sgn, gm, gh2);
     std::swap(gh, gh2);
