@@ -14,7 +14,7 @@
 //
 // Self (t == t') and edge-adjacent pairs use the reference's singularity
 // extraction (src/assembly/EFIE.jl:534-684): they are precomputed in FP64 into
-// per-triangle tables by k_near_self / k_near_adj and looked up by the tile
+// per-triangle tables by k_near and looked up by the tile
 // kernel.  The adjacent-cell integral is not symmetric in (outer, inner); the
 // reference evaluates entry (min(m,n), max(m,n)) with the lower-index basis's
 // triangle as the outer one, and the tile kernel follows the caller's basis
@@ -148,145 +148,159 @@ struct NearArgs {
 //   J = sum_ab (f_e(a).f_e'(b) - 4/k^2) Gs_ab w_a w_b
 //     + sum_a w_a [ (f_e(a).f_e'(a) - 4/k^2) S_a/(4 pi 2A) + sum_b f_e(a).(r_b - r_a) w_b/(4 pi R_ab) ]
 // with f_e(r) = r - v_e.
-__device__ void near_self_one(const NearArgs& a, i64 t, double* jself) {
+// Lane ia of the pair's group forms outer point ia's terms.
+__device__ void near_self_point(const NearArgs& a, i64 t, int ia, c2 (&J)[9]) {
   const double* P = a.rq7 + t * 21;
   const double* V = a.vtx + t * 9;
-  double A = a.area[t];
-  c2 J[9];
+  const double A = a.area[t];
+  const double* ra = P + 3 * ia;
+  const double wa = a.w7[ia];
+  double fa[3][3], rem[3] = {0, 0, 0};
 #pragma unroll
-  for (int i = 0; i < 9; ++i) J[i] = {0.0, 0.0};
-  // smooth part, 7 x 7 with G_smooth
-  for (int ia = 0; ia < 7; ++ia) {
-    const double* ra = P + 3 * ia;
-    double fa[3][3];
+  for (int e = 0; e < 3; ++e)
 #pragma unroll
-    for (int e = 0; e < 3; ++e)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) fa[e][c] = ra[c] - V[3 * e + c];
-    for (int ib = 0; ib < 7; ++ib) {
-      const double* rb = P + 3 * ib;
-      c2 Gs = greens_smooth(dist3(ra, rb), a.q);
-      double wt = a.w7[ia] * a.w7[ib];
-#pragma unroll
-      for (int e = 0; e < 3; ++e)
-#pragma unroll
-        for (int f = 0; f < 3; ++f) {
-          double dd = fa[e][0] * (rb[0] - V[3 * f]) + fa[e][1] * (rb[1] - V[3 * f + 1]) + fa[e][2] * (rb[2] - V[3 * f + 2]);
-          c2 coef = {dd - a.four_ik2.re, -a.four_ik2.im};
-          J[3 * e + f] = cadd(J[3 * e + f], cscale(cmul(coef, Gs), wt));
-        }
-    }
-  }
-  // singular part: analytic inner integral + bounded remainder
-  for (int ia = 0; ia < 7; ++ia) {
-    const double* ra = P + 3 * ia;
-    double S = int_1overR(ra, V, V + 3, V + 6);
-    double sc = a.w7[ia] * S * INV4PI / (2.0 * A);
-    double rem[3] = {0, 0, 0};
-    for (int ib = 0; ib < 7; ++ib) {
-      const double* rb = P + 3 * ib;
-      double R = dist3(ra, rb);
-      if (R == 0.0) continue;
-      double k = a.w7[ia] * a.w7[ib] * INV4PI / R;
-#pragma unroll
-      for (int e = 0; e < 3; ++e)
-        rem[e] += ((ra[0] - V[3 * e]) * (rb[0] - ra[0]) + (ra[1] - V[3 * e + 1]) * (rb[1] - ra[1]) +
-                   (ra[2] - V[3 * e + 2]) * (rb[2] - ra[2])) * k;
-    }
+    for (int c = 0; c < 3; ++c) fa[e][c] = ra[c] - V[3 * e + c];
+  for (int ib = 0; ib < 7; ++ib) {
+    const double* rb = P + 3 * ib;
+    const double R = dist3(ra, rb), wt = wa * a.w7[ib];
+    // smooth part, G_smooth
+    const c2 Gs = greens_smooth(R, a.q);
 #pragma unroll
     for (int e = 0; e < 3; ++e)
 #pragma unroll
       for (int f = 0; f < 3; ++f) {
-        double dd = (ra[0] - V[3 * e]) * (ra[0] - V[3 * f]) + (ra[1] - V[3 * e + 1]) * (ra[1] - V[3 * f + 1]) +
-                    (ra[2] - V[3 * e + 2]) * (ra[2] - V[3 * f + 2]);
+        double dd = fa[e][0] * (rb[0] - V[3 * f]) + fa[e][1] * (rb[1] - V[3 * f + 1]) + fa[e][2] * (rb[2] - V[3 * f + 2]);
         c2 coef = {dd - a.four_ik2.re, -a.four_ik2.im};
-        J[3 * e + f] = cadd(J[3 * e + f], cscale(coef, sc));
-        J[3 * e + f].re += rem[e];
+        J[3 * e + f] = cadd(J[3 * e + f], cscale(cmul(coef, Gs), wt));
       }
-  }
-  c2* out = reinterpret_cast<c2*>(jself) + t * 9;
+    // singular part: bounded remainder
+    if (R != 0.0) {
+      const double k = wt * INV4PI / R;
 #pragma unroll
-  for (int i = 0; i < 9; ++i) out[i] = J[i];
+      for (int e = 0; e < 3; ++e)
+        rem[e] += (fa[e][0] * (rb[0] - ra[0]) + fa[e][1] * (rb[1] - ra[1]) + fa[e][2] * (rb[2] - ra[2])) * k;
+    }
+  }
+  // analytic inner integral
+  const double S = int_1overR(ra, V, V + 3, V + 6);
+  const double sc = wa * S * INV4PI / (2.0 * A);
+#pragma unroll
+  for (int e = 0; e < 3; ++e)
+#pragma unroll
+    for (int f = 0; f < 3; ++f) {
+      double dd = fa[e][0] * fa[f][0] + fa[e][1] * fa[f][1] + fa[e][2] * fa[f][2];
+      c2 coef = {dd - a.four_ik2.re, -a.four_ik2.im};
+      J[3 * e + f] = cadd(J[3 * e + f], cscale(coef, sc));
+      J[3 * e + f].re += rem[e];
+    }
 }
 
 // Adjacent cell (src/assembly/EFIE.jl:611-684), outer triangle t, inner
 // triangle u = nb[t][j], normalised by (2A_t)(2A_u):
 //   J = sum_ab^{nq} (f_e(a).f'_e'(b) - 4/k^2) Gs_ab w_a w_b
 //     + sum_a^7 w_a [ sum_b^7 f_e(a).f'_e'(b) w_b/(4 pi R_ab) - 4/k^2 S_u(a)/(4 pi 2A_u) ]
-__device__ void near_adj_one(const NearArgs& a, i64 idx, double* jadj) {
-  i64 t = idx / 3;
-  int u = a.nb[idx];
-  c2* out = reinterpret_cast<c2*>(jadj) + idx * 9;
-  if (u < 0) {
-#pragma unroll
-    for (int i = 0; i < 9; ++i) out[i] = {0.0, 0.0};
-    return;
-  }
+__device__ void near_adj_point(const NearArgs& a, i64 t, int u, int ia, c2 (&J)[9]) {
   const double* Vt = a.vtx + t * 9;
   const double* Vu = a.vtx + (i64)u * 9;
-  double Au = a.area[u];
-  c2 J[9];
-#pragma unroll
-  for (int i = 0; i < 9; ++i) J[i] = {0.0, 0.0};
   const int nq = a.nq;
-  for (int ia = 0; ia < nq; ++ia) {
+  auto dots = [&](const double* ra, const double* rb, double (&dd)[9]) {
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+#pragma unroll
+      for (int f = 0; f < 3; ++f)
+        dd[3 * e + f] = (ra[0] - Vt[3 * e]) * (rb[0] - Vu[3 * f]) + (ra[1] - Vt[3 * e + 1]) * (rb[1] - Vu[3 * f + 1]) +
+                        (ra[2] - Vt[3 * e + 2]) * (rb[2] - Vu[3 * f + 2]);
+  };
+  double dd[9];
+  if (ia < nq) {
     const double* ra = a.rq + (t * nq + ia) * 3;
     for (int ib = 0; ib < nq; ++ib) {
       const double* rb = a.rq + ((i64)u * nq + ib) * 3;
-      c2 Gs = greens_smooth(dist3(ra, rb), a.q);
-      double wt = a.w[ia] * a.w[ib];
+      const c2 Gs = greens_smooth(dist3(ra, rb), a.q);
+      const double wt = a.w[ia] * a.w[ib];
+      dots(ra, rb, dd);
 #pragma unroll
-      for (int e = 0; e < 3; ++e)
-#pragma unroll
-        for (int f = 0; f < 3; ++f) {
-          double dd = (ra[0] - Vt[3 * e]) * (rb[0] - Vu[3 * f]) + (ra[1] - Vt[3 * e + 1]) * (rb[1] - Vu[3 * f + 1]) +
-                      (ra[2] - Vt[3 * e + 2]) * (rb[2] - Vu[3 * f + 2]);
-          c2 coef = {dd - a.four_ik2.re, -a.four_ik2.im};
-          J[3 * e + f] = cadd(J[3 * e + f], cscale(cmul(coef, Gs), wt));
-        }
+      for (int i = 0; i < 9; ++i) {
+        c2 coef = {dd[i] - a.four_ik2.re, -a.four_ik2.im};
+        J[i] = cadd(J[i], cscale(cmul(coef, Gs), wt));
+      }
     }
   }
-  for (int ia = 0; ia < 7; ++ia) {
-    const double* ra = a.rq7 + t * 21 + 3 * ia;
-    double S = int_1overR(ra, Vu, Vu + 3, Vu + 6);
-    double sc = a.w7[ia] * S * INV4PI / (2.0 * Au);
-    double vs[9];
+  const double* ra = a.rq7 + t * 21 + 3 * ia;
+  const double S = int_1overR(ra, Vu, Vu + 3, Vu + 6);
+  const double sc = a.w7[ia] * S * INV4PI / (2.0 * a.area[u]);
+  double vs[9];
 #pragma unroll
-    for (int i = 0; i < 9; ++i) vs[i] = 0.0;
-    for (int ib = 0; ib < 7; ++ib) {
-      const double* rb = a.rq7 + (i64)u * 21 + 3 * ib;
-      double R = dist3(ra, rb);
-      if (R == 0.0) continue;
-      double k = a.w7[ia] * a.w7[ib] * INV4PI / R;
+  for (int i = 0; i < 9; ++i) vs[i] = 0.0;
+  for (int ib = 0; ib < 7; ++ib) {
+    const double* rb = a.rq7 + (i64)u * 21 + 3 * ib;
+    const double R = dist3(ra, rb);
+    if (R == 0.0) continue;
+    const double k = a.w7[ia] * a.w7[ib] * INV4PI / R;
+    dots(ra, rb, dd);
 #pragma unroll
-      for (int e = 0; e < 3; ++e)
-#pragma unroll
-        for (int f = 0; f < 3; ++f)
-          vs[3 * e + f] += ((ra[0] - Vt[3 * e]) * (rb[0] - Vu[3 * f]) + (ra[1] - Vt[3 * e + 1]) * (rb[1] - Vu[3 * f + 1]) +
-                            (ra[2] - Vt[3 * e + 2]) * (rb[2] - Vu[3 * f + 2])) * k;
-    }
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-      J[i].re += vs[i] - sc * a.four_ik2.re;
-      J[i].im -= sc * a.four_ik2.im;
-    }
+    for (int i = 0; i < 9; ++i) vs[i] += dd[i] * k;
   }
 #pragma unroll
-  for (int i = 0; i < 9; ++i) out[i] = J[i];
+  for (int i = 0; i < 9; ++i) {
+    J[i].re += vs[i] - sc * a.four_ik2.re;
+    J[i].im -= sc * a.four_ik2.im;
+  }
 }
 
-__global__ __launch_bounds__(64) void k_near_self(NearArgs a, double* jself) {
-  const i64 t = blockIdx.x * (i64)blockDim.x + threadIdx.x;
-  if (t < a.nt) near_self_one(a, t, jself);
+// v plus the same value of the lanes one DPP step away
+template <int CTRL>
+__device__ inline double dpp_plus(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)(b & 0xffffffffLL), CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, false);
+  return v + __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
-__global__ __launch_bounds__(64) void k_near_adj(NearArgs a, double* jadj) {
-  const i64 idx = blockIdx.x * (i64)blockDim.x + threadIdx.x;
-  if (idx < a.nt * 3) near_adj_one(a, idx, jadj);
+__device__ inline double sum8(double v) {
+  v = dpp_plus<0xB1>(v);    // quad_perm 1,0,3,2
+  v = dpp_plus<0x4E>(v);    // quad_perm 2,3,0,1
+  return dpp_plus<0x141>(v);  // row_half_mirror
 }
 
-// Many meshes in one launch: item g of the concatenated lists (per mesh m,
-// items per triangle x its triangles starting at toff[m]) belongs to the mesh
-// found by binary search; each mesh's tables start at per x 9 complex x toff[m].
+// Pair p of a mesh: p < nt the self cell of triangle p, else the adjacent cell
+// (p - nt) = 3 t + neighbour slot.  Eight lanes per pair, lane ia its outer
+// point ia (7 of them), the nine sums added over the eight lanes.  Bound by the
+// latency of the G_smooth series and of the closed-form integral's logarithms
+// and arctangents: 24 us for small meshes, 34 us for 5120 triangles (one thread
+// per pair, 49 points in sequence, took 80 + 50 us for the self and the adjacent
+// cells of any mesh up to ~10 000 triangles); beyond ~50 000 triangles the FP64
+// rate decides and both forms take the same time.
+constexpr int kNearLanes = 8;
+__device__ void near_pair(const NearArgs& a, i64 p, double* jself, double* jadj) {
+  const int ia = threadIdx.x & (kNearLanes - 1);
+  const bool self = p < a.nt;
+  const int u = self ? 0 : a.nb[p - a.nt];
+  c2 J[9];
+#pragma unroll
+  for (int i = 0; i < 9; ++i) J[i] = {0.0, 0.0};
+  if (ia < 7) {
+    if (self)
+      near_self_point(a, p, ia, J);
+    else if (u >= 0)
+      near_adj_point(a, (p - a.nt) / 3, u, ia, J);
+  }
+  c2* out = self ? reinterpret_cast<c2*>(jself) + p * 9 : reinterpret_cast<c2*>(jadj) + (p - a.nt) * 9;
+#pragma unroll
+  for (int i = 0; i < 9; ++i) {
+    const c2 s = {sum8(J[i].re), sum8(J[i].im)};
+    if (ia == (i & 7)) out[i] = s;
+  }
+}
+
+// the lanes of a group stay together: p is clamped, not branched on, for the
+// last group
+__global__ __launch_bounds__(64) void k_near(NearArgs a, double* jself, double* jadj) {
+  const i64 p = blockIdx.x * (i64)(64 / kNearLanes) + threadIdx.x / kNearLanes;
+  near_pair(a, min(p, 4 * a.nt - 1), jself, jadj);
+}
+
+// The same tables of many meshes in one launch: pair index over all
+// meshes' pairs, the mesh found from the triangle offsets.
 __device__ inline int mesh_of(const i64* __restrict__ toff, int nmesh, i64 g) {
   int lo = 0, hi = nmesh - 1;
   while (lo < hi) {
@@ -298,19 +312,11 @@ __device__ inline int mesh_of(const i64* __restrict__ toff, int nmesh, i64 g) {
   }
   return lo;
 }
-__global__ __launch_bounds__(64) void k_near_self_multi(const NearArgs* __restrict__ args,
-                                                        const i64* __restrict__ toff, int nmesh, double* jself) {
-  const i64 g = blockIdx.x * (i64)blockDim.x + threadIdx.x;
-  if (g >= toff[nmesh]) return;
-  const int m = mesh_of(toff, nmesh, g);
-  near_self_one(args[m], g - toff[m], jself + 18 * toff[m]);
-}
-__global__ __launch_bounds__(64) void k_near_adj_multi(const NearArgs* __restrict__ args,
-                                                       const i64* __restrict__ toff, int nmesh, double* jadj) {
-  const i64 g = blockIdx.x * (i64)blockDim.x + threadIdx.x;
-  if (g >= 3 * toff[nmesh]) return;
-  const int m = mesh_of(toff, nmesh, g / 3);
-  near_adj_one(args[m], g - 3 * toff[m], jadj + 54 * toff[m]);
+__global__ __launch_bounds__(64) void k_near_multi(const NearArgs* __restrict__ args, const i64* __restrict__ toff,
+                                                   int nmesh, double* jself, double* jadj) {
+  const i64 g = min(blockIdx.x * (i64)(64 / kNearLanes) + threadIdx.x / kNearLanes, 4 * toff[nmesh] - 1);
+  const int m = mesh_of(toff, nmesh, g / 4);
+  near_pair(args[m], g - 4 * toff[m], jself + 18 * toff[m], jadj + 54 * toff[m]);
 }
 
 // ------------------------------------------------------------------ far tiles
@@ -977,9 +983,8 @@ static NearArgs near_args(const AsmArgs& a, const TriTables& t) {
 
 void launch_near_tables(const AsmArgs& a, const TriTables& t, double* jself, double* jadj, hipStream_t s) {
   NearArgs n = near_args(a, t);
-  unsigned g1 = (unsigned)((a.nt + 63) / 64), g2 = (unsigned)((3 * a.nt + 63) / 64);
-  k_near_self<<<g1, 64, 0, s>>>(n, jself);
-  k_near_adj<<<g2, 64, 0, s>>>(n, jadj);
+  constexpr int per = 64 / kNearLanes;  // pairs per workgroup
+  k_near<<<(unsigned)((4 * a.nt + per - 1) / per), 64, 0, s>>>(n, jself, jadj);
   HIP_OK(hipGetLastError());
 }
 
@@ -1001,8 +1006,8 @@ void launch_near_tables_multi(const std::vector<AsmArgs>& a, const std::vector<c
   const NearArgs* dargs = reinterpret_cast<const NearArgs*>(staging.p);
   const i64* doff = reinterpret_cast<const i64*>(staging.p + obase);
   const i64 total = toff[nmesh];
-  k_near_self_multi<<<(unsigned)((total + 63) / 64), 64, 0, s>>>(dargs, doff, nmesh, jself);
-  k_near_adj_multi<<<(unsigned)((3 * total + 63) / 64), 64, 0, s>>>(dargs, doff, nmesh, jadj);
+  constexpr int per = 64 / kNearLanes;
+  k_near_multi<<<(unsigned)((4 * total + per - 1) / per), 64, 0, s>>>(dargs, doff, nmesh, jself, jadj);
   HIP_OK(hipGetLastError());
 }
 
