@@ -1046,8 +1046,10 @@ def mesh_resolution_report(mesh, freq_hz, points_per_wavelength=10.0, c0=C0_DEFA
     """src/geometry/Mesh.jl:3418-3471"""
     lam = c0 / freq_hz
     t = mesh.tri - 1
-    e = np.concatenate([t[:, [0, 1]], t[:, [1, 2]], t[:, [2, 0]]])
-    e = np.unique(np.sort(e, axis=1), axis=0)
+    a = np.concatenate([t[:, 0], t[:, 1], t[:, 2]])
+    b = np.concatenate([t[:, 1], t[:, 2], t[:, 0]])
+    key = np.unique(np.minimum(a, b) * mesh.nv + np.maximum(a, b))  # one integer per edge
+    e = np.stack([key // mesh.nv, key % mesh.nv], axis=1)
     lens = np.sort(np.linalg.norm(mesh.xyz[e[:, 0]] - mesh.xyz[e[:, 1]], axis=1))
     target = lam / points_per_wavelength
     return dict(wavelength_m=lam, target_max_edge_m=target, edge_min_m=lens[0], edge_max_m=lens[-1],

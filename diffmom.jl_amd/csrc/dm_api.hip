@@ -45,16 +45,25 @@ void* scratch_of(int device) {
 }
 }  // namespace
 
+void DevCache::forget(void* p, size_t b) {
+  bytes -= b;
+  if (freed.erase(p)) freed_bytes -= b;
+}
 void* DevCache::take(size_t b) {
   auto it = free_blocks.find(b);
   if (it == free_blocks.end()) return nullptr;
   void* p = it->second;
   free_blocks.erase(it);
-  bytes -= b;
+  forget(p, b);
   return p;
 }
 bool DevCache::give(void* p, size_t b) {
   if (bytes + b > cap) return false;
+  if (freeing) {
+    if (b > kFreedBlock || freed_bytes + b > kFreedTotal) return false;
+    freed.insert(p);
+    freed_bytes += b;
+  }
   pending.emplace_back(b, p);
   bytes += b;
   return true;
@@ -76,7 +85,7 @@ void DevCache::promote(hipStream_t a, hipStream_t b) {
 void DevCache::trim() {
   for (auto& e : free_blocks) {
     (void)hipFree(e.second);
-    bytes -= e.first;
+    forget(e.second, e.first);
   }
   free_blocks.clear();
 }
@@ -84,7 +93,8 @@ void DevCache::clear() {
   trim();
   for (auto& e : pending) (void)hipFree(e.second);
   pending.clear();
-  bytes = 0;
+  freed.clear();
+  bytes = freed_bytes = 0;
 }
 
 namespace {
@@ -111,24 +121,6 @@ int guard(F&& f) {
     return DM_ERR_DEVICE;
   }
 }
-
-// A public call on a context: its lock, its device, and its memory cache for
-// the buffers the call allocates and releases.
-struct CtxScope {
-  std::lock_guard<std::mutex> lk;
-  dm_ctx* c;
-  DevCache* prev;
-  explicit CtxScope(dm_ctx* c_) : lk(c_->mu), c(c_), prev(tl_cache) {
-    HIP_OK(hipSetDevice(c->device));
-    c->cache.promote(c->stream, c->stream2);
-    tl_cache = &c->cache;
-  }
-  ~CtxScope() {
-    c->cache.promote(c->stream, c->stream2);
-    tl_cache = prev;
-  }
-};
-
 
 // _validated_efie_prefactors: src/assembly/EFIE.jl:297-330
 void validate_prefactors(double kr, double ki, double eta0) {
@@ -615,7 +607,8 @@ int dm_mesh_check(const dm_mesh* mesh, int allow_boundary, int require_closed, d
 int dm_mesh_areas(const dm_mesh* mesh, double* areas) {
   return guard([&] {
     check_ctx(mesh, "mesh");
-    for (i64 t = 0; t < mesh->nt; ++t) areas[t] = dmh::triangle_area(*mesh, t);
+    const std::vector<double>& a = dmh::triangle_areas(*mesh);
+    std::copy(a.begin(), a.end(), areas);
   });
 }
 
@@ -695,8 +688,7 @@ int dm_rwg_export(const dm_rwg* r, int64_t* tplus, int64_t* tminus, int64_t* eve
 int dm_rwg_free(dm_rwg* rwg) {
   return guard([&] {
     if (!rwg) return;
-    std::lock_guard<std::mutex> lk(rwg->ctx->mu);
-    (void)hipSetDevice(rwg->ctx->device);
+    FreeScope sc(rwg->ctx);
     delete rwg;
   });
 }
@@ -977,8 +969,7 @@ int dm_zmat_entries(const dm_zmat* z, int form, const int64_t* m, const int64_t*
 int dm_zmat_free(dm_zmat* z) {
   return guard([&] {
     if (!z) return;
-    std::lock_guard<std::mutex> lk(z->ctx->mu);
-    (void)hipSetDevice(z->ctx->device);
+    FreeScope sc(z->ctx);
     delete z;
   });
 }
@@ -1288,8 +1279,7 @@ int dm_precond_apply(dm_ctx* ctx, const dm_precond* P, const double* x, double* 
 int dm_precond_free(dm_precond* P) {
   return guard([&] {
     if (!P) return;
-    std::lock_guard<std::mutex> lk(P->ctx->mu);
-    (void)hipSetDevice(P->ctx->device);
+    FreeScope sc(P->ctx);
     delete P;
   });
 }

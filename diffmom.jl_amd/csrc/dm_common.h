@@ -10,6 +10,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <set>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -47,9 +48,17 @@ struct DmError : std::runtime_error {
 // streams have been seen idle, so no queued kernel can still touch it.
 // dm_destroy frees everything kept; a failed hipMalloc frees the reusable
 // blocks and retries.
+// Handles that a caller frees give their memory back to the device, except
+// blocks of up to kFreedBlock bytes, of which kFreedTotal in all are kept (a
+// hipFree costs ~0.2 ms and waits for the device: programs that make and free
+// many small matrices spent most of their time there).
 struct DevCache {
+  static constexpr size_t kFreedBlock = size_t(128) << 20, kFreedTotal = size_t(2) << 30;
   int device = -1;
   size_t cap = 0, bytes = 0;
+  bool freeing = false;          // a handle is being freed (FreeScope)
+  size_t freed_bytes = 0;        // kept blocks that came from freed handles
+  std::set<void*> freed;
   std::multimap<size_t, void*> free_blocks;
   std::vector<std::pair<size_t, void*>> pending;
   void* take(size_t b);
@@ -57,6 +66,7 @@ struct DevCache {
   void promote(hipStream_t a, hipStream_t b);  // pending -> reusable when both streams are idle
   void trim();                                 // free the reusable blocks
   void clear();                                // free everything
+  void forget(void* p, size_t b);              // a kept block leaves the cache
 };
 // the cache of the context whose public call runs on this thread (or null)
 extern thread_local DevCache* tl_cache;
@@ -66,20 +76,29 @@ struct DBuf {
   T* p = nullptr;
   size_t n = 0;
   int dev = -1;
+  bool own = true;  // false: part of another buffer (view)
   DBuf() = default;
   DBuf(const DBuf&) = delete;
   DBuf& operator=(const DBuf&) = delete;
   ~DBuf() { release(); }
   void release() {
-    if (p) {
+    if (p && own) {
       const size_t b = n * sizeof(T);
       if (!(tl_cache && tl_cache->device == dev && tl_cache->give(p, b))) (void)hipFree(p);
     }
     p = nullptr;
     n = 0;
+    own = true;
+  }
+  // count elements at q, inside a buffer that outlives this one
+  void view(T* q, size_t count) {
+    release();
+    p = q;
+    n = count;
+    own = false;
   }
   void alloc(size_t count) {
-    if (count == n && p) return;
+    if (count == n && p && own) return;
     release();
     if (count == 0) return;
     const size_t b = count * sizeof(T);
@@ -159,6 +178,29 @@ struct ProfScope {
   }
 };
 
+// A public call on a context: its lock, its device, and its memory cache for
+// the buffers the call allocates and releases.
+struct CtxScope {
+  std::lock_guard<std::mutex> lk;
+  dm_ctx* c;
+  DevCache* prev;
+  explicit CtxScope(dm_ctx* c_) : lk(c_->mu), c(c_), prev(tl_cache) {
+    HIP_OK(hipSetDevice(c->device));
+    c->cache.promote(c->stream, c->stream2);
+    tl_cache = &c->cache;
+  }
+  ~CtxScope() {
+    c->cache.promote(c->stream, c->stream2);
+    tl_cache = prev;
+  }
+};
+// The same for freeing a handle of the context: small blocks stay in the cache.
+struct FreeScope {
+  CtxScope sc;
+  explicit FreeScope(dm_ctx* c) : sc(c) { c->cache.freeing = true; }
+  ~FreeScope() { sc.c->cache.freeing = false; }
+};
+
 // Message returned by dm_last_error() for the calling thread.
 void dm_set_error(const std::string& msg);
 
@@ -167,11 +209,14 @@ struct dm_mesh {
   i64 nv = 0, nt = 0;
   std::vector<double> xyz;  // 3 x nv
   std::vector<i64> tri;     // 3 x nt, 1-based
+  mutable std::once_flag areas_once;
+  mutable std::vector<double> areas;  // dmh::triangle_areas
 };
 
 // Per-quadrature-order triangle tables (device), built lazily per RWG handle.
 struct TriTables {
   int quad_order = 0, nq = 0;
+  DBuf<char> all;     // the buffer that holds the tables below
   DBuf<double> cen;   // nt*3 centroid
   DBuf<double> uq;    // nt*nq*3 quad points relative to the centroid
   DBuf<double> av;    // nt*9 vertex offsets from the centroid
@@ -179,7 +224,6 @@ struct TriTables {
   DBuf<double> rq7;   // nt*7*3 absolute 7-point rule points
   DBuf<double> vtx;   // nt*9 absolute vertices
   DBuf<double> area;  // nt
-  std::vector<double> h_rq, h_area;
 };
 
 // Near-field sparse-approximate-inverse pattern (internal basis order).
@@ -213,7 +257,8 @@ struct dm_rwg {
   int nblk = 0;
   int max_blk_tris = 0;
   std::vector<int> blk_off, blk_tri;  // CSR: triangles touched by each block
-  // device copies
+  // device copies, parts of one buffer
+  DBuf<char> d_all;
   DBuf<int> d_ext;          // n
   DBuf<int> d_iofe;         // n: caller index -> internal index
   DBuf<double> d_len;       // n (internal order)
@@ -329,6 +374,7 @@ void build_rwg_canonical(const dm_mesh& m, dm_rwg& r);
 void finalize_rwg(dm_rwg& r);  // validates, orders, tiles, uploads
 void mesh_check(const dm_mesh& m, int allow_boundary, int require_closed, double area_tol_rel);
 double triangle_area(const dm_mesh& m, i64 t0);
+const std::vector<double>& triangle_areas(const dm_mesh& m);  // formed on first use
 const TriTables& tables(dm_rwg& r, int quad_order);
 int quad_rule(int order, double* xi, double* w);
 std::shared_ptr<const SpaiPattern> spai_pattern(dm_rwg& r, double cutJ, int maxJ);

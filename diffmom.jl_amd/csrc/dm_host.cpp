@@ -8,10 +8,10 @@
 #include <array>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <numeric>
 #include <sstream>
-#include <tuple>
 
 #include "dm_common.h"
 
@@ -85,11 +85,58 @@ double triangle_area(const dm_mesh& m, i64 t0) {
   return std::ldexp(0.5 * fr, xn + x1 + x2);
 }
 
+const std::vector<double>& triangle_areas(const dm_mesh& m) {
+  std::call_once(m.areas_once, [&] {
+    m.areas.resize(m.nt);
+    for (i64 t = 0; t < m.nt; ++t) m.areas[t] = triangle_area(m, t);
+  });
+  return m.areas;
+}
+
+namespace {
+// The 3 nt triangle sides (t, le) -> 3 t + le, ordered by their vertex pair
+// (lower, higher vertex) and then by the side's index: an LSD radix sort of
+// the pair keys, stable, one byte per pass.
+struct Side {
+  uint64_t key;  // lower << 32 | higher vertex (1-based)
+  int64_t idx;
+};
+std::vector<Side> sorted_sides(const dm_mesh& m) {
+  DM_REQUIRE(m.nv < (1LL << 32), DM_ERR_ARGUMENT, "mesh too large for 32-bit vertex indices");
+  const size_t n = 3 * (size_t)m.nt;
+  std::vector<Side> a(n), b(n);
+  uint64_t all = 0;
+  for (i64 t = 0; t < m.nt; ++t)
+    for (int le = 0; le < 3; ++le) {
+      const uint64_t u = (uint64_t)m.tri[3 * t + le], v = (uint64_t)m.tri[3 * t + (le + 1) % 3];
+      const uint64_t k = std::min(u, v) << 32 | std::max(u, v);
+      a[3 * t + le] = {k, 3 * t + le};
+      all |= k;
+    }
+  for (int sh = 0; sh < 64; sh += 8) {
+    if (!((all >> sh) & 255)) continue;  // this byte is zero in every key
+    size_t at[257] = {0};
+    for (const Side& e : a) ++at[((e.key >> sh) & 255) + 1];
+    for (int i = 0; i < 256; ++i) at[i + 1] += at[i];
+    for (const Side& e : a) b[at[(e.key >> sh) & 255]++] = e;
+    a.swap(b);
+  }
+  return a;
+}
+// end of the run of sides that share side i's vertex pair
+inline size_t run_end(const std::vector<Side>& s, size_t i) {
+  size_t j = i + 1;
+  while (j < s.size() && s[j].key == s[i].key) ++j;
+  return j;
+}
+}  // namespace
+
 // assert_mesh_quality: src/geometry/Mesh.jl:1093-1255.
 void mesh_check(const dm_mesh& m, int allow_boundary, int require_closed, double area_tol_rel) {
   DM_REQUIRE(std::isfinite(area_tol_rel) && area_tol_rel >= 0, DM_ERR_ARGUMENT,
              "area_tol_rel must be finite and nonnegative");
   i64 nv = m.nv, nt = m.nt;
+  const std::vector<double>& area = triangle_areas(m);
   std::vector<char> finite(nv, 1);
   i64 invalid_vertices = 0;
   for (i64 i = 0; i < nv; ++i)
@@ -108,7 +155,7 @@ void mesh_check(const dm_mesh& m, int allow_boundary, int require_closed, double
   };
   for (i64 t = 0; t < nt; ++t) {
     if (!valid_face(t)) continue;
-    double a = triangle_area(m, t);
+    const double a = area[t];
     if (!(std::isfinite(a) && a > 0)) continue;
     for (int j = 0; j < 3; ++j)
       for (int c = 0; c < 3; ++c) {
@@ -126,29 +173,49 @@ void mesh_check(const dm_mesh& m, int allow_boundary, int require_closed, double
     tol_abs = s * s;
   }
   i64 invalid_tris = 0, degenerate = 0, duplicate = 0, nonmanifold = 0, conflicts = 0, boundary = 0;
-  std::map<std::array<i64, 3>, int> faces;
-  std::map<std::pair<i64, i64>, std::vector<int>> edges;
+  // equal faces (same three vertices): all but the first are duplicates
+  std::vector<std::pair<std::array<i64, 3>, i64>> faces;
+  faces.reserve(nt);
+  std::vector<char> use(nt, 0);  // valid, first of its face, finite area: its sides count
   for (i64 t = 0; t < nt; ++t) {
     if (!valid_face(t)) { ++invalid_tris; continue; }
     const i64* tr = &m.tri[3 * t];
     std::array<i64, 3> key = {tr[0], tr[1], tr[2]};
     std::sort(key.begin(), key.end());
-    bool dup = faces.count(key) > 0;
-    if (dup) ++duplicate; else faces[key] = 1;
-    double a = triangle_area(m, t);
-    if (!std::isfinite(a)) { ++invalid_tris; continue; }
-    if (a <= tol_abs) ++degenerate;
-    if (dup) continue;
-    for (int j = 0; j < 3; ++j) {
-      i64 a0 = tr[j], b0 = tr[(j + 1) % 3];
-      edges[{std::min(a0, b0), std::max(a0, b0)}].push_back(a0 < b0 ? 1 : -1);
-    }
+    faces.push_back({key, t});
+    use[t] = 1;
   }
-  for (auto& kv : edges) {
-    size_t d = kv.second.size();
+  std::sort(faces.begin(), faces.end());
+  for (size_t i = 1; i < faces.size(); ++i)
+    if (faces[i].first == faces[i - 1].first) {
+      ++duplicate;
+      use[faces[i].second] = 2;
+    }
+  for (i64 t = 0; t < nt; ++t) {
+    if (!use[t]) continue;
+    if (!std::isfinite(area[t])) {
+      ++invalid_tris;
+      use[t] = 0;
+      continue;
+    }
+    if (area[t] <= tol_abs) ++degenerate;
+    if (use[t] == 2) use[t] = 0;
+  }
+  const std::vector<Side> sides = sorted_sides(m);
+  for (size_t i = 0; i < sides.size();) {
+    const size_t j = run_end(sides, i);
+    int d = 0, dir = 0;  // sides that count, their directions' sum
+    for (size_t q = i; q < j; ++q) {
+      const i64 t = sides[q].idx / 3;
+      if (!use[t]) continue;
+      const int le = (int)(sides[q].idx % 3);
+      ++d;
+      dir += m.tri[3 * t + le] < m.tri[3 * t + (le + 1) % 3] ? 1 : -1;
+    }
     if (d == 1) ++boundary;
-    else if (d == 2) { if (kv.second[0] == kv.second[1]) ++conflicts; }
-    else ++nonmanifold;
+    else if (d == 2) { if (dir != 0) ++conflicts; }
+    else if (d > 2) ++nonmanifold;
+    i = j;
   }
   std::ostringstream os;
   bool bad = false;
@@ -169,26 +236,17 @@ void mesh_check(const dm_mesh& m, int allow_boundary, int require_closed, double
 // lower-index triangle (the first one to list the edge).  Basis order: sorted
 // (v1 < v2) edge keys.
 void build_rwg_canonical(const dm_mesh& m, dm_rwg& r) {
-  std::vector<std::tuple<i64, i64, i64, int>> rec;  // (va, vb, t, le)
-  rec.reserve(3 * m.nt);
-  for (i64 t = 0; t < m.nt; ++t)
-    for (int le = 0; le < 3; ++le) {
-      i64 a = m.tri[3 * t + le], b = m.tri[3 * t + (le + 1) % 3];
-      rec.emplace_back(std::min(a, b), std::max(a, b), t + 1, le);
-    }
-  std::sort(rec.begin(), rec.end());
+  const std::vector<Side> rec = sorted_sides(m);
+  const std::vector<double>& area = triangle_areas(m);
   r.tplus.clear(); r.tminus.clear(); r.evert.clear(); r.vplus_opp.clear(); r.vminus_opp.clear();
   r.len.clear(); r.area_p.clear(); r.area_m.clear();
   size_t i = 0;
   while (i < rec.size()) {
-    size_t j = i + 1;
-    while (j < rec.size() && std::get<0>(rec[j]) == std::get<0>(rec[i]) &&
-           std::get<1>(rec[j]) == std::get<1>(rec[i]))
-      ++j;
+    const size_t j = run_end(rec, i);
     if (j - i == 2) {
-      i64 va = std::get<0>(rec[i]), vb = std::get<1>(rec[i]);
-      i64 t1 = std::get<2>(rec[i]), t2 = std::get<2>(rec[i + 1]);
-      int l1 = std::get<3>(rec[i]), l2 = std::get<3>(rec[i + 1]);
+      i64 va = (i64)(rec[i].key >> 32), vb = (i64)(rec[i].key & 0xffffffffu);
+      i64 t1 = rec[i].idx / 3 + 1, t2 = rec[i + 1].idx / 3 + 1;
+      int l1 = (int)(rec[i].idx % 3), l2 = (int)(rec[i + 1].idx % 3);
       r.tplus.push_back(t1);
       r.tminus.push_back(t2);
       r.evert.push_back(va);
@@ -199,8 +257,8 @@ void build_rwg_canonical(const dm_mesh& m, dm_rwg& r) {
       double len = std::hypot(std::hypot(p2.x - p1.x, p2.y - p1.y), p2.z - p1.z);
       DM_REQUIRE(len > 0 && std::isfinite(len), DM_ERR_DOMAIN, "RWG edge has zero or unrepresentable length");
       r.len.push_back(len);
-      r.area_p.push_back(triangle_area(m, t1 - 1));
-      r.area_m.push_back(triangle_area(m, t2 - 1));
+      r.area_p.push_back(area[t1 - 1]);
+      r.area_m.push_back(area[t2 - 1]);
     }
     i = j;
   }
@@ -210,6 +268,25 @@ void build_rwg_canonical(const dm_mesh& m, dm_rwg& r) {
 }
 
 namespace {
+// Several host arrays in one device buffer: one allocation and one copy
+// instead of one of each per array.
+struct Packed {
+  std::vector<char> host;
+  std::vector<std::function<void(char*)>> place;
+  template <class T>
+  void add(DBuf<T>& b, const std::vector<T>& v) {
+    const size_t off = (host.size() + 255) & ~size_t(255);
+    host.resize(off + v.size() * sizeof(T));
+    if (!v.empty()) std::memcpy(host.data() + off, v.data(), v.size() * sizeof(T));
+    const size_t n = v.size();
+    place.push_back([&b, off, n](char* base) { b.view(reinterpret_cast<T*>(base + off), n); });
+  }
+  void upload(DBuf<char>& all, hipStream_t s) {
+    all.upload(host.data(), host.size(), s);
+    for (auto& f : place) f(all.p);
+  }
+};
+
 // Recursive coordinate bisection of the bases in [b, e): `units` units of
 // `unit` bases each (the last one possibly short), cut across the widest
 // extent of their centres c so that the lower side holds a whole number of
@@ -246,6 +323,7 @@ void finalize_rwg(dm_rwg& r) {
   r.eminus.resize(n);
   std::vector<int> hrwg_ext(nt * 3, -1);
   std::vector<double> hsig(nt * 3, 0.0);
+  const std::vector<double>& mesh_area = triangle_areas(m);
   auto locate = [&](i64 t, i64 vopp, const char* side, i64 idx) {
     DM_REQUIRE(t >= 1 && t <= nt, DM_ERR_ARGUMENT,
                std::string("RWG ") + std::to_string(idx + 1) + ": " + side + " triangle out of range");
@@ -273,25 +351,17 @@ void finalize_rwg(dm_rwg& r) {
     // f_n = sigma * len/(2 A_rwg) * (r - v_opp); quadrature weights use the mesh
     // area, so the half carries sigma * A_mesh / A_rwg (exactly sigma when the
     // caller's areas are the mesh's own).
-    hsig[hp] = r.coeff_p[i] * (triangle_area(m, r.tplus[i] - 1) / r.area_p[i]);
-    hsig[hm] = -r.coeff_m[i] * (triangle_area(m, r.tminus[i] - 1) / r.area_m[i]);
+    hsig[hp] = r.coeff_p[i] * (mesh_area[r.tplus[i] - 1] / r.area_p[i]);
+    hsig[hm] = -r.coeff_m[i] * (mesh_area[r.tminus[i] - 1] / r.area_m[i]);
   }
   // Edge adjacency, src/assembly/EFIE.jl:140-231: triangles sharing a recorded edge.
-  std::vector<std::tuple<i64, i64, int>> rec;
-  rec.reserve(3 * nt);
-  for (i64 t = 0; t < nt; ++t)
-    for (int j = 0; j < 3; ++j) {
-      i64 a = m.tri[3 * t + j], b = m.tri[3 * t + (j + 1) % 3];
-      rec.emplace_back(std::min(a, b), std::max(a, b), (int)t);
-    }
-  std::sort(rec.begin(), rec.end());
+  const std::vector<Side> rec = sorted_sides(m);
   std::vector<std::pair<int, int>> pairs;
   for (size_t i = 0; i < rec.size();) {
-    size_t j = i + 1;
-    while (j < rec.size() && std::get<0>(rec[j]) == std::get<0>(rec[i]) && std::get<1>(rec[j]) == std::get<1>(rec[i])) ++j;
+    const size_t j = run_end(rec, i);
     for (size_t a = i; a < j; ++a)
       for (size_t b = a + 1; b < j; ++b) {
-        int t1 = std::get<2>(rec[a]), t2 = std::get<2>(rec[b]);
+        int t1 = (int)(rec[a].idx / 3), t2 = (int)(rec[b].idx / 3);
         if (t1 != t2) pairs.emplace_back(std::min(t1, t2), std::max(t1, t2));
       }
     i = j;
@@ -380,18 +450,20 @@ void finalize_rwg(dm_rwg& r) {
     em[i] = r.eminus[e];
   }
   hipStream_t s = r.ctx->stream;
-  r.d_ext.upload(r.ext_of_int, s);
-  r.d_iofe.upload(r.int_of_ext, s);
-  r.d_len.upload(len_i, s);
-  r.d_hrwg.upload(hrwg, s);
-  r.d_hsig.upload(hsig, s);
-  r.d_nb.upload(r.nb, s);
-  r.d_blk_off.upload(r.blk_off, s);
-  r.d_blk_tri.upload(r.blk_tri, s);
-  r.d_tplus_i.upload(tp, s);
-  r.d_tminus_i.upload(tm, s);
-  r.d_eplus_i.upload(ep, s);
-  r.d_eminus_i.upload(em, s);
+  Packed pk;
+  pk.add(r.d_ext, r.ext_of_int);
+  pk.add(r.d_iofe, r.int_of_ext);
+  pk.add(r.d_len, len_i);
+  pk.add(r.d_hrwg, hrwg);
+  pk.add(r.d_hsig, hsig);
+  pk.add(r.d_nb, r.nb);
+  pk.add(r.d_blk_off, r.blk_off);
+  pk.add(r.d_blk_tri, r.blk_tri);
+  pk.add(r.d_tplus_i, tp);
+  pk.add(r.d_tminus_i, tm);
+  pk.add(r.d_eplus_i, ep);
+  pk.add(r.d_eminus_i, em);
+  pk.upload(r.d_all, s);
   HIP_OK(hipStreamSynchronize(s));
 }
 
@@ -538,7 +610,8 @@ const TriTables& tables(dm_rwg& r, int quad_order) {
   double xi[14], w[7], xi7[14], w7[7];
   int nq = quad_rule(quad_order, xi, w);
   quad_rule(7, xi7, w7);
-  std::vector<double> cen(nt * 3), uq(nt * nq * 3), av(nt * 9), rq(nt * nq * 3), rq7(nt * 21), vtx(nt * 9), area(nt);
+  std::vector<double> cen(nt * 3), uq(nt * nq * 3), av(nt * 9), rq(nt * nq * 3), rq7(nt * 21), vtx(nt * 9);
+  const std::vector<double>& area = triangle_areas(m);
   auto affine = [](double a, double b, double c, double x1, double x2) {
     double w1 = 1.0 - x1 - x2;
     return std::fma(w1, a, std::fma(x1, b, x2 * c));
@@ -569,19 +642,18 @@ const TriTables& tables(dm_rwg& r, int quad_order) {
       rq7[(t * 7 + q) * 3 + 1] = affine(v[0].y, v[1].y, v[2].y, xi7[2 * q], xi7[2 * q + 1]);
       rq7[(t * 7 + q) * 3 + 2] = affine(v[0].z, v[1].z, v[2].z, xi7[2 * q], xi7[2 * q + 1]);
     }
-    area[t] = triangle_area(m, t);
   }
   hipStream_t s = r.ctx->stream;
   T.nq = nq;
-  T.cen.upload(cen, s);
-  T.uq.upload(uq, s);
-  T.av.upload(av, s);
-  T.rq.upload(rq, s);
-  T.rq7.upload(rq7, s);
-  T.vtx.upload(vtx, s);
-  T.area.upload(area, s);
-  T.h_rq = rq;
-  T.h_area = area;
+  Packed pk;
+  pk.add(T.cen, cen);
+  pk.add(T.uq, uq);
+  pk.add(T.av, av);
+  pk.add(T.rq, rq);
+  pk.add(T.rq7, rq7);
+  pk.add(T.vtx, vtx);
+  pk.add(T.area, area);
+  pk.upload(T.all, s);
   HIP_OK(hipStreamSynchronize(s));
   T.quad_order = quad_order;
   return T;

@@ -231,10 +231,6 @@ int mp_guard(F&& f) {
   }
 }
 
-struct Scope {
-  std::lock_guard<std::mutex> lk;
-  explicit Scope(dm_ctx* c) : lk(c->mu) { HIP_OK(hipSetDevice(c->device)); }
-};
 }  // namespace
 
 extern "C" {
@@ -245,7 +241,7 @@ int dm_mpnn_create(dm_ctx* ctx, const float* params, dm_mpnn** out) {
   return mp_guard([&] {
     DM_REQUIRE(ctx && params && out, DM_ERR_ARGUMENT, "NULL argument");
     for (int i = 0; i < dmn::NPARAM; ++i) DM_REQUIRE(std::isfinite(params[i]), DM_ERR_ARGUMENT, "parameters must be finite");
-    Scope sc(ctx);
+    CtxScope sc(ctx);
     hipStream_t s = ctx->stream;
     auto net = std::make_unique<dm_mpnn>();
     net->ctx = ctx;
@@ -266,7 +262,7 @@ int dm_mpnn_create(dm_ctx* ctx, const float* params, dm_mpnn** out) {
 int dm_mpnn_get_params(const dm_mpnn* net, float* out) {
   return mp_guard([&] {
     DM_REQUIRE(net && out, DM_ERR_ARGUMENT, "NULL argument");
-    Scope sc(net->ctx);
+    CtxScope sc(net->ctx);
     HIP_OK(hipMemcpy(out, net->p.p, net->p.bytes(), hipMemcpyDeviceToHost));
   });
 }
@@ -274,7 +270,7 @@ int dm_mpnn_get_params(const dm_mpnn* net, float* out) {
 int dm_mpnn_free(dm_mpnn* net) {
   return mp_guard([&] {
     if (!net) return;
-    Scope sc(net->ctx);
+    FreeScope sc(net->ctx);
     delete net;
   });
 }
@@ -317,7 +313,7 @@ int dm_mpnn_data_create(dm_ctx* ctx, int64_t nnode, const int32_t* nbr, const fl
         dinv[i] = 1.0f / (float)std::max(deg, 1);
       }
     }
-    Scope sc(ctx);
+    CtxScope sc(ctx);
     hipStream_t s = ctx->stream;
     auto d = std::make_unique<dm_mpnn_data>();
     d->ctx = ctx;
@@ -346,7 +342,7 @@ int dm_mpnn_residual_operator(dm_ctx* ctx, const dm_zmat* z, const dm_precond* p
     DM_REQUIRE(z->forms & DM_Z64, DM_ERR_ARGUMENT, "the operator needs the full complex128 matrix (DM_Z64)");
     const i64 n = z->n;
     DM_REQUIRE(n <= 16384, DM_ERR_ARGUMENT, "training operators are limited to 16384 bases");
-    Scope sc(ctx);
+    CtxScope sc(ctx);
     hipStream_t s = ctx->stream;
     // S as a dense internal-order matrix (S applied to the identity), then
     // A = Z S on the FP64 matrix cores, then the node-order complex64 copy
@@ -375,7 +371,7 @@ int dm_mpnn_data_set_matrix(dm_mpnn_data* d, int64_t s0, int64_t s1, const float
     for (int64_t k = s0; k < s1; ++k)
       DM_REQUIRE(d->ptr[k + 1] - d->ptr[k] == n, DM_ERR_ARGUMENT, "a sample's node count differs from the operator order");
     for (i64 i = 0; i < 2 * n * n; ++i) DM_REQUIRE(std::isfinite(a[i]), DM_ERR_ARGUMENT, "operator entries must be finite");
-    Scope sc(d->ctx);
+    CtxScope sc(d->ctx);
     hipStream_t s = d->ctx->stream;
     if (d->mat_of.empty()) d->mat_of.assign(d->ns, -1);
     if (d->p.n == 0) d->p.alloc(2 * d->nnode);
@@ -392,7 +388,7 @@ int dm_mpnn_data_set_matrix(dm_mpnn_data* d, int64_t s0, int64_t s1, const float
 int dm_mpnn_data_free(dm_mpnn_data* d) {
   return mp_guard([&] {
     if (!d) return;
-    Scope sc(d->ctx);
+    FreeScope sc(d->ctx);
     delete d;
   });
 }
@@ -404,7 +400,7 @@ int dm_mpnn_loss_grad(dm_ctx* ctx, dm_mpnn* net, const dm_mpnn_data* d, int64_t 
     DM_REQUIRE(net->ctx == ctx && d->ctx == ctx, DM_ERR_ARGUMENT, "objects belong to another context");
     DM_REQUIRE(s0 >= 0 && s0 < s1 && s1 <= d->ns, DM_ERR_ARGUMENT, "sample range out of bounds");
     require_operators(*d, s0, s1);
-    Scope sc(ctx);
+    CtxScope sc(ctx);
     hipStream_t s = ctx->stream;
     Work w;
     w.loss.alloc(1);
@@ -423,7 +419,7 @@ int dm_mpnn_train(dm_ctx* ctx, dm_mpnn* net, const dm_mpnn_data* d, int epochs, 
     DM_REQUIRE(epochs >= 1 && batch_samples >= 1, DM_ERR_ARGUMENT, "epochs and batch size must be positive");
     DM_REQUIRE(std::isfinite(lr) && lr > 0, DM_ERR_ARGUMENT, "learning rate must be finite and positive");
     require_operators(*d, 0, d->ns);
-    Scope sc(ctx);
+    CtxScope sc(ctx);
     hipStream_t s = ctx->stream;
     std::vector<std::pair<int, int>> batches;
     for (int a = 0; a < d->ns; a += (int)batch_samples) batches.push_back({a, std::min<int>(d->ns, a + (int)batch_samples)});
@@ -459,7 +455,7 @@ int dm_mpnn_apply(dm_ctx* ctx, const dm_mpnn* net, const dm_rwg* rwg, double k, 
   return mp_guard([&] {
     DM_REQUIRE(ctx && net && rwg && z && r && out, DM_ERR_ARGUMENT, "NULL argument");
     DM_REQUIRE(net->ctx == ctx && rwg->ctx == ctx, DM_ERR_ARGUMENT, "objects belong to another context");
-    Scope sc(ctx);
+    CtxScope sc(ctx);
     hipStream_t s = ctx->stream;
     const i64 n = rwg->n;
     std::vector<int> nbr;
