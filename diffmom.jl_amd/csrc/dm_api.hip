@@ -1185,13 +1185,32 @@ int dm_farfield(dm_ctx* ctx, const dm_rwg* rwg, const double* rhat, int64_t nome
     const TriTables& T = dmh::tables(r, quad_order);
     hipStream_t s = ctx->stream;
     const i64 n = r.n;
-    // radiation vectors of a chunk of directions (<= ~1 GiB), then E = G I on
-    // the matrix cores, column by column of currents in blocks of 1024
-    const i64 chunk = std::max<i64>(1, std::min<i64>(nomega, (1LL << 30) / (48 * std::max<i64>(n, 1))));
-    const int RB = (int)std::min<i64>(ncur, 1024);
-    DBuf<double> dr, dg, di, de, ws;
+    DBuf<double> dr, dg, di, de, ws, part;
     dr.upload(rhat, 3 * nomega, s);
-    dg.alloc((size_t)2 * 3 * chunk * n);
+    if (dmf::farfield_direct(ncur)) {
+      // few currents: straight from the quadrature points
+      const i64 chunk = std::min<i64>(nomega, 1 << 16);
+      di.alloc((size_t)2 * n * ncur);
+      de.alloc((size_t)2 * 3 * chunk * ncur);
+      ws.alloc(dmf::farfield_direct_ws(r, T, chunk));
+      HIP_OK(hipMemcpy2DAsync(di.p, 16 * n, I, 16 * ldi, 16 * n, ncur, hipMemcpyHostToDevice, s));
+      for (i64 q0 = 0; q0 < nomega; q0 += chunk) {
+        const i64 nq = std::min(chunk, nomega - q0);
+        for (i64 j = 0; j < ncur; j += dmf::kFfCurrents) {
+          ProfScope p(ctx, "farfield_direct", s);
+          dmf::farfield_few(r, T, dr.p + 3 * q0, nq, k, eta0, di.p + 2 * n * j, n,
+                            (int)std::min<i64>(dmf::kFfCurrents, ncur - j), de.p + 6 * nq * j, 3 * nq, ws.p, s);
+        }
+        HIP_OK(hipMemcpy2DAsync(E + 2 * 3 * q0, 16 * lde, de.p, 16 * 3 * nq, 16 * 3 * nq, ncur, hipMemcpyDeviceToHost, s));
+      }
+      HIP_OK(hipStreamSynchronize(s));
+      return;
+    }
+    // transverse radiation vectors of a chunk of directions (<= ~1 GiB), then
+    // E = G I on the matrix cores, column by column of currents in blocks of 1024
+    const i64 chunk = std::max<i64>(1, std::min<i64>(std::min<i64>(nomega, 1 << 18), (1LL << 30) / (32 * std::max<i64>(n, 1))));
+    const int RB = (int)std::min<i64>(ncur, 1024);
+    dg.alloc((size_t)2 * 2 * chunk * n);
     di.alloc((size_t)2 * n * RB);
     de.alloc((size_t)2 * 3 * chunk * RB);
     ws.alloc(dml::gemm_c128_workspace_bytes(n, RB) / sizeof(double));
@@ -1202,11 +1221,14 @@ int dm_farfield(dm_ctx* ctx, const dm_rwg* rwg, const double* rhat, int64_t nome
         const i64 nq = std::min(chunk, nomega - q0);
         {
           ProfScope p(ctx, "radiation", s);
-          dmf::radiation_vectors(r, T, dr.p + 3 * q0, nq, k, eta0, dg.p, s);
+          dmf::radiation_uv(r, T, dr.p + 3 * q0, nq, k, eta0, dg.p, s);
         }
         {
           ProfScope p(ctx, "farfield_gemm", s);
-          dml::gemm_c128(3 * nq, n, dg.p, 3 * nq, di.p, n, R, de.p, 3 * nq, ws.p, s);
+          const int nk = dml::gemm_c128_split(2 * nq, n, R);
+          if (part.n < (size_t)2 * nk * 2 * nq * R) part.alloc((size_t)2 * nk * 2 * nq * R);
+          dml::gemm_c128_parts(2 * nq, n, dg.p, 2 * nq, di.p, n, R, nk, part.p, ws.p, s);
+          dmf::farfield_join(nq, R, nk, dr.p + 3 * q0, part.p, de.p, 3 * nq, s);
         }
         HIP_OK(hipMemcpy2DAsync(E + 2 * (lde * j0 + 3 * q0), 16 * lde, de.p, 16 * 3 * nq, 16 * 3 * nq, R,
                                 hipMemcpyDeviceToHost, s));

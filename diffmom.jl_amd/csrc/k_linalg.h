@@ -107,6 +107,12 @@ void zx_bf16(i64 n, i64 ld, const void* planes, const double* X, i64 ldx, int R,
 size_t gemm_c128_workspace_bytes(i64 n, int R);
 void gemm_c128(i64 mr, i64 n, const double* A, i64 lda, const double* X, i64 ldx, int R, double* Y, i64 ldy,
                void* ws, hipStream_t s, bool subtract = false);
+// The same product in nk parts of the inner dimension (gemm_c128_split(mr, n,
+// R) of them, enough workgroups to fill the chip), part c at part + 2 c mr R
+// (column-major mr x R), to be added by the caller.
+int gemm_c128_split(i64 mr, i64 n, int R);
+void gemm_c128_parts(i64 mr, i64 n, const double* A, i64 lda, const double* X, i64 ldx, int R, int nk, double* part,
+                     void* ws, hipStream_t s);
 void zx_mfma64(i64 n, i64 ld, const double* z64, const double* X, i64 ldx, int R, double* Y, i64 ldy, void* ws,
                hipStream_t s);
 }  // namespace dml
@@ -116,6 +122,20 @@ namespace dmf {
 // written at row out_idx[i] (identity or caller order).
 void planewave(const dm_rwg& r, const TriTables& t, const double* kvec, const double* pol, const double* E0, int M,
                const int* out_idx, double* V, i64 ldv, hipStream_t s);
+// Far fields E = G I (3 nomega x R) of currents in caller order.  Few currents
+// (farfield_direct): directly from the quadrature points, kFfCurrents at a time;
+// more: radiation_uv forms the transverse components of G (2 nomega x n, caller
+// basis order), gemm_c128_parts multiplies, farfield_join adds the partial
+// products and restores x, y, z.
+constexpr int kFfCurrents = 4;
+bool farfield_direct(i64 ncur);
+size_t farfield_direct_ws(const dm_rwg& r, const TriTables& t, i64 nomega);
+void farfield_few(const dm_rwg& r, const TriTables& t, const double* rhat, i64 nomega, double k, double eta0,
+                  const double* I, i64 ldi, int R, double* E, i64 lde, double* ws, hipStream_t s);
+void radiation_uv(const dm_rwg& r, const TriTables& t, const double* rhat, i64 nomega, double k, double eta0,
+                  double* G, hipStream_t s);
+void farfield_join(i64 nomega, int R, int nk, const double* rhat, const double* part, double* E, i64 lde,
+                   hipStream_t s);
 void radiation_vectors(const dm_rwg& r, const TriTables& t, const double* rhat, i64 nomega, double k, double eta0,
                        double* G, hipStream_t s);
 }  // namespace dmf
