@@ -15,7 +15,7 @@
 namespace {
 
 constexpr int BT = 256;          // threads per workgroup
-constexpr int BROWS = 16;        // rows per thread in the dot kernel (one wave reduction per 16 KB read)
+constexpr int BROWS = 8;         // rows per thread in the dot kernel (one wave reduction per 8 KB read)
 constexpr int BCHUNK = BT * BROWS;
 constexpr int BKMAX = 512;       // basis vectors per column
 
@@ -25,8 +25,30 @@ __device__ inline double wsum(double v) {
   return v;
 }
 
+// v plus the lanes one DPP step away (lanes outside the row mask add zero)
+template <int CTRL, int ROWS>
+__device__ inline double dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b & 0xffffffffLL), CTRL, ROWS, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xF, false);
+  return v + __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+// sum over the wave, in lane 63
+__device__ inline double wsum63(double x) {
+  x = dpp_add<0xB1, 0xF>(x);   // quad_perm 1,0,3,2
+  x = dpp_add<0x4E, 0xF>(x);   // quad_perm 2,3,0,1
+  x = dpp_add<0x141, 0xF>(x);  // row_half_mirror
+  x = dpp_add<0x140, 0xF>(x);  // row_mirror
+  x = dpp_add<0x142, 0xA>(x);  // row_bcast15
+  return dpp_add<0x143, 0xC>(x);  // row_bcast31
+}
+
 // part[(r * kcap + i) * nch + c] = sum over the rows of chunk c of conj(V_i[r]) . W[r]
-// (each workgroup keeps its chunk of W[r] in registers and walks the k basis vectors)
+// (each workgroup keeps its chunk of W[r] in registers and walks the k basis
+// vectors).  HBM-bound: the next vector's loads are issued before this one's
+// sums (rows past n read row n - 1 against w = 0: a load behind a branch made
+// every row wait for the one before it: 0.47 against 0.44 ms on average for
+// bases of 1 to 58 vectors, 30720 rows, 128 columns).
 __global__ __launch_bounds__(BT) void k_bdots(i64 n, int R, int k, int kcap, const double2* __restrict__ V,
                                               const double2* __restrict__ W, const int* __restrict__ act,
                                               double2* __restrict__ part, int nch) {
@@ -35,28 +57,33 @@ __global__ __launch_bounds__(BT) void k_bdots(i64 n, int R, int k, int kcap, con
   __shared__ double2 red[BT / 64][BKMAX];
   const i64 base = (i64)c * BCHUNK + threadIdx.x;
   const i64 NR = n * R;
-  double2 w[BROWS];
+  double2 w[BROWS], a[BROWS], nx[BROWS];
+  i64 row[BROWS];
 #pragma unroll
   for (int e = 0; e < BROWS; ++e) {
-    i64 m = base + e * BT;
-    w[e] = m < n ? W[(i64)r * n + m] : make_double2(0.0, 0.0);
+    const i64 m = base + e * BT;
+    row[e] = (i64)r * n + min(m, n - 1);
+    w[e] = W[row[e]];
+    if (m >= n) w[e] = make_double2(0.0, 0.0);
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int e = 0; e < BROWS; ++e) a[e] = V[row[e]];
   for (int i = 0; i < k; ++i) {
-    const double2* v = V + (i64)i * NR + (i64)r * n;
+    const double2* v = V + (i64)min(i + 1, k - 1) * NR;
+#pragma unroll
+    for (int e = 0; e < BROWS; ++e) nx[e] = v[row[e]];
     double ar = 0, ai = 0;
 #pragma unroll
     for (int e = 0; e < BROWS; ++e) {
-      i64 m = base + e * BT;
-      if (m < n) {
-        double2 a = v[m];
-        ar += a.x * w[e].x + a.y * w[e].y;
-        ai += a.x * w[e].y - a.y * w[e].x;
-      }
+      ar += a[e].x * w[e].x + a[e].y * w[e].y;
+      ai += a[e].x * w[e].y - a[e].y * w[e].x;
     }
-    ar = wsum(ar);
-    ai = wsum(ai);
-    if (lane == 0) red[wave][i] = make_double2(ar, ai);
+    ar = wsum63(ar);
+    ai = wsum63(ai);
+    if (lane == 63) red[wave][i] = make_double2(ar, ai);
+#pragma unroll
+    for (int e = 0; e < BROWS; ++e) a[e] = nx[e];
   }
   __syncthreads();
   for (int i = threadIdx.x; i < k; i += BT) {
@@ -86,7 +113,8 @@ __global__ void k_bdots_reduce(int R, int k, int kcap, int nch, const double2* _
 }
 
 // W[r] -= sum_{i<k} V_i[r] h[r, i]; each thread takes BUROWS rows (stride
-// BT), so a workgroup's staging of h serves BT * BUROWS rows
+// BT), so a workgroup's staging of h serves BT * BUROWS rows.  HBM-bound: 16
+// loads in flight per thread (rows past n read row n - 1).
 constexpr int BUROWS = 4;
 __global__ __launch_bounds__(BT) void k_bupdate(i64 n, int R, int k, int kcap, const double2* __restrict__ V,
                                                 const double2* __restrict__ h, const int* __restrict__ act,
@@ -97,26 +125,32 @@ __global__ __launch_bounds__(BT) void k_bupdate(i64 n, int R, int k, int kcap, c
   for (int i = threadIdx.x; i < k; i += BT) hs[i] = h[(i64)r * kcap + i];
   __syncthreads();
   const i64 m0 = blockIdx.x * (i64)(BT * BUROWS) + threadIdx.x;
-  const i64 NR = n * R, off = (i64)r * n + m0;
+  const i64 NR = n * R;
+  i64 row[BUROWS];
   double ar[BUROWS], ai[BUROWS];
 #pragma unroll
-  for (int u = 0; u < BUROWS; ++u) ar[u] = ai[u] = 0.0;
+  for (int u = 0; u < BUROWS; ++u) {
+    row[u] = (i64)r * n + min(m0 + BT * u, n - 1);
+    ar[u] = ai[u] = 0.0;
+  }
+#pragma unroll 4
   for (int i = 0; i < k; ++i) {
     const double2 b = hs[i];
+    const double2* v = V + (i64)i * NR;
+    double2 a[BUROWS];
+#pragma unroll
+    for (int u = 0; u < BUROWS; ++u) a[u] = v[row[u]];
 #pragma unroll
     for (int u = 0; u < BUROWS; ++u) {
-      if (m0 + BT * u < n) {
-        const double2 a = V[(i64)i * NR + off + BT * u];
-        ar[u] += a.x * b.x - a.y * b.y;
-        ai[u] += a.x * b.y + a.y * b.x;
-      }
+      ar[u] += a[u].x * b.x - a[u].y * b.y;
+      ai[u] += a[u].x * b.y + a[u].y * b.x;
     }
   }
 #pragma unroll
   for (int u = 0; u < BUROWS; ++u) {
     if (m0 + BT * u < n) {
-      const double2 o = W[off + BT * u];
-      W[off + BT * u] = make_double2(o.x - ar[u], o.y - ai[u]);
+      const double2 o = W[row[u]];
+      W[row[u]] = make_double2(o.x - ar[u], o.y - ai[u]);
     }
   }
 }
@@ -135,6 +169,7 @@ __global__ __launch_bounds__(BT) void k_bcombine(i64 n, int R, int kcap, const d
   if (m >= n) return;
   const i64 NR = n * R, off = (i64)r * n + m;
   double ar = 0, ai = 0;
+#pragma unroll 8
   for (int i = 0; i < k; ++i) {
     double2 a = V[(i64)i * NR + off], b = ys[i];
     ar += a.x * b.x - a.y * b.y;
