@@ -189,7 +189,12 @@ __global__ void k_split_planes64(i64 n, i64 np, int R, const double2* __restrict
 // four column blocks of a row block are dispatched back to back on one XCD,
 // which share its A' stages in L2.
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-constexpr int ZB_LDA = 40;  // bf16 per LDS row (32 + 8 padding)
+// LDS place of the 16-byte piece kq (rows 8 kq .. + 7 of the stage) of X column
+// col: a column's four pieces are permuted by its block of four, so that the
+// lanes a 16-byte read or write serves together (0-3, 12-15, 20-27, ...) hit
+// 16 different groups of four banks.  Rows padded to 40 values instead met in
+// pairs: a quarter of the kernel's cycles.
+__device__ inline int zb_at(int col, int kq) { return 4 * col + (kq ^ (-(col >> 2) & 3)); }
 
 __device__ inline void split3(float x, __bf16& h, __bf16& m, __bf16& l) {
   h = (__bf16)x;
@@ -245,12 +250,20 @@ __global__ void k_split_x_bf16(i64 n, i64 np, int R, int Rp, const double2* __re
 // NT = 6: the six part products (FP32 accuracy); NT = 3: h h', h m', m h'
 // only (the dropped terms are each below 2^-18 relative, ~1e-5 in all), for
 // relaxed products late in a Krylov solve.
+// n = 30720, R = 128: NT = 3 takes 2.75 ms (3.31 when all six X planes were
+// staged), NT = 6 4.9 ms = 1.19 PFLOP/s with the matrix cores 0.71 busy at the
+// 1.6 GHz that the power limit leaves (a plain 8192^3 bf16 product reaches the
+// same rate); n = 7680: 304 us (320 with bank conflicts).  128 complex rows
+// per workgroup (four row blocks per wave, or eight waves) measured 2 to 20 %
+// slower: one wave per SIMD, or more waves at one barrier.
 template <int NT>
 __global__ __launch_bounds__(256, 1) void k_zx_bf16(i64 n, i64 R2, int nrb, int ncb, const __bf16* __restrict__ Ap,
                                                     i64 aplane,
                                                     const __bf16* __restrict__ Xp, i64 np, i64 xplane, int R,
                                                     i64 kc, double2* __restrict__ part) {
-  __shared__ __align__(16) __bf16 Bs[2][6][ZX_BN][ZB_LDA];
+  constexpr int NA = NT == 6 ? 3 : 2, NP = 2 * NA;  // planes of A' and of X that the products use
+  constexpr int NB = NP * ZX_BN * 4 / 256;          // 16-byte pieces of an X stage per thread
+  __shared__ __align__(16) __bf16 Bs[2][NP][4 * ZX_BN][8];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // XCD-aware tile order: workgroup w runs on XCD w % 8; its index j = w / 8
   // on that XCD gives row block 8 (j / ncb) + w % 8 and column block j % ncb
@@ -267,29 +280,31 @@ __global__ __launch_bounds__(256, 1) void k_zx_bf16(i64 n, i64 R2, int nrb, int 
   // global memory straight into the MFMA operand layout (lane l: row l % 16,
   // columns 8 (l / 16) .. + 7 of the stage, one 16-byte load from the
   // 8-column-group planes).  X is shared by the four waves and staged in LDS
-  // (two buffers, one barrier per stage): 6 planes x 64 columns x 4 groups of
-  // 8 rows = 1536 16-byte pieces, 6 per thread.
+  // (two buffers, one barrier per stage): the planes that the products use (6,
+  // or 4 without the l parts) x 64 columns x 4 groups of 8 rows, NB 16-byte
+  // pieces per thread.
   const int g = lane >> 4;
   const i64 arow = 2 * m0 + 32 * wave + (lane & 15);
-  v8bf ra[3][2];
-  u4v rb[6];
+  v8bf ra[NA][2];
+  u4v rb[NB];
   auto gload = [&](i64 k0) {
 #pragma unroll
-    for (int q = 0; q < 3; ++q)
+    for (int q = 0; q < NA; ++q)
 #pragma unroll
       for (int r = 0; r < 2; ++r)
         ra[q][r] = *reinterpret_cast<const v8bf*>(Ap + q * aplane + ((k0 / 8 + g) * R2 + arow + 16 * r) * 8);
 #pragma unroll
-    for (int i = 0; i < 6; ++i) {
+    for (int i = 0; i < NB; ++i) {
       const int c = tid + 256 * i, q = c >> 8, rem = c & 255, col = rem >> 2, kq = rem & 3;
-      rb[i] = *reinterpret_cast<const u4v*>(Xp + q * xplane + (i64)(c0 + col) * np + k0 + 8 * kq);
+      const int pl = q < NA ? q : q - NA + 3;
+      rb[i] = *reinterpret_cast<const u4v*>(Xp + pl * xplane + (i64)(c0 + col) * np + k0 + 8 * kq);
     }
   };
   auto lstore = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < 6; ++i) {
+    for (int i = 0; i < NB; ++i) {
       const int c = tid + 256 * i, q = c >> 8, rem = c & 255, col = rem >> 2, kq = rem & 3;
-      *reinterpret_cast<u4v*>(&Bs[buf][q][col][8 * kq]) = rb[i];
+      *reinterpret_cast<u4v*>(&Bs[buf][q][zb_at(col, kq)][0]) = rb[i];
     }
   };
   v4f accP[2][4], accQ[2][4];
@@ -307,15 +322,15 @@ __global__ __launch_bounds__(256, 1) void k_zx_bf16(i64 n, i64 R2, int nrb, int 
     const int buf = st & 1;
     // all operands of the stage, then the six part products, each over the
     // wave's 16 independent accumulator tiles (no back-to-back dependence)
-    v8bf A[3][2], Br[3][4], Bi[3][4];
+    v8bf A[NA][2], Br[NA][4], Bi[NA][4];
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
+    for (int q = 0; q < NA; ++q) {
 #pragma unroll
       for (int r = 0; r < 2; ++r) A[q][r] = ra[q][r];
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) {
-        Br[q][cb] = *reinterpret_cast<const v8bf*>(&Bs[buf][q][16 * cb + (lane & 15)][8 * g]);
-        Bi[q][cb] = *reinterpret_cast<const v8bf*>(&Bs[buf][3 + q][16 * cb + (lane & 15)][8 * g]);
+        Br[q][cb] = *reinterpret_cast<const v8bf*>(&Bs[buf][q][zb_at(16 * cb + (lane & 15), g)][0]);
+        Bi[q][cb] = *reinterpret_cast<const v8bf*>(&Bs[buf][NA + q][zb_at(16 * cb + (lane & 15), g)][0]);
       }
     }
     if (st + 1 < nst) gload(k_begin + (i64)(st + 1) * 32);
