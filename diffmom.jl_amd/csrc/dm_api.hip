@@ -367,8 +367,7 @@ void solve_columns(dm_ctx* ctx, const dm_solve_opts& o, const dm_rwg& r, DevOp* 
       double res = solve_one(ctx, o, A64, A32, M, Bd + 2 * n * j, x.p, n, K, st, ok, z64_ready);
       worst = std::max(worst, res);
       all_ok = all_ok && ok;
-      launch_permute(n, r.d_ext.p, x.p, xe.p, 0, s);
-      if (conj_out) dml::conj(n, xe.p, s);
+      launch_permute_cols(n, 1, r.d_ext.p, x.p, n, xe.p, n, 0, conj_out, s);
       HIP_OK(hipMemcpyAsync(X + 2 * ldx * j, xe.p, 16 * n, hipMemcpyDeviceToHost, s));
     }
     HIP_OK(hipStreamSynchronize(s));
@@ -388,11 +387,10 @@ void solve_columns(dm_ctx* ctx, const dm_solve_opts& o, const dm_rwg& r, DevOp* 
     for (int c = 0; c < R; ++c) {
       st.iterations += iters[c];
       worst = std::max(worst, res[c]);
-      launch_permute(n, r.d_ext.p, Xb.p + 2 * n * c, xe.p + 2 * n * c, 0, s);
     }
+    launch_permute_cols(n, R, r.d_ext.p, Xb.p, n, xe.p, n, 0, conj_out, s);
     st.outer_iterations = std::max(st.outer_iterations, outer);
     all_ok = all_ok && ok;
-    if (conj_out) dml::conj(n * R, xe.p, s);
     HIP_OK(hipMemcpy2DAsync(X + 2 * ldx * j0, 16 * ldx, xe.p, 16 * n, 16 * n, R, hipMemcpyDeviceToHost, s));
     HIP_OK(hipStreamSynchronize(s));
   }
@@ -1000,12 +998,26 @@ int dm_apply(dm_ctx* ctx, const dm_zmat* z, int form, int adjoint, const double*
       yi.alloc(2 * n * R);
       ws.alloc(std::max<size_t>(op->batch_ws(R), 1));
       HIP_OK(hipMemcpy2DAsync(xe.p, 16 * n, X + 2 * ldx * j0, 16 * ldx, 16 * n, R, hipMemcpyHostToDevice, s));
-      if (adjoint) dml::conj(n * R, xe.p, s);
-      for (int j = 0; j < R; ++j) launch_permute(n, z->rwg->d_ext.p, xe.p + 2 * n * j, xi.p + 2 * n * j, 1, s);
-      op->apply_batch(xi.p, yi.p, R, ws.p, s);
-      for (int j = 0; j < R; ++j) launch_permute(n, z->rwg->d_ext.p, yi.p + 2 * n * j, xe.p + 2 * n * j, 0, s);
-      if (adjoint) dml::conj(n * R, xe.p, s);
-      HIP_OK(hipMemcpy2DAsync(Y + 2 * ldy * j0, 16 * ldy, xe.p, 16 * n, 16 * n, R, hipMemcpyDeviceToHost, s));
+      const int* ext = z->rwg->d_ext.p;
+      const double* out = xe.p;
+      if (R < kMfmaMinRhs && gemv_small_fits(n) && (form == DM_Z64 || form == DM_Z32)) {
+        ProfScope p(ctx, form == DM_Z64 ? "gemv_z64" : "gemv_z32", s);
+        for (int j = 0; j < R; ++j) {
+          const i64 at = 2 * n * j;
+          if (form == DM_Z64)
+            launch_gemv_small_z64(n, z->ld, z->z64.p, ext, xe.p + at, yi.p + at, adjoint != 0, s);
+          else
+            launch_gemv_small_z32(n, z->ld, z->z32.p, ext, xe.p + at, yi.p + at, adjoint != 0, s);
+        }
+        out = yi.p;
+      } else {
+        // one permutation launch per direction for all columns (64 columns of
+        // 7680: two launches a column took 0.3 ms)
+        launch_permute_cols(n, R, ext, xe.p, n, xi.p, n, 1, adjoint != 0, s);
+        op->apply_batch(xi.p, yi.p, R, ws.p, s);
+        launch_permute_cols(n, R, ext, yi.p, n, xe.p, n, 0, adjoint != 0, s);
+      }
+      HIP_OK(hipMemcpy2DAsync(Y + 2 * ldy * j0, 16 * ldy, out, 16 * n, 16 * n, R, hipMemcpyDeviceToHost, s));
       HIP_OK(hipStreamSynchronize(s));
     }
   });
@@ -1089,12 +1101,10 @@ int dm_mf_apply(dm_ctx* ctx, const dm_mfop* op, int adjoint, const double* x, do
     xi.alloc(2 * n);
     yi.alloc(2 * n);
     HIP_OK(hipMemcpyAsync(xe.p, x, 16 * n, hipMemcpyHostToDevice, s));
-    if (adjoint) dml::conj(n, xe.p, s);
-    launch_permute(n, r.d_ext.p, xe.p, xi.p, 1, s);
+    launch_permute_cols(n, 1, r.d_ext.p, xe.p, n, xi.p, n, 1, adjoint != 0, s);
     HIP_OK(hipMemsetAsync(yi.p, 0, 16 * n, s));
     launch_mf_apply(a, xi.p, yi.p, r.max_blk_tris, s);
-    launch_permute(n, r.d_ext.p, yi.p, xe.p, 0, s);
-    if (adjoint) dml::conj(n, xe.p, s);
+    launch_permute_cols(n, 1, r.d_ext.p, yi.p, n, xe.p, n, 0, adjoint != 0, s);
     HIP_OK(hipMemcpyAsync(y, xe.p, 16 * n, hipMemcpyDeviceToHost, s));
     HIP_OK(hipStreamSynchronize(s));
   });
@@ -1538,12 +1548,13 @@ int dm_solve(dm_ctx* ctx, const dm_zmat* z, const double* B, int64_t ldb, int64_
     bool all_ok = true;
     double worst = 0;
     DBuf<double> be, Bd;
-    be.alloc(2 * n);
+    constexpr i64 kCols = 64;  // columns staged in caller order per launch
+    be.alloc((size_t)2 * n * std::max<i64>(std::min(nrhs, kCols), 1));
     Bd.alloc((size_t)2 * n * std::max<i64>(nrhs, 1));
-    for (i64 j = 0; j < nrhs; ++j) {
-      HIP_OK(hipMemcpyAsync(be.p, B + 2 * ldb * j, 16 * n, hipMemcpyHostToDevice, s));
-      if (o.adjoint) dml::conj(n, be.p, s);
-      launch_permute(n, r.d_ext.p, be.p, Bd.p + 2 * n * j, 1, s);
+    for (i64 j = 0; j < nrhs; j += kCols) {
+      const i64 c = std::min(kCols, nrhs - j);
+      HIP_OK(hipMemcpy2DAsync(be.p, 16 * n, B + 2 * ldb * j, 16 * ldb, 16 * n, c, hipMemcpyHostToDevice, s));
+      launch_permute_cols(n, c, r.d_ext.p, be.p, n, Bd.p + 2 * n * j, n, 1, o.adjoint != 0, s);
     }
     solve_columns(ctx, o, r, A64.get(), A32.get(), M.get(), Bd.p, n, nrhs, X, ldx, st, worst, all_ok, nullptr,
                   o.adjoint != 0);

@@ -458,6 +458,13 @@ void launch_mf_apply(const AsmArgs& a, const double* x, double* y, int max_tris,
 // dense products (internal order, column-major, complex interleaved)
 void launch_gemv_z64(i64 n, i64 ld, const double* z, const double* x, double* y, hipStream_t s);
 void launch_gemv_z32(i64 n, i64 ld, const float* z, const double* x, double* y, hipStream_t s);
+// The same for a small matrix (gemv_small_fits), x and y in caller order (idx:
+// internal -> caller; they must not overlap); conj: Y = conj(Z conj(x)).
+bool gemv_small_fits(i64 n);
+void launch_gemv_small_z64(i64 n, i64 ld, const double* z, const int* idx, const double* x, double* y, bool conj,
+                           hipStream_t s);
+void launch_gemv_small_z32(i64 n, i64 ld, const float* z, const int* idx, const double* x, double* y, bool conj,
+                           hipStream_t s);
 
 // small vector kernels
 void launch_permute(i64 n, const int* idx, const double* src, double* dst, int gather, hipStream_t s);

@@ -99,8 +99,11 @@ __global__ __launch_bounds__(256) void k_gemv_z64(i64 n, i64 ld, const double2* 
 
 // y = Z x with complex64 storage and FP64 arithmetic (the product is HBM
 // bound, so FP64 accumulation costs nothing).  Lane reads two consecutive
-// entries (16 bytes) per column.
-template <int NC>
+// entries (16 bytes) per column, U steps' loads ahead of their sums (a step past
+// the end reads the last pair and is left out).  Two columns a wave and two
+// steps: 7698 unknowns 89 us = 5.3 TB/s, 30720: 5.6; four columns and one step
+// at a time had too few waves and loads in flight (7698: 158 us = 3.0 TB/s).
+template <int NC, int U>
 __global__ __launch_bounds__(256) void k_gemv_z32(i64 n, i64 ld, const float4* __restrict__ z4,
                                                   const double2* __restrict__ x, double2* __restrict__ y) {
   const int lane = threadIdx.x & 63;
@@ -111,14 +114,29 @@ __global__ __launch_bounds__(256) void k_gemv_z32(i64 n, i64 ld, const float4* _
   for (int c = 0; c < NC; ++c) ar[c] = ai[c] = 0.0;
   const i64 ld2 = ld >> 1;  // ld is even
   const i64 n2 = n >> 1;
-  for (i64 m2 = lane; m2 < n2; m2 += 64) {
-    double2 x0 = x[2 * m2], x1 = x[2 * m2 + 1];
+  const float4* zc[NC];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      i64 col = c0 + c < n ? c0 + c : c0;
-      float4 a = ld_stream(z4 + col * ld2 + m2);
-      ar[c] += (double)a.x * x0.x - (double)a.y * x0.y + (double)a.z * x1.x - (double)a.w * x1.y;
-      ai[c] += (double)a.x * x0.y + (double)a.y * x0.x + (double)a.z * x1.y + (double)a.w * x1.x;
+  for (int c = 0; c < NC; ++c) zc[c] = z4 + (c0 + c < n ? c0 + c : c0) * ld2;
+  for (i64 m2 = lane; m2 < n2; m2 += 64 * U) {
+    float4 a[U][NC];
+    double2 x0[U], x1[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const i64 q = min(m2 + 64 * u, n2 - 1);
+      x0[u] = x[2 * q];
+      x1[u] = x[2 * q + 1];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) a[u][c] = ld_stream(zc[c] + q);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (m2 + 64 * u >= n2) break;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const float4 v = a[u][c];
+        ar[c] += (double)v.x * x0[u].x - (double)v.y * x0[u].y + (double)v.z * x1[u].x - (double)v.w * x1[u].y;
+        ai[c] += (double)v.x * x0[u].y + (double)v.y * x0[u].x + (double)v.z * x1[u].y + (double)v.w * x1[u].x;
+      }
     }
   }
   if ((n & 1) && lane == 0) {
@@ -138,6 +156,47 @@ __global__ __launch_bounds__(256) void k_gemv_z32(i64 n, i64 ld, const float4* _
     double sr = wave_sum(ar[c]), si = wave_sum(ai[c]);
     if (lane == 0 && c0 + c < n) y[c0 + c] = make_double2(sr, si);
   }
+}
+
+// y = Z x of a small matrix with x and y in caller order (idx: internal ->
+// caller), conjugated on the way in and out for the adjoint: one launch instead
+// of gather, product and scatter.  Latency-bound: the workgroup gathers x into
+// LDS while each wave's first eight loads of its column are in flight.
+template <class T>
+__global__ __launch_bounds__(256) void k_gemv_small(i64 n, i64 ld, const T* __restrict__ z, const int* __restrict__ idx,
+                                                    const double2* __restrict__ x, double2* __restrict__ y, int conj) {
+  extern __shared__ double2 xs[];  // n
+  const int lane = threadIdx.x & 63;
+  const i64 c = (i64)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const T* zc = z + min(c, n - 1) * ld;
+  const double sg = conj ? -1.0 : 1.0;
+  T a[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) a[u] = zc[min((i64)lane + 64 * u, n - 1)];
+  const int ic = idx[min(c, n - 1)];
+  for (i64 m = threadIdx.x; m < n; m += 256) {
+    const double2 v = x[idx[m]];
+    xs[m] = make_double2(v.x, sg * v.y);
+  }
+  __syncthreads();
+  double ar = 0, ai = 0;
+  for (i64 m0 = lane; m0 < n; m0 += 512) {
+    T b[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) b[u] = zc[min(m0 + 512 + 64 * u, n - 1)];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (m0 + 64 * u < n) {
+        const double2 v = xs[m0 + 64 * u];
+        ar += (double)a[u].x * v.x - (double)a[u].y * v.y;
+        ai += (double)a[u].x * v.y + (double)a[u].y * v.x;
+      }
+      a[u] = b[u];
+    }
+  }
+  ar = wave_sum_dpp(ar);
+  ai = wave_sum_dpp(ai);
+  if (lane == 0 && c < n) y[ic] = make_double2(ar, sg * ai);
 }
 
 // One column per blockIdx.y; conj: the conjugated values.
@@ -658,10 +717,33 @@ void launch_gemv_z64(i64 n, i64 ld, const double* z, const double* x, double* y,
 }
 
 void launch_gemv_z32(i64 n, i64 ld, const float* z, const double* x, double* y, hipStream_t s) {
-  constexpr int NC = 4;
+  constexpr int NC = 2;
   DM_REQUIRE((ld & 1) == 0, DM_ERR_ARGUMENT, "complex64 matrix leading dimension must be even");
-  k_gemv_z32<NC><<<nblocks(n, 4 * NC), 256, 0, s>>>(
+  k_gemv_z32<NC, 2><<<nblocks(n, 4 * NC), 256, 0, s>>>(
       n, ld, reinterpret_cast<const float4*>(z), reinterpret_cast<const double2*>(x), reinterpret_cast<double2*>(y));
+  HIP_OK(hipGetLastError());
+}
+
+// Up to 3072 unknowns (48 KB of x in LDS, three workgroups per CU); past that
+// the product itself is HBM-bound and x is better read in order.  A whole
+// product call from the host, us, three launches / one, complex128: 79 unknowns
+// 40 / 36, 1473: 49 / 42, 2907: 63.5 / 62.5, 3804: 77 / 84; complex64: 1473: 46
+// / 41.5, 2907: 58.5 / 54, 4030: 67 / 74.
+bool gemv_small_fits(i64 n) { return n <= 3072; }
+
+void launch_gemv_small_z64(i64 n, i64 ld, const double* z, const int* idx, const double* x, double* y, bool conj,
+                           hipStream_t s) {
+  k_gemv_small<double2><<<nblocks(n, 4), 256, sizeof(double2) * n, s>>>(
+      n, ld, reinterpret_cast<const double2*>(z), idx, reinterpret_cast<const double2*>(x),
+      reinterpret_cast<double2*>(y), conj ? 1 : 0);
+  HIP_OK(hipGetLastError());
+}
+
+void launch_gemv_small_z32(i64 n, i64 ld, const float* z, const int* idx, const double* x, double* y, bool conj,
+                           hipStream_t s) {
+  k_gemv_small<float2><<<nblocks(n, 4), 256, sizeof(double2) * n, s>>>(
+      n, ld, reinterpret_cast<const float2*>(z), idx, reinterpret_cast<const double2*>(x),
+      reinterpret_cast<double2*>(y), conj ? 1 : 0);
   HIP_OK(hipGetLastError());
 }
 
