@@ -20,57 +20,65 @@
 
 namespace {
 
-constexpr int SPAI_MAXJ = 80;   // columns per least-squares problem (LDS bound)
-constexpr int SPAI_CHUNK = 8;   // rows of A staged per pass
+constexpr int SPAI_MAXJ = 80;  // columns per least-squares problem
+constexpr int SPAI_CHUNK = 8;  // rows of A staged per pass
 
-// One column per workgroup.  LDS holds, for the widest support mJ of the
-// pattern (not the cap), the Gram matrix's lower triangle packed by rows
-// (entry (a, b), b <= a, at a (a + 1) / 2 + b), SPAI_CHUNK staged rows of A,
-// the right-hand side and the support's column ids: about 27 KB at mJ = 49,
-// so five columns share a CU (with at most 102 VGPRs: five waves per SIMD).  The four waves form the Gram matrix (each
-// thread owns 2 x 2 blocks of it: one LDS read per complex multiply-add, two
-// barriers per chunk of rows); the Cholesky factorization (left-looking)
-// and the two triangular solves (right-hand side in registers, each solved
-// entry broadcast by a lane read) are then wave 0's alone, ordered by
-// wave-level fences instead of workgroup barriers (the other waves return).
-__device__ inline int tri(int a, int b) { return a * (a + 1) / 2 + b; }
+// One column per workgroup of NT threads; thread t owns one 4 x 4 block (A, B)
+// of the lower triangle of the extended Gram matrix [G, rhs; rhs^H, 1], held in
+// registers from the first row of A to the solution:
+//   Gram: chunks of SPAI_CHUNK rows staged in LDS (two buffers; the next chunk's
+//     entries are on their way while this one's products are formed); per row a
+//     thread reads 8 values for 16 complex products.
+//   Cholesky, right-looking by block columns: the diagonal block's thread
+//     factors it, the blocks below solve against it and put their result in LDS,
+//     the blocks to the right subtract their products.  The extended row turns
+//     into y^H = (L^-1 rhs)^H on the way.
+//   Backward: per block column the diagonal's thread solves its four entries and
+//     the blocks to its left in that row take them out of y.
+// The largest NT is bound by FP64 arithmetic in the Gram part, the small ones by
+// the serial steps, of which several workgroups per CU overlap.
+// 4720 columns, supports of 80 and about 200 rows: 1.25 ms (Gram matrix in LDS,
+// factorization and solves by one wave: 3.2); 30720 of 49: 2.1 ms (2.9).
+// Blocks are numbered down block columns, so that the waves of finished columns
+// drop out of the later steps.
+template <int NT>
+struct SpaiShape;  // NB: block rows (NB (NB + 1) / 2 <= NT)
+template <>
+struct SpaiShape<64> {
+  static constexpr int NB = 10;
+};
+template <>
+struct SpaiShape<128> {
+  static constexpr int NB = 15;
+};
+template <>
+struct SpaiShape<256> {
+  static constexpr int NB = 22;
+};
 
-// (a, b) with b <= a from the packed lower-triangle index e = a (a + 1) / 2 + b
-__device__ inline void untri(int e, int& a, int& b) {
-  a = (int)((sqrtf(8.0f * (float)e + 1.0f) - 1.0f) * 0.5f);
-  while (a * (a + 1) / 2 > e) --a;
-  while ((a + 1) * (a + 2) / 2 <= e) ++a;
-  b = e - a * (a + 1) / 2;
+// a -= p conj(q)
+__device__ inline void csub_pq(double2& a, double2 p, double2 q) {
+  a.x = fma(-p.x, q.x, a.x);
+  a.x = fma(-p.y, q.y, a.x);
+  a.y = fma(-p.y, q.x, a.y);
+  a.y = fma(p.x, q.y, a.y);
+}
+// a += conj(p) q
+__device__ inline void cacc_pq(double2& a, double2 p, double2 q) {
+  a.x = fma(p.x, q.x, a.x);
+  a.x = fma(p.y, q.y, a.x);
+  a.y = fma(p.x, q.y, a.y);
+  a.y = fma(-p.y, q.x, a.y);
 }
 
-// The lanes of one wave see each other's earlier LDS writes after this point
-// (a code-motion barrier between wavefront-scope release and acquire fences).
-__device__ inline void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-constexpr int kSpaiThreads = 256;
-constexpr int kAchLd = SPAI_CHUNK + 1;  // staged column stride (odd: conflict-free LDS reads)
-constexpr int kSpaiPre = (SPAI_CHUNK * SPAI_MAXJ + kSpaiThreads - 1) / kSpaiThreads;  // staged entries per thread
-static_assert(SPAI_MAXJ < 128, "a lane holds at most two rows of a column's system");
-
-// v of lane src (uniform) in every lane
-__device__ inline double bcast(double v, int src) {
-  const long long u = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)(u & 0xffffffffLL), src);
-  const int hi = __builtin_amdgcn_readlane((int)(u >> 32), src);
-  return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
-}
-__device__ inline double2 bcast2(double2 v, int src) { return make_double2(bcast(v.x, src), bcast(v.y, src)); }
-
-__global__ __launch_bounds__(kSpaiThreads, 5) void k_spai_build(int n, int per, ZRef z, int mJ,
-                                                             const int* __restrict__ jptr,
-                                                             const int* __restrict__ jidx,
-                                                             const int* __restrict__ iptr,
-                                                             const int* __restrict__ iidx,
-                                                             double2* __restrict__ vals, int* __restrict__ status) {
+template <int NT>
+__global__ __launch_bounds__(NT, 3) void k_spai_build(int n, int per, ZRef z, const int* __restrict__ jptr,
+                                                      const int* __restrict__ jidx, const int* __restrict__ iptr,
+                                                      const int* __restrict__ iidx, double2* __restrict__ vals,
+                                                      int* __restrict__ status) {
+  constexpr int NB = SpaiShape<NT>::NB;
+  constexpr int kPre = (4 * NB * SPAI_CHUNK + NT - 1) / NT;  // staged entries per thread
+  static_assert(NB * (NB + 1) / 2 <= NT && NT % SPAI_CHUNK == 0, "one block per thread");
   // XCD-aware order: workgroup w runs on XCD w % 8, which takes the columns
   // [x per, (x + 1) per) in order, so the columns in flight on one XCD are
   // neighbours whose rows of Z overlap and are read through the same L2.
@@ -78,178 +86,195 @@ __global__ __launch_bounds__(kSpaiThreads, 5) void k_spai_build(int n, int per, 
   if (j >= n) return;
   const int j0 = jptr[j], nJ = jptr[j + 1] - j0;
   const int i0 = iptr[j], nI = iptr[j + 1] - i0;
-  extern __shared__ __align__(16) char smem[];
-  double2* G = reinterpret_cast<double2*>(smem);
-  double2* Ach = G + mJ * (mJ + 1) / 2;
-  double2* rhs = Ach + kAchLd * mJ;
-  int* cols = reinterpret_cast<int*>(rhs + mJ);
+  // staged rows, column c of row r at [r][c % 4][c / 4] (a wave's block rows are
+  // consecutive); the factorization's panel at [v][u][A] in the same place
+  __shared__ double2 st[2][SPAI_CHUNK][4][NB];
+  __shared__ double2 dl[4][4];
+  __shared__ double dil[4];
+  __shared__ double2 ys[4 * NB];
+  double2(*panel)[4][NB] = st[0];
   const int tid = threadIdx.x;
-  for (int a = tid; a < nJ; a += kSpaiThreads) {
-    const int c = jidx[j0 + a];
-    cols[a] = c;
-    // rhs = A^H e_j = conj(Z[j, J]) (row j of Z restricted to the pattern)
-    const double2 v = zat(z, j, c);
-    rhs[a] = make_double2(v.x, -v.y);
+  const int nb = nJ / 4 + 1;  // block rows of the nJ + 1 extended ones
+  int A = -1, B = -1;
+  if (tid < nb * (nb + 1) / 2) {
+    int e = tid;
+    for (B = 0; e >= nb - B; ++B) e -= nb - B;
+    A = B + e;
   }
-  for (int e = tid; e < nJ * (nJ + 1) / 2; e += kSpaiThreads) G[e] = make_double2(0.0, 0.0);
-  // G = A^H A accumulated over chunks of SPAI_CHUNK rows staged column by
-  // column (Ach[a * kAchLd + r]; rows past the end of A are zero).  Thread t
-  // owns the 2 x 2 blocks 255 - t, 511 - t, ... of the block lower triangle
-  // (block rows A >= B; a second block falls to the last wave, not to wave 0,
-  // which goes on to the factorization) and adds each chunk's sums to them.
-  const int nb = (nJ + 1) / 2, nblk = nb * (nb + 1) / 2;
-  // each thread stages the same (row, column) places of every chunk; the
-  // next chunk's entries are loaded into registers before this chunk's sums
-  // are formed, so their latency is hidden behind the arithmetic
-  int pr[kSpaiPre], pa[kSpaiPre];
-  double2 pre[kSpaiPre];
+  // staging: this thread's row of every chunk, its columns
+  const int sr = tid % SPAI_CHUNK;
+  int sc[kPre], col[kPre];
 #pragma unroll
-  for (int q = 0; q < kSpaiPre; ++q) {
-    const int e = tid + q * kSpaiThreads;
-    pr[q] = e < SPAI_CHUNK * nJ ? e / nJ : SPAI_CHUNK;
-    pa[q] = e < SPAI_CHUNK * nJ ? e - pr[q] * nJ : 0;
+  for (int q = 0; q < kPre; ++q) {
+    sc[q] = tid / SPAI_CHUNK + q * (NT / SPAI_CHUNK);
+    col[q] = jidx[j0 + min(sc[q], nJ - 1)];
   }
-  auto fetch = [&](int r0) {
+  double2 pre[kPre];
+  auto row_of = [&](int r0) { return iidx[i0 + min(r0 + sr, nI - 1)]; };
+  auto fetch = [&](int r0, int row) {
 #pragma unroll
-    for (int q = 0; q < kSpaiPre; ++q)
-      pre[q] = pr[q] < SPAI_CHUNK && r0 + pr[q] < nI ? zat(z, iidx[i0 + r0 + pr[q]], cols[pa[q]])
-                                                     : make_double2(0.0, 0.0);
+    for (int q = 0; q < kPre; ++q) {
+      pre[q] = zat(z, row, col[q]);
+      if (r0 + sr >= nI || sc[q] >= nJ) pre[q] = make_double2(0.0, 0.0);
+    }
   };
-  __syncthreads();  // cols
-  fetch(0);
-  for (int r0 = 0; r0 < nI; r0 += SPAI_CHUNK) {
-    __syncthreads();
+  auto stage = [&](int buf) {
 #pragma unroll
-    for (int q = 0; q < kSpaiPre; ++q)
-      if (pr[q] < SPAI_CHUNK) Ach[pa[q] * kAchLd + pr[q]] = pre[q];
-    __syncthreads();
-    if (r0 + SPAI_CHUNK < nI) fetch(r0 + SPAI_CHUNK);
-    for (int e = kSpaiThreads - 1 - tid; e < nblk; e += kSpaiThreads) {
-      int A, B;
-      untri(e, A, B);
-      // columns past nJ - 1 (odd nJ) read column nJ - 1 and are not stored
-      const double2* ca0 = Ach + 2 * A * kAchLd;
-      const double2* ca1 = Ach + min(2 * A + 1, nJ - 1) * kAchLd;
-      const double2* cb0 = Ach + 2 * B * kAchLd;
-      const double2* cb1 = Ach + min(2 * B + 1, nJ - 1) * kAchLd;
-      double sr[4] = {0, 0, 0, 0}, si[4] = {0, 0, 0, 0};
-      auto mac = [&](int u, double2 p, double2 q) {
-        // conj(p) q
-        sr[u] = fma(p.x, q.x, sr[u]);
-        sr[u] = fma(p.y, q.y, sr[u]);
-        si[u] = fma(p.x, q.y, si[u]);
-        si[u] = fma(-p.y, q.x, si[u]);
-      };
-#pragma unroll 4
-      for (int ii = 0; ii < SPAI_CHUNK; ++ii) {
-        const double2 p0 = ca0[ii], p1 = ca1[ii], q0 = cb0[ii], q1 = cb1[ii];
-        mac(0, p0, q0);
-        mac(1, p0, q1);
-        mac(2, p1, q0);
-        mac(3, p1, q1);
+    for (int q = 0; q < kPre; ++q)
+      if (sc[q] < 4 * nb) st[buf][sr][sc[q] & 3][sc[q] >> 2] = pre[q];
+  };
+  double2 acc[4][4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[u][v] = make_double2(0.0, 0.0);
+  fetch(0, row_of(0));
+  int row = row_of(SPAI_CHUNK);
+  stage(0);
+  __syncthreads();
+  for (int r0 = 0, buf = 0; r0 < nI; r0 += SPAI_CHUNK, buf ^= 1) {
+    const bool more = r0 + SPAI_CHUNK < nI;
+    if (more) {
+      fetch(r0 + SPAI_CHUNK, row);
+      row = row_of(r0 + 2 * SPAI_CHUNK);
+    }
+    if (A >= 0) {
+#pragma unroll 2
+      for (int r = 0; r < SPAI_CHUNK; ++r) {
+        double2 p[4], q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          p[u] = st[buf][r][u][A];
+          q[u] = st[buf][r][u][B];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) cacc_pq(acc[u][v], p[u], q[v]);
       }
-      const int a0 = 2 * A, b0 = 2 * B;
-      auto add = [&](int a, int b, int u) {
-        G[tri(a, b)].x += sr[u];
-        G[tri(a, b)].y += si[u];
-      };
-      add(a0, b0, 0);
-      if (b0 + 1 <= a0) add(a0, b0 + 1, 1);
-      if (a0 + 1 < nJ) {
-        add(a0 + 1, b0, 2);
-        if (b0 + 1 < nJ) add(a0 + 1, b0 + 1, 3);
+    }
+    if (more) stage(buf ^ 1);
+    __syncthreads();
+  }
+  // the extended row (rhs^H = Z[j, J]) and the identity past it
+  const int eu = nJ & 3;  // its place in block row nb - 1
+  if (A == nb - 1) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int b = 4 * B + v;
+        if (u == eu && b < nJ) acc[u][v] = zat(z, j, jidx[j0 + b]);
+        if (4 * A + u >= nJ && b == 4 * A + u) acc[u][v] = make_double2(1.0, 0.0);
+      }
+  }
+  bool bad = false;
+  for (int K = 0; K < nb; ++K) {
+    if (A == K && B == K) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        double d = acc[v][v].x;
+#pragma unroll
+        for (int w = 0; w < v; ++w) d = fma(-acc[v][w].x, acc[v][w].x, fma(-acc[v][w].y, acc[v][w].y, d));
+        if (4 * K + v >= nJ) d = 1.0;
+        if (!(d > 0.0)) {
+          bad = true;
+          d = 1e-300;
+        }
+        const double il = rsqrt(d);
+        dil[v] = il;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (u <= v) continue;
+          double2 x = acc[u][v];
+#pragma unroll
+          for (int w = 0; w < v; ++w) csub_pq(x, acc[u][w], acc[v][w]);
+          acc[u][v] = make_double2(x.x * il, x.y * il);
+          dl[u][v] = acc[u][v];
+        }
+        acc[v][v] = make_double2(il, 0.0);  // 1 / L[v][v]
+      }
+    }
+    __syncthreads();
+    if (B == K && A > K) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const double il = dil[v];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          double2 x = acc[u][v];
+#pragma unroll
+          for (int w = 0; w < v; ++w) csub_pq(x, acc[u][w], dl[v][w]);
+          acc[u][v] = make_double2(x.x * il, x.y * il);
+          panel[v][u][A] = acc[u][v];
+        }
+      }
+    }
+    __syncthreads();
+    if (B > K) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        double2 p[4], q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          p[u] = panel[v][u][A];
+          q[u] = panel[v][u][B];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int w = 0; w < 4; ++w) csub_pq(acc[u][w], p[u], q[w]);
+      }
+    }
+  }
+  // y = conj of the extended row; entries past nJ - 1 are zero
+  if (A == nb - 1) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (u == eu)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          ys[4 * B + v] = 4 * B + v < nJ ? make_double2(acc[u][v].x, -acc[u][v].y) : make_double2(0.0, 0.0);
+  }
+  for (int K = nb - 1; K >= 0; --K) {
+    __syncthreads();
+    if (A == K && B == K) {
+      // L(K, K)^H m = y
+      double2 m[4];
+#pragma unroll
+      for (int v = 3; v >= 0; --v) {
+        double2 x = ys[4 * K + v];
+#pragma unroll
+        for (int u = 3; u > v; --u) {
+          // x -= conj(L[u][v]) m[u]
+          x.x -= acc[u][v].x * m[u].x + acc[u][v].y * m[u].y;
+          x.y -= acc[u][v].x * m[u].y - acc[u][v].y * m[u].x;
+        }
+        const double il = acc[v][v].x;
+        m[v] = make_double2(x.x * il, x.y * il);
+        ys[4 * K + v] = m[v];
+      }
+    }
+    __syncthreads();
+    if (A == K && B < K) {
+      double2 m[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) m[u] = ys[4 * K + u];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        double2 x = ys[4 * B + v];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          x.x -= acc[u][v].x * m[u].x + acc[u][v].y * m[u].y;
+          x.y -= acc[u][v].x * m[u].y - acc[u][v].y * m[u].x;
+        }
+        ys[4 * B + v] = x;
       }
     }
   }
   __syncthreads();
-  if (tid >= 64) return;
-  const int lane = tid;
-  bool bad = false;
-  // the right-hand side in registers: lane l holds rows l and l + 64
-  // (nJ <= SPAI_MAXJ < 128); its LDS place then keeps 1 / L[k][k]
-  double2 b[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int i = lane + 64 * h;
-    b[h] = i < nJ ? rhs[i] : make_double2(0.0, 0.0);
-  }
-  double* dinv = reinterpret_cast<double*>(rhs);
-  wave_sync();
-  // Cholesky G = L L^H in place (lower triangle), left-looking: column k of
-  // L from the dot products of rows i >= k with row k over the columns
-  // p < k (independent LDS reads, no round trip per update).  Lane l owns
-  // rows l and l + 64.
-  for (int k = 0; k < nJ; ++k) {
-    double2 s[2];
-    double dk = 0.0;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int i = lane + 64 * h;
-      s[h] = make_double2(0.0, 0.0);
-      if (i < k || i >= nJ) continue;
-      double2 v = G[tri(i, k)];
-      for (int p = 0; p < k; ++p) {
-        const double2 a = G[tri(i, p)], b = G[tri(k, p)];
-        // v -= L[i][p] conj(L[k][p])
-        v.x = fma(-a.x, b.x, v.x);
-        v.x = fma(-a.y, b.y, v.x);
-        v.y = fma(-a.y, b.x, v.y);
-        v.y = fma(a.x, b.y, v.y);
-      }
-      s[h] = v;
-      if (i == k) dk = v.x;
-    }
-    double d = bcast(dk, k & 63);
-    if (!(d > 0.0)) {
-      bad = true;
-      d = 1e-300;
-    }
-    const double lkk = sqrt(d), il = 1.0 / lkk;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int i = lane + 64 * h;
-      if (i < k || i >= nJ) continue;
-      G[tri(i, k)] = i == k ? make_double2(lkk, 0.0) : make_double2(s[h].x * il, s[h].y * il);
-    }
-    if (lane == 0) dinv[k] = il;
-    wave_sync();
-  }
-  // forward: L y = rhs (y_k reaches every lane through a lane read)
-  for (int k = 0; k < nJ; ++k) {
-    const double il = dinv[k];
-    const double2 bk = bcast2(k < 64 ? b[0] : b[1], k & 63);
-    const double2 yk = make_double2(bk.x * il, bk.y * il);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int i = lane + 64 * h;
-      if (i == k) b[h] = yk;
-      if (i <= k || i >= nJ) continue;
-      const double2 l = G[tri(i, k)];
-      b[h].x -= l.x * yk.x - l.y * yk.y;
-      b[h].y -= l.x * yk.y + l.y * yk.x;
-    }
-  }
-  // backward: L^H m = y
-  for (int k = nJ - 1; k >= 0; --k) {
-    const double il = dinv[k];
-    const double2 bk = bcast2(k < 64 ? b[0] : b[1], k & 63);
-    const double2 mk = make_double2(bk.x * il, bk.y * il);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int i = lane + 64 * h;
-      if (i == k) b[h] = mk;
-      if (i >= k) continue;
-      const double2 l = G[tri(k, i)];  // (L^H)[i][k] = conj(L[k][i])
-      b[h].x -= l.x * mk.x + l.y * mk.y;
-      b[h].y -= l.x * mk.y - l.y * mk.x;
-    }
-  }
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int i = lane + 64 * h;
-    if (i < nJ) vals[j0 + i] = b[h];
-  }
-  if (lane == 0 && bad) status[0] = j + 1;
+  for (int a = tid; a < nJ; a += NT) vals[j0 + a] = ys[a];
+  if (bad) status[0] = j + 1;
 }
 
 // y = M x with M in CSR form (row n: columns colidx[rowptr[n]..], values csrval).
@@ -355,13 +380,16 @@ int spai_max_cols() { return SPAI_MAXJ; }
 void spai_build(i64 n, const ZRef& z, int maxJ, const int* jptr, const int* jidx, const int* iptr, const int* iidx,
                 double* vals, int* status, hipStream_t s) {
   DM_REQUIRE(maxJ >= 1 && maxJ <= SPAI_MAXJ, DM_ERR_ARGUMENT, "near-field preconditioner: support width out of range");
-  const size_t smem = sizeof(double2) * ((size_t)maxJ * (maxJ + 1) / 2 + (size_t)kAchLd * maxJ + maxJ) +
-                      sizeof(int) * maxJ;
-  HIP_OK(hipFuncSetAttribute((const void*)k_spai_build, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
   DM_REQUIRE(n < (1LL << 31) - 8, DM_ERR_ARGUMENT, "near-field preconditioner: too many bases for one launch");
-  const int per = (int)((n + 7) / 8);
-  k_spai_build<<<8u * (unsigned)per, kSpaiThreads, smem, s>>>((int)n, per, z, maxJ, jptr, jidx, iptr, iidx,
-                                                              reinterpret_cast<double2*>(vals), status);
+  const int per = (int)((n + 7) / 8), nb = maxJ / 4 + 1;
+  double2* v = reinterpret_cast<double2*>(vals);
+  // the fewest threads that give every block of the widest support one
+  if (nb <= SpaiShape<64>::NB)
+    k_spai_build<64><<<8u * (unsigned)per, 64, 0, s>>>((int)n, per, z, jptr, jidx, iptr, iidx, v, status);
+  else if (nb <= SpaiShape<128>::NB)
+    k_spai_build<128><<<8u * (unsigned)per, 128, 0, s>>>((int)n, per, z, jptr, jidx, iptr, iidx, v, status);
+  else
+    k_spai_build<256><<<8u * (unsigned)per, 256, 0, s>>>((int)n, per, z, jptr, jidx, iptr, iidx, v, status);
   HIP_OK(hipGetLastError());
 }
 
