@@ -9,11 +9,12 @@
 // One wave per column: the internal order's blocks of 64 bases are compact
 // patches, so their bounding boxes select the candidates (every lane tests a
 // block, the chosen blocks' 64 bases are tested together, and the candidates
-// stay in index order); each candidate's rank by (distance, index) is counted
-// against the others in LDS, which needs no sort.  Bound by the rank counting
-// (~c^2 comparisons for c candidates, c ~ 200-400 on uniform meshes).  A plate
-// of 4720 bases with a cutoff of one wavelength: the host form (hash grid, sort
-// per column, one thread) takes 140 ms, this 1.2 ms (1.1 ms of it k_pat_cols).
+// stay in index order); the nearest maxJ (and 512) are the candidates up to a
+// distance found bit by bit (first_k), which needs no sort.  Bound by the waves'
+// serial steps.  A plate of 4720 bases with a cutoff of one wavelength: the host
+// form (hash grid, sort per column, one thread) takes 140 ms, this 0.25 ms
+// (0.14 of it k_pat_cols; counting every candidate's rank against the others, c^2
+// comparisons, it was 1.1).
 #include <hip/hip_runtime.h>
 
 #include "dm_common.h"
@@ -73,6 +74,39 @@ __device__ inline void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Which of a wave's cnt distances (lane, lane + 64, ... in v; infinite past cnt)
+// are among the first k by (distance, position): bit q of sel.  The k-th smallest
+// distance is built bit by bit from the top (distances are not negative, so they
+// order as integers), each bit by a count of the smaller ones; among equal ones
+// the first positions are taken.
+__device__ inline void first_k(const double (&v)[kCap / 64], int cnt, int k, unsigned long long below, unsigned& sel) {
+  sel = ~0u;
+  if (cnt <= k) return;
+  unsigned long long t = 0;
+  int less = 0;
+  for (int bit = 62; bit >= 0; --bit) {
+    const unsigned long long trial = t | 1ull << bit;
+    int c = 0;
+#pragma unroll
+    for (int q = 0; q < kCap / 64; ++q)
+      if (q * 64 < cnt) c += __popcll(__ballot((unsigned long long)__double_as_longlong(v[q]) < trial));
+    if (c < k) {
+      t = trial;
+      less = c;
+    }
+  }
+  sel = 0;
+  int eq = k - less;  // equal ones still to be taken
+#pragma unroll
+  for (int q = 0; q < kCap / 64; ++q) {
+    if (q * 64 >= cnt) continue;
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v[q]);
+    const unsigned long long same = __ballot(b == t);
+    if (b < t || (b == t && (int)__popcll(same & below) < eq)) sel |= 1u << q;
+    eq -= (int)__popcll(same);
+  }
+}
+
 // Lists of column j at tJ + j maxJ and tI + j kMaxI, their lengths and the
 // radius.  The search radius R starts at `cell` and grows by `cell` until both
 // lists are certain to be complete; a patch with more than kCap bases within R
@@ -119,46 +153,25 @@ __global__ __launch_bounds__(64 * kWaves) void k_pat_cols(i64 n, i64 nblk, const
       R = 0.5 * (lo + hi);
       continue;
     }
-    // rank of candidates lane, lane + 64, ... (equal distances: list order is
-    // index order)
-    int rank[kCap / 64];
+    // candidates lane, lane + 64, ... (list order is index order)
+    double dv[kCap / 64];
 #pragma unroll
-    for (int q0 = 0; q0 < kCap / 64; q0 += 4) {
-      if (q0 * 64 >= cnt) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) rank[q0 + q] = kCap;
-        continue;
-      }
-      double de[4];
-      int r[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int e = lane + 64 * (q0 + q);
-        de[q] = d[max(min(e, cnt - 1), 0)];
-        r[q] = 0;
-      }
-#pragma unroll 4
-      for (int i = 0; i < cnt; ++i) {
-        const double di = d[i];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) r[q] += (di < de[q] || (di == de[q] && i < lane + 64 * (q0 + q))) ? 1 : 0;
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q) rank[q0 + q] = lane + 64 * (q0 + q) < cnt ? r[q] : kCap;
-    }
+    for (int q = 0; q < kCap / 64; ++q)
+      dv[q] = q * 64 < cnt && lane + 64 * q < cnt ? d[lane + 64 * q] : INFINITY;
+    unsigned selJ, selI;  // bit q: among the first maxJ (kMaxI) by (distance, index)
+    first_k(dv, cnt, maxJ, below, selJ);
+    first_k(dv, cnt, kMaxI, below, selI);
     int nJ = 0;
     bool self = false, next = false;
     double rJ = 0.0;
 #pragma unroll
     for (int q = 0; q < kCap / 64; ++q) {
       if (q * 64 >= cnt) continue;
-      const int e = max(min(lane + 64 * q, cnt - 1), 0);
-      const double dd = d[e];
-      const bool in = rank[q] < maxJ && dd <= cutJ;
+      const bool near = dv[q] <= cutJ && lane + 64 * q < cnt, in = near && (selJ >> q & 1);
       nJ += __popcll(__ballot(in));
-      self = self || (in && m[e] == (int)j);
-      next = next || (rank[q] == maxJ && dd <= cutJ);
-      if (in) rJ = fmax(rJ, dd);
+      self = self || (in && m[lane + 64 * q] == (int)j);
+      next = next || (near && !in);  // past the first maxJ
+      if (in) rJ = fmax(rJ, dv[q]);
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) rJ = fmax(rJ, __shfl_xor(rJ, o, 64));
@@ -180,10 +193,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_pat_cols(i64 n, i64 nblk, const
 #pragma unroll
     for (int q = 0; q < kCap / 64; ++q) {
       if (q * 64 >= cnt) continue;
-      const int e = max(min(lane + 64 * q, cnt - 1), 0);
-      const double dd = d[e];
-      const int mm = m[e];
-      const bool inJ = rank[q] < maxJ && dd <= cutJ, inI = rank[q] < kMaxI && dd <= rI;
+      const bool ok = lane + 64 * q < cnt;
+      const int mm = m[ok ? lane + 64 * q : 0];
+      const bool inJ = ok && (selJ >> q & 1) && dv[q] <= cutJ, inI = ok && (selI >> q & 1) && dv[q] <= rI;
       const unsigned long long bJ = __ballot(inJ), bI = __ballot(inI);
       if (inJ) tJ[j * maxJ + at + __popcll(bJ & below)] = mm;
       if (inI) tI[j * kMaxI + nI + __popcll(bI & below)] = mm;
