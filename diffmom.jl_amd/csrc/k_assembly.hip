@@ -712,11 +712,18 @@ __device__ inline void tile_body(const AsmArgs& a, int cap, AccT* __restrict__ z
     pair_loop(std::true_type{});
   else
     pair_loop(std::false_type{});
+  const i64 r0 = (i64)bi * TB, c0 = (i64)bj * TB;
+  // MODE 1: entry tid of x times its length, rows' then columns' (loaded while
+  // the last pairs of other waves are formed)
+  double2 xl = make_double2(0.0, 0.0);
+  if constexpr (MODE == 1) {
+    const i64 g = tid < TB ? r0 + tid : c0 + tid - TB;
+    if (tid < 2 * TB && g < a.n) xl = make_double2(a.len[g] * x[2 * g], a.len[g] * x[2 * g + 1]);
+  }
   __syncthreads();
 
   // Z_mn = -i k eta0 len_m len_n * tile ; P = -i k eta0 = (k_im eta0, -k_re eta0)
   const double Pr = a.k_im * a.eta0, Pi = -a.k_re * a.eta0;
-  const i64 r0 = (i64)bi * TB, c0 = (i64)bj * TB;
   float* const dual = sizeof(AccT) == 8 ? a.z32_dual : nullptr;
   const bool diag = bi == bj;
   if constexpr (MODE == 0) {
@@ -779,28 +786,39 @@ __device__ inline void tile_body(const AsmArgs& a, int cap, AccT* __restrict__ z
     }
     if (bad) atomicOr(a.flag, 1);
   } else {
-    // y[rows] += Z_tile x[cols]; y[cols] += Z_tile^T x[rows] (off-diagonal tiles)
-    for (int k = tid; k < 2 * TB; k += NTHR) {
-      bool rows = k < TB;
-      int r = rows ? k : k - TB;
-      if (!rows && diag) continue;
-      i64 go = rows ? r0 + r : c0 + r;
-      if (go >= a.n) continue;
+    // y[rows] += Z_tile x[cols]; y[cols] += Z_tile^T x[rows] (off-diagonal
+    // tiles): eight lanes per entry of y, TB / 8 terms each (stride 1 within a
+    // lane: the 64 lanes' reads fall on all banks); x in the place of the
+    // sides' images.  7680 unknowns: 777 us; one thread per entry, reading x
+    // and the lengths term by term: 1048.
+    double2* xs = reinterpret_cast<double2*>(lds_align16(smem, smem + sizeof(AccT) * 2 * TB * ldt));
+    if (tid < 2 * TB) xs[tid] = xl;
+    __syncthreads();
+    const int l = tid & 7, per = TB / 8;
+    for (int k = tid >> 3; k < (diag ? TB : 2 * TB); k += NTHR / 8) {
+      const bool rows = k < TB;
+      const int o = rows ? k : k - TB;
+      const i64 go = rows ? r0 + o : c0 + o;
       double accr = 0, acci = 0;
-      for (int c = 0; c < TB; ++c) {
-        i64 gi2 = rows ? c0 + c : r0 + c;
-        if (gi2 >= a.n) break;
-        int rr = rows ? r : c, cc = rows ? c : r;
+      for (int t = 0; t < per; ++t) {
+        const int c = per * l + t;
+        int rr = rows ? o : c, cc = rows ? c : o;
         if (diag && rr > cc) { int t2 = rr; rr = cc; cc = t2; }
-        double tr = (double)zt[rr * ldt + cc], ti = (double)zt[TB * ldt + rr * ldt + cc];
-        double l2 = a.len[go] * a.len[gi2];
-        double vr = (Pr * tr - Pi * ti) * l2, vi = (Pr * ti + Pi * tr) * l2;
-        double xr = x[2 * gi2], xi = x[2 * gi2 + 1];
-        accr += vr * xr - vi * xi;
-        acci += vr * xi + vi * xr;
+        const double tr = (double)zt[rr * ldt + cc], ti = (double)zt[TB * ldt + rr * ldt + cc];
+        const double2 xv = xs[rows ? TB + c : c];
+        accr += tr * xv.x - ti * xv.y;
+        acci += tr * xv.y + ti * xv.x;
       }
-      atomicAdd(y + 2 * go, accr);
-      atomicAdd(y + 2 * go + 1, acci);
+#pragma unroll
+      for (int q = 4; q > 0; q >>= 1) {
+        accr += __shfl_xor(accr, q, 8);
+        acci += __shfl_xor(acci, q, 8);
+      }
+      if (l == 0 && go < a.n) {
+        const double ln = a.len[go];
+        atomicAdd(y + 2 * go, (Pr * accr - Pi * acci) * ln);
+        atomicAdd(y + 2 * go + 1, (Pr * acci + Pi * accr) * ln);
+      }
     }
   }
 }
@@ -815,23 +833,21 @@ __global__ __launch_bounds__(NTHR) void k_tile(AsmArgs a, int cap, AccT* __restr
   tile_body<T, AccT, NQ, NTHR, MODE>(a, cap, zout, x, y, bi, bj);
 }
 
-// Persistent assembly of several meshes in one launch: every workgroup takes
-// the next tile from a global counter over the concatenated tile lists
-// (meshes in the caller's order, largest first for balance) until all
-// cum[nmesh] tiles are done.
+// Persistent assembly of several meshes in one launch: workgroup g starts with
+// tile g and takes the next ones from a global counter (which starts at the
+// grid's size) over the concatenated tile lists (meshes in the caller's order,
+// largest first for balance) until all cum[nmesh] tiles are done.
 template <typename T, typename AccT, int NQ, int NTHR, int MODE>
 __global__ __launch_bounds__(NTHR) void k_tile_multi(const AsmArgs* __restrict__ args, AccT* const* __restrict__ zouts,
                                                       const i64* __restrict__ cum, int nmesh, int cap,
                                                       int* __restrict__ counter) {
   __shared__ int item;
   const i64 total = cum[nmesh];
-  for (;;) {
-    if (threadIdx.x == 0) item = atomicAdd(counter, 1);
-    __syncthreads();
-    const i64 w = item;
-    __syncthreads();
-    if (w >= total) break;
-    int m = 0;
+  int m = 0;  // a workgroup's tiles come in ascending order, so its mesh only moves on
+  for (i64 w = blockIdx.x; w < total;) {
+    // the next tile's number is on its way while this tile is formed
+    int next = 0;
+    if (threadIdx.x == 0) next = atomicAdd(counter, 1);
     while (m + 1 < nmesh && cum[m + 1] <= w) ++m;
     const i64 l = w - cum[m];
     i64 b = (i64)((sqrt(8.0 * (double)l + 1.0) - 1.0) * 0.5);
@@ -839,6 +855,9 @@ __global__ __launch_bounds__(NTHR) void k_tile_multi(const AsmArgs* __restrict__
     while ((b + 1) * (b + 2) / 2 <= l) ++b;
     const AsmArgs& a = args[m];  // read in place: a private copy would live in scratch
     tile_body<T, AccT, NQ, NTHR, MODE>(a, cap, zouts[m], nullptr, nullptr, (int)(l - b * (b + 1) / 2), (int)b);
+    if (threadIdx.x == 0) item = next;
+    __syncthreads();
+    w = item;
     __syncthreads();
   }
 }
@@ -914,7 +933,9 @@ void launch_tile(const AsmArgs& a, int cap, AccT* z, const double* x, double* y,
 
 template <typename T, typename AccT, int MODE>
 void launch_tile_multi(const std::vector<AsmArgs>& args, const std::vector<AccT*>& zouts, int cap, hipStream_t s) {
-  constexpr int NTHR = 512;
+  // as in launch_tile; 64 plates, 9262 tiles: 1.37 ms with 512 threads, 1.18 with 1024
+  // (1.11 with the next tile's number fetched ahead)
+  constexpr int NTHR = sizeof(T) == 8 ? 1024 : 512;
   const int nmesh = (int)args.size();
   DM_REQUIRE(nmesh >= 1, DM_ERR_ARGUMENT, "no meshes");
   const int nq = args[0].nq;
@@ -932,7 +953,6 @@ void launch_tile_multi(const std::vector<AsmArgs>& args, const std::vector<AccT*
   dz.upload(zouts, s);
   dcum.upload(cum, s);
   counter.alloc(1);
-  k_fill_int<<<1, 1, 0, s>>>(counter.p, 0);
   int dev = 0, ncu = 0;
   HIP_OK(hipGetDevice(&dev));
   HIP_OK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
@@ -944,6 +964,7 @@ void launch_tile_multi(const std::vector<AsmArgs>& args, const std::vector<AccT*
     int per_cu = 0;                                                                                        \
     HIP_OK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, NTHR, smem));                        \
     i64 grid = std::min<i64>(cum[nmesh], (i64)std::max(per_cu, 1) * ncu);                                  \
+    k_fill_int<<<1, 1, 0, s>>>(counter.p, (int)grid);                                                      \
     kfn<<<dim3((unsigned)grid), dim3(NTHR), smem, s>>>(dargs.p, dz.p, dcum.p, nmesh, cap, counter.p);      \
     break;                                                                                                 \
   }

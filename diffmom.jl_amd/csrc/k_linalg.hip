@@ -174,9 +174,16 @@ __global__ __launch_bounds__(256) void k_gemv_small(i64 n, i64 ld, const T* __re
 #pragma unroll
   for (int u = 0; u < 8; ++u) a[u] = zc[min((i64)lane + 64 * u, n - 1)];
   const int ic = idx[min(c, n - 1)];
-  for (i64 m = threadIdx.x; m < n; m += 256) {
-    const double2 v = x[idx[m]];
-    xs[m] = make_double2(v.x, sg * v.y);
+  for (i64 m0 = threadIdx.x; m0 < n; m0 += 1024) {
+    int p[4];
+    double2 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) p[u] = idx[min(m0 + 256 * u, n - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = x[p[u]];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (m0 + 256 * u < n) xs[m0 + 256 * u] = make_double2(v[u].x, sg * v[u].y);
   }
   __syncthreads();
   double ar = 0, ai = 0;
