@@ -32,7 +32,7 @@ struct BatchKrylov {
     if (flexible) grow(Zs, blk * m);
     grow(W, blk);
     grow(T, blk);
-    grow(part, 2 * dmb::part_count(n, R, kcap));
+    grow(part, (size_t)2 * R * kcap * dmb::dot_chunks(n));
     grow(h, (size_t)2 * 2 * R * kcap);
     grow(nr, R);
     grow(y, (size_t)2 * R * kcap);
@@ -157,7 +157,8 @@ void gmres_batch(dm_ctx* ctx, i64 n, int R, DevOp& A, DevPrec* M, const double* 
       {
         ProfScope p(ctx, "arnoldi", s);
         dmb::dots(n, R, k, K.kcap, K.V.p, K.W.p, K.act.p, K.part.p, h1, s);
-        dmb::update_dots(n, R, k, K.kcap, K.V.p, h1, K.act.p, K.W.p, K.part.p, h2, s);
+        dmb::update(n, R, k, K.kcap, K.V.p, h1, K.act.p, K.W.p, s);
+        dmb::dots(n, R, k, K.kcap, K.V.p, K.W.p, K.act.p, K.part.p, h2, s);
         dmb::update(n, R, k, K.kcap, K.V.p, h2, K.act.p, K.W.p, s);
         dmb::norm2(n, R, K.W.p, K.act.p, K.nr.p, s);
         dmb::givens(R, j, mcap, K.kcap, h1, h2, K.nr.p, Hd.p, csd.p, snd.p, gd.p, K.sc.p, K.act.p, epsd.p, jcnt.p,

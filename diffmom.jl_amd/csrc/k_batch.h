@@ -6,16 +6,13 @@
 
 namespace dmb {
 int max_basis();               // largest k supported by dots / update / combine
-size_t part_count(i64 n, int R, int kcap);  // complex values of part (dots, update_dots)
+int dot_chunks(i64 n);         // row chunks of dots: part holds R * kcap * dot_chunks(n) complex
 // h[r, i] = V_i[r]^H W[r] for i < k
 void dots(i64 n, int R, int k, int kcap, const double* V, const double* W, const int* act, double* part, double* h,
           hipStream_t s);
 // W[r] -= sum_{i<k} V_i[r] h[r, i]
 void update(i64 n, int R, int k, int kcap, const double* V, const double* h, const int* act, double* W,
             hipStream_t s);
-// update with h1, then dots of the updated W into h2
-void update_dots(i64 n, int R, int k, int kcap, const double* V, const double* h1, const int* act, double* W,
-                 double* part, double* h2, hipStream_t s);
 // X[r] += sum_{i<cnt[r]} V_i[r] y[r, i]
 void combine(i64 n, int R, int kcap, const double* V, const double* y, const int* cnt, double* X, hipStream_t s);
 // out[r] = ||W[r]||^2 (act may be null: every column)

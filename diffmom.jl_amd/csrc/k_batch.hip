@@ -155,103 +155,6 @@ __global__ __launch_bounds__(BT) void k_bupdate(i64 n, int R, int k, int kcap, c
   }
 }
 
-// Update and dots in one pass over the basis: W[r] -= sum_{i<k} V_i[r] h[r, i],
-// then part[(r * nch + c) * k + i] = sum over the rows of chunk c of
-// conj(V_i[r]) . W[r] with the updated W.  HBM-bound: the workgroup keeps its
-// BFROWS rows of all k vectors in LDS between the two (1152 bytes a vector), so
-// the basis is read once instead of twice.  Vectors go to the waves in
-// turn for the update, 8 loads in flight each, and to groups of 8 lanes for
-// the dots (the pitch of 72 keeps two groups on different halves of the banks).
-constexpr int BFROWS = 64, BFPITCH = 72;
-template <int NT>
-__global__ __launch_bounds__(NT) void k_bupdots(i64 n, int R, int k, int kcap, const double2* __restrict__ V,
-                                                const double2* __restrict__ h, const int* __restrict__ act,
-                                                double2* __restrict__ W, double2* __restrict__ part, int nch) {
-  constexpr int T = BFROWS, P = BFPITCH, S = NT / T;
-  const int c = blockIdx.x, r = blockIdx.y;
-  if (!act[r]) return;
-  extern __shared__ double2 vt[];  // k x BFPITCH
-  __shared__ double2 ws[S][T];
-  const int lane = threadIdx.x % T, sub = threadIdx.x / T;
-  const i64 m = c * (i64)T + lane;
-  const i64 off = (i64)r * n + min(m, n - 1), NR = n * R;
-  const double2* hr = h + (i64)r * kcap;
-  const double2 o = W[off];
-  double ar = 0, ai = 0;
-  for (int i0 = sub; i0 < k; i0 += 8 * S) {
-    double2 a[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) a[u] = V[(i64)min(i0 + S * u, k - 1) * NR + off];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int i = i0 + S * u;
-      if (i < k) {
-        const double2 b = hr[i];
-        ar += a[u].x * b.x - a[u].y * b.y;
-        ai += a[u].x * b.y + a[u].y * b.x;
-        vt[i * P + lane] = a[u];
-      }
-    }
-  }
-  ws[sub][lane] = make_double2(ar, ai);
-  __syncthreads();
-  if (sub == 0) {
-    double sr = 0, si = 0;
-#pragma unroll
-    for (int q = 0; q < S; ++q) {
-      sr += ws[q][lane].x;
-      si += ws[q][lane].y;
-    }
-    const double2 v = make_double2(o.x - sr, o.y - si);
-    if (m < n) W[off] = v;
-    ws[0][lane] = m < n ? v : make_double2(0.0, 0.0);
-  }
-  __syncthreads();
-  const int jl = threadIdx.x & 7;
-  double2 w[T / 8];
-#pragma unroll
-  for (int t = 0; t < T / 8; ++t) w[t] = ws[0][jl + 8 * t];
-  for (int i = threadIdx.x >> 3; i < k; i += NT / 8) {
-    double dr = 0, di = 0;
-#pragma unroll
-    for (int t = 0; t < T / 8; ++t) {
-      const double2 a = vt[i * P + jl + 8 * t];
-      dr += a.x * w[t].x + a.y * w[t].y;
-      di += a.x * w[t].y - a.y * w[t].x;
-    }
-    dr = dpp_add<0x141, 0xF>(dpp_add<0x4E, 0xF>(dpp_add<0xB1, 0xF>(dr)));
-    di = dpp_add<0x141, 0xF>(dpp_add<0x4E, 0xF>(dpp_add<0xB1, 0xF>(di)));
-    if (jl == 0) part[((i64)r * nch + c) * k + i] = make_double2(dr, di);
-  }
-}
-
-// h[r, i] = sum_c part[(r * nch + c) * k + i]; 64 vectors per workgroup, one
-// sixteenth of the chunks per wave.
-__global__ __launch_bounds__(1024) void k_bupdots_reduce(int k, int kcap, int nch, const double2* __restrict__ part,
-                                                         const int* __restrict__ act, double2* __restrict__ h) {
-  const int r = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (!act[r]) return;
-  __shared__ double2 red[16][64];
-  const int i = blockIdx.x * 64 + lane;
-  const double2* p = part + (i64)r * nch * k + min(i, k - 1);
-  double sr = 0, si = 0;
-#pragma unroll 8
-  for (int c = wave; c < nch; c += 16) {
-    const double2 v = p[(i64)c * k];
-    sr += v.x;
-    si += v.y;
-  }
-  red[wave][lane] = make_double2(sr, si);
-  __syncthreads();
-  if (wave == 0 && i < k) {
-    for (int q = 1; q < 16; ++q) {
-      sr += red[q][lane].x;
-      si += red[q][lane].y;
-    }
-    h[(i64)r * kcap + i] = make_double2(sr, si);
-  }
-}
-
 // X[r] += sum_{i<cnt[r]} V_i[r] y[r, i]
 __global__ __launch_bounds__(BT) void k_bcombine(i64 n, int R, int kcap, const double2* __restrict__ V,
                                                  const double2* __restrict__ y, const int* __restrict__ cnt,
@@ -465,47 +368,6 @@ void update(i64 n, int R, int k, int kcap, const double* V, const double* h, con
   k_bupdate<<<g, BT, 0, s>>>(n, R, k, kcap, reinterpret_cast<const double2*>(V), reinterpret_cast<const double2*>(h),
                              act, reinterpret_cast<double2*>(W));
   HIP_OK(hipGetLastError());
-}
-
-// One pass up to 64 vectors (two workgroups per CU still fit): past that the
-// vectors need 144 KB or rows of 512 bytes, and both measured no faster than
-// two passes.  Up to 36 vectors 256 threads have all loads in flight at once
-// and more workgroups share a CU; past that 512 threads do.  30720 rows, 128
-// columns, us, two passes / 256 / 512 threads: 8 vectors 222 / 149 / 273, 32:
-// 730 / 495 / 549, 48: 1090 / 989 / 835, 64: 1410 / 1156 / 1040.
-constexpr int kFuseNarrow = 36, kFuseMax = 64;
-
-size_t part_count(i64 n, int R, int kcap) {
-  const i64 fused = std::min(kcap, kFuseMax) * ((n + BFROWS - 1) / BFROWS);
-  return (size_t)R * std::max<i64>((i64)kcap * dot_chunks(n), fused);
-}
-
-template <int NT>
-static void updots(i64 n, int R, int k, int kcap, const double* V, const double* h1, const int* act, double* W,
-                   double* part, double* h2, hipStream_t s) {
-  DM_REQUIRE(k <= kcap && R >= 1 && R <= 65535, DM_ERR_ARGUMENT, "batch width out of range");
-  const int nch = (int)((n + BFROWS - 1) / BFROWS);
-  const size_t smem = sizeof(double2) * (size_t)k * BFPITCH;
-  HIP_OK(hipFuncSetAttribute((const void*)k_bupdots<NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-  k_bupdots<NT><<<dim3((unsigned)nch, (unsigned)R), NT, smem, s>>>(
-      n, R, k, kcap, reinterpret_cast<const double2*>(V), reinterpret_cast<const double2*>(h1), act,
-      reinterpret_cast<double2*>(W), reinterpret_cast<double2*>(part), nch);
-  k_bupdots_reduce<<<dim3((unsigned)((k + 63) / 64), (unsigned)R), 1024, 0, s>>>(
-      k, kcap, nch, reinterpret_cast<const double2*>(part), act, reinterpret_cast<double2*>(h2));
-  HIP_OK(hipGetLastError());
-}
-
-void update_dots(i64 n, int R, int k, int kcap, const double* V, const double* h1, const int* act, double* W,
-                 double* part, double* h2, hipStream_t s) {
-  if (k <= 0) return;
-  if (k > kFuseMax) {
-    update(n, R, k, kcap, V, h1, act, W, s);
-    dots(n, R, k, kcap, V, W, act, part, h2, s);
-  } else if (k <= kFuseNarrow) {
-    updots<256>(n, R, k, kcap, V, h1, act, W, part, h2, s);
-  } else {
-    updots<512>(n, R, k, kcap, V, h1, act, W, part, h2, s);
-  }
 }
 
 void combine(i64 n, int R, int kcap, const double* V, const double* y, const int* cnt, double* X, hipStream_t s) {
