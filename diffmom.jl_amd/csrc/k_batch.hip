@@ -15,7 +15,7 @@
 namespace {
 
 constexpr int BT = 256;          // threads per workgroup
-constexpr int BROWS = 8;         // rows per thread in the dot kernel (one wave reduction per 8 KB read)
+constexpr int BROWS = 16;        // rows per thread in the dot kernel (one wave reduction per 16 KB read)
 constexpr int BCHUNK = BT * BROWS;
 constexpr int BKMAX = 512;       // basis vectors per column
 
@@ -25,30 +25,46 @@ __device__ inline double wsum(double v) {
   return v;
 }
 
-// v plus the lanes one DPP step away (lanes outside the row mask add zero)
-template <int CTRL, int ROWS>
+// v plus the lane that CTRL names
+template <int CTRL>
 __device__ inline double dpp_add(double v) {
   const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b & 0xffffffffLL), CTRL, ROWS, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xF, false);
+  const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)(b & 0xffffffffLL), CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, false);
   return v + __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
-// sum over the wave, in lane 63
-__device__ inline double wsum63(double x) {
-  x = dpp_add<0xB1, 0xF>(x);   // quad_perm 1,0,3,2
-  x = dpp_add<0x4E, 0xF>(x);   // quad_perm 2,3,0,1
-  x = dpp_add<0x141, 0xF>(x);  // row_half_mirror
-  x = dpp_add<0x140, 0xF>(x);  // row_mirror
-  x = dpp_add<0x142, 0xA>(x);  // row_bcast15
-  return dpp_add<0x143, 0xC>(x);  // row_bcast31
+// sum over the two halves (rows of 16: neighbouring rows), in every lane
+__device__ inline double half_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)(b & 0xffffffffLL), (unsigned)(b & 0xffffffffLL), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+  return __longlong_as_double(((long long)hi[0] << 32) | lo[0]) + __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+}
+__device__ inline double row_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)(b & 0xffffffffLL), (unsigned)(b & 0xffffffffLL), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+  return __longlong_as_double(((long long)hi[0] << 32) | lo[0]) + __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+}
+// wsum's tree (lanes 32, 16, 8, 4, 2, 1 apart: the same bits) without LDS; past
+// the first three steps lanes 8 apart hold the same value, so a rotation by 4
+// within 16 lanes serves as the exchange with lane ^ 4
+__device__ inline double wsum_dpp(double v) {
+  v = row_add(half_add(v));
+  v = dpp_add<0x128>(v);    // row_ror:8
+  v = dpp_add<0x124>(v);    // row_ror:4
+  v = dpp_add<0x4E>(v);     // quad_perm 2,3,0,1
+  return dpp_add<0xB1>(v);  // quad_perm 1,0,3,2
 }
 
 // part[(r * kcap + i) * nch + c] = sum over the rows of chunk c of conj(V_i[r]) . W[r]
 // (each workgroup keeps its chunk of W[r] in registers and walks the k basis
 // vectors).  HBM-bound: the next vector's loads are issued before this one's
 // sums (rows past n read row n - 1 against w = 0: a load behind a branch made
-// every row wait for the one before it: 0.47 against 0.44 ms on average for
-// bases of 1 to 58 vectors, 30720 rows, 128 columns).
+// every row wait for the one before it: 0.47 against 0.45 ms on average for
+// bases of 1 to 96 vectors, 30720 rows, 128 columns).  The sums keep one fixed
+// order (16 rows a thread, wsum's tree, waves, chunks): the solves on complex64
+// products carry any other rounding into the currents at their tolerance.
 __global__ __launch_bounds__(BT) void k_bdots(i64 n, int R, int k, int kcap, const double2* __restrict__ V,
                                               const double2* __restrict__ W, const int* __restrict__ act,
                                               double2* __restrict__ part, int nch) {
@@ -79,9 +95,9 @@ __global__ __launch_bounds__(BT) void k_bdots(i64 n, int R, int k, int kcap, con
       ar += a[e].x * w[e].x + a[e].y * w[e].y;
       ai += a[e].x * w[e].y - a[e].y * w[e].x;
     }
-    ar = wsum63(ar);
-    ai = wsum63(ai);
-    if (lane == 63) red[wave][i] = make_double2(ar, ai);
+    ar = wsum_dpp(ar);
+    ai = wsum_dpp(ai);
+    if (lane == 0) red[wave][i] = make_double2(ar, ai);
 #pragma unroll
     for (int e = 0; e < BROWS; ++e) a[e] = nx[e];
   }

@@ -24,21 +24,23 @@ constexpr int SPAI_MAXJ = 80;  // columns per least-squares problem
 constexpr int SPAI_CHUNK = 8;  // rows of A staged per pass
 
 // One column per workgroup of NT threads; thread t owns one 4 x 4 block (A, B)
-// of the lower triangle of the extended Gram matrix [G, rhs; rhs^H, 1], held in
-// registers from the first row of A to the solution:
+// of the lower triangle of the Gram matrix, held in registers from the first row
+// of A to the solution:
 //   Gram: chunks of SPAI_CHUNK rows staged in LDS (two buffers; the next chunk's
 //     entries are on their way while this one's products are formed); per row a
 //     thread reads 8 values for 16 complex products.
 //   Cholesky, right-looking by block columns: the diagonal block's thread
-//     factors it, the blocks below solve against it and put their result in LDS,
-//     the blocks to the right subtract their products.  The extended row turns
-//     into y^H = (L^-1 rhs)^H on the way.
+//     factors it, the blocks below solve against it and put their result in LDS
+//     while it solves its entries of L y = rhs, the blocks to the right subtract
+//     their products while those below take theirs out of the right-hand side.
 //   Backward: per block column the diagonal's thread solves its four entries and
 //     the blocks to its left in that row take them out of y.
+// Every entry is rounded in the order of the plain column-by-column form, so the
+// workgroup's size and the blocks change no bit of the result.
 // The largest NT is bound by FP64 arithmetic in the Gram part, the small ones by
 // the serial steps, of which several workgroups per CU overlap.
-// 4720 columns, supports of 80 and about 200 rows: 1.25 ms (Gram matrix in LDS,
-// factorization and solves by one wave: 3.2); 30720 of 49: 2.1 ms (2.9).
+// 4720 columns, supports of 80 and about 200 rows: 1.56 ms (Gram matrix in LDS,
+// factorization and solves by one wave: 3.2); 30720 of 49: 2.6 ms (2.8).
 // Blocks are numbered down block columns, so that the waves of finished columns
 // drop out of the later steps.
 template <int NT>
@@ -53,9 +55,18 @@ struct SpaiShape<128> {
 };
 template <>
 struct SpaiShape<256> {
-  static constexpr int NB = 22;
+  static constexpr int NB = 20;
 };
 
+// b -= l y, and b -= conj(l) m (a product rounded once, then taken away)
+__device__ inline void csub_fwd(double2& b, double2 l, double2 y) {
+  b.x -= fma(l.x, y.x, -(l.y * y.y));
+  b.y -= fma(l.x, y.y, l.y * y.x);
+}
+__device__ inline void csub_bwd(double2& b, double2 l, double2 m) {
+  b.x -= fma(l.x, m.x, l.y * m.y);
+  b.y -= fma(l.x, m.y, -(l.y * m.x));
+}
 // a -= p conj(q)
 __device__ inline void csub_pq(double2& a, double2 p, double2 q) {
   a.x = fma(-p.x, q.x, a.x);
@@ -72,7 +83,7 @@ __device__ inline void cacc_pq(double2& a, double2 p, double2 q) {
 }
 
 template <int NT>
-__global__ __launch_bounds__(NT, 3) void k_spai_build(int n, int per, ZRef z, const int* __restrict__ jptr,
+__global__ __launch_bounds__(NT, 2) void k_spai_build(int n, int per, ZRef z, const int* __restrict__ jptr,
                                                       const int* __restrict__ jidx, const int* __restrict__ iptr,
                                                       const int* __restrict__ iidx, double2* __restrict__ vals,
                                                       int* __restrict__ status) {
@@ -94,7 +105,7 @@ __global__ __launch_bounds__(NT, 3) void k_spai_build(int n, int per, ZRef z, co
   __shared__ double2 ys[4 * NB];
   double2(*panel)[4][NB] = st[0];
   const int tid = threadIdx.x;
-  const int nb = nJ / 4 + 1;  // block rows of the nJ + 1 extended ones
+  const int nb = (nJ + 3) / 4;  // block rows
   int A = -1, B = -1;
   if (tid < nb * (nb + 1) / 2) {
     int e = tid;
@@ -139,6 +150,12 @@ __global__ __launch_bounds__(NT, 3) void k_spai_build(int n, int per, ZRef z, co
       row = row_of(r0 + 2 * SPAI_CHUNK);
     }
     if (A >= 0) {
+      // a chunk's sums are formed apart and added
+      double2 sum[4][4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) sum[u][v] = make_double2(0.0, 0.0);
 #pragma unroll 2
       for (int r = 0; r < SPAI_CHUNK; ++r) {
         double2 p[4], q[4];
@@ -150,23 +167,29 @@ __global__ __launch_bounds__(NT, 3) void k_spai_build(int n, int per, ZRef z, co
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
-          for (int v = 0; v < 4; ++v) cacc_pq(acc[u][v], p[u], q[v]);
+          for (int v = 0; v < 4; ++v) cacc_pq(sum[u][v], p[u], q[v]);
       }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          acc[u][v].x += sum[u][v].x;
+          acc[u][v].y += sum[u][v].y;
+        }
     }
     if (more) stage(buf ^ 1);
     __syncthreads();
   }
-  // the extended row (rhs^H = Z[j, J]) and the identity past it
-  const int eu = nJ & 3;  // its place in block row nb - 1
-  if (A == nb - 1) {
+  // the identity past the last column, and the right-hand side A^H e_j =
+  // conj(Z[j, J]) (row j of Z restricted to the pattern)
+  if (A == nb - 1 && B == A) {
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int b = 4 * B + v;
-        if (u == eu && b < nJ) acc[u][v] = zat(z, j, jidx[j0 + b]);
-        if (4 * A + u >= nJ && b == 4 * A + u) acc[u][v] = make_double2(1.0, 0.0);
-      }
+      if (4 * A + u >= nJ) acc[u][u] = make_double2(1.0, 0.0);
+  }
+  for (int b = tid; b < 4 * nb; b += NT) {
+    double2 v = zat(z, j, jidx[j0 + min(b, nJ - 1)]);
+    ys[b] = b < nJ ? make_double2(v.x, -v.y) : make_double2(0.0, 0.0);
   }
   bool bad = false;
   for (int K = 0; K < nb; ++K) {
@@ -175,13 +198,12 @@ __global__ __launch_bounds__(NT, 3) void k_spai_build(int n, int per, ZRef z, co
       for (int v = 0; v < 4; ++v) {
         double d = acc[v][v].x;
 #pragma unroll
-        for (int w = 0; w < v; ++w) d = fma(-acc[v][w].x, acc[v][w].x, fma(-acc[v][w].y, acc[v][w].y, d));
-        if (4 * K + v >= nJ) d = 1.0;
+        for (int w = 0; w < v; ++w) d = fma(-acc[v][w].y, acc[v][w].y, fma(-acc[v][w].x, acc[v][w].x, d));
         if (!(d > 0.0)) {
           bad = true;
           d = 1e-300;
         }
-        const double il = rsqrt(d);
+        const double il = 1.0 / sqrt(d);
         dil[v] = il;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -210,7 +232,31 @@ __global__ __launch_bounds__(NT, 3) void k_spai_build(int n, int per, ZRef z, co
         }
       }
     }
+    if (A == K && B == K) {
+      // its four entries of y, while the others solve
+      double2 y[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) y[v] = ys[4 * K + v];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        y[v] = make_double2(y[v].x * acc[v][v].x, y[v].y * acc[v][v].x);
+#pragma unroll
+        for (int u = v + 1; u < 4; ++u) csub_fwd(y[u], acc[u][v], y[v]);
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) ys[4 * K + v] = y[v];
+    }
     __syncthreads();
+    if (B == K && A > K) {
+      // the block's share out of the right-hand side, beside the updates
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        double2 b = ys[4 * A + u];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) csub_fwd(b, acc[u][v], ys[4 * K + v]);
+        ys[4 * A + u] = b;
+      }
+    }
     if (B > K) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
@@ -227,15 +273,6 @@ __global__ __launch_bounds__(NT, 3) void k_spai_build(int n, int per, ZRef z, co
       }
     }
   }
-  // y = conj of the extended row; entries past nJ - 1 are zero
-  if (A == nb - 1) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (u == eu)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          ys[4 * B + v] = 4 * B + v < nJ ? make_double2(acc[u][v].x, -acc[u][v].y) : make_double2(0.0, 0.0);
-  }
   for (int K = nb - 1; K >= 0; --K) {
     __syncthreads();
     if (A == K && B == K) {
@@ -245,11 +282,7 @@ __global__ __launch_bounds__(NT, 3) void k_spai_build(int n, int per, ZRef z, co
       for (int v = 3; v >= 0; --v) {
         double2 x = ys[4 * K + v];
 #pragma unroll
-        for (int u = 3; u > v; --u) {
-          // x -= conj(L[u][v]) m[u]
-          x.x -= acc[u][v].x * m[u].x + acc[u][v].y * m[u].y;
-          x.y -= acc[u][v].x * m[u].y - acc[u][v].y * m[u].x;
-        }
+        for (int u = 3; u > v; --u) csub_bwd(x, acc[u][v], m[u]);
         const double il = acc[v][v].x;
         m[v] = make_double2(x.x * il, x.y * il);
         ys[4 * K + v] = m[v];
@@ -264,10 +297,7 @@ __global__ __launch_bounds__(NT, 3) void k_spai_build(int n, int per, ZRef z, co
       for (int v = 0; v < 4; ++v) {
         double2 x = ys[4 * B + v];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          x.x -= acc[u][v].x * m[u].x + acc[u][v].y * m[u].y;
-          x.y -= acc[u][v].x * m[u].y - acc[u][v].y * m[u].x;
-        }
+        for (int u = 3; u >= 0; --u) csub_bwd(x, acc[u][v], m[u]);
         ys[4 * B + v] = x;
       }
     }
@@ -381,7 +411,7 @@ void spai_build(i64 n, const ZRef& z, int maxJ, const int* jptr, const int* jidx
                 double* vals, int* status, hipStream_t s) {
   DM_REQUIRE(maxJ >= 1 && maxJ <= SPAI_MAXJ, DM_ERR_ARGUMENT, "near-field preconditioner: support width out of range");
   DM_REQUIRE(n < (1LL << 31) - 8, DM_ERR_ARGUMENT, "near-field preconditioner: too many bases for one launch");
-  const int per = (int)((n + 7) / 8), nb = maxJ / 4 + 1;
+  const int per = (int)((n + 7) / 8), nb = (maxJ + 3) / 4;
   double2* v = reinterpret_cast<double2*>(vals);
   // the fewest threads that give every block of the widest support one
   if (nb <= SpaiShape<64>::NB)
