@@ -629,9 +629,10 @@ __global__ __launch_bounds__(256) void k_lu_top(i64 ld, int k0, int w, const dou
 // ldu) on the FP64 matrix cores: 64 x 64 complex per workgroup, the whole
 // inner dimension staged at once (67 KB of LDS, two workgroups a CU), each
 // wave 32 real rows of the interleaved L (see k_zx.hip for the real form and
-// the output layout).  24 us on average over the panels of 1976 columns; the
-// matrix cores and the read-modify-write of T (from the last-level cache) take
-// about the same time.
+// the output layout).  20 us on average over the panels of 1976 columns (26
+// with each load behind its range test and T read last); the matrix cores and
+// the read-modify-write of T (from the last-level cache) take about the same
+// time.
 constexpr int LU_T = 64;
 __global__ __launch_bounds__(256, 2) void k_lu_update(i64 mr, i64 ncols, const double2* __restrict__ L, i64 ld,
                                                       const double2* __restrict__ U, i64 ldu,
@@ -639,21 +640,36 @@ __global__ __launch_bounds__(256, 2) void k_lu_update(i64 mr, i64 ncols, const d
   __shared__ double As[kLuW][2 * LU_T + 2];
   __shared__ double Br[kLuW][LU_T + 1];
   __shared__ double Bi[kLuW][LU_T + 1];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4;
   const i64 m0 = (i64)blockIdx.x * LU_T, c0 = (i64)blockIdx.y * LU_T;
+  // all loads clamped and unconditional, so that they are in flight together:
+  // L and U tiles, then the entries this lane updates (places past the end
+  // repeat the last row or column; their products are not stored)
+  double2 lv[8], uv[8], ev[2][4][2];
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
-    const int idx = tid + 256 * q, kk = idx >> 6, v = idx & 63;
-    const double2 e = m0 + v < mr ? L[m0 + v + (i64)kk * ld] : make_double2(0.0, 0.0);
-    As[kk][2 * v] = e.x;
-    As[kk][2 * v + 1] = e.y;
+    const int idx = tid + 256 * q;
+    lv[q] = L[min(m0 + (idx & 63), mr - 1) + (i64)(idx >> 6) * ld];
+    uv[q] = U[(idx & 31) + min(c0 + (idx >> 5), ncols - 1) * ldu];
   }
+  // lanes with even g hold rows r = 0, 1, odd g rows r = 2, 3 of a pair
+  auto row_at = [&](int r2, int h) {
+    return m0 + ((32 * wave + 16 * r2 + (g & ~1) + 4 * ((g & 1) ? 2 + h : h)) >> 1);
+  };
+#pragma unroll
+  for (int r2 = 0; r2 < 2; ++r2)
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        ev[r2][cb][h] = T[min(row_at(r2, h), mr - 1) + min(c0 + 16 * cb + (lane & 15), ncols - 1) * ldt];
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
-    const int idx = tid + 256 * q, kk = idx & 31, v = idx >> 5;
-    const double2 e = c0 + v < ncols ? U[kk + (c0 + v) * ldu] : make_double2(0.0, 0.0);
-    Br[kk][v] = e.x;
-    Bi[kk][v] = e.y;
+    const int idx = tid + 256 * q;
+    As[idx >> 6][2 * (idx & 63)] = lv[q].x;
+    As[idx >> 6][2 * (idx & 63) + 1] = lv[q].y;
+    Br[idx & 31][idx >> 5] = uv[q].x;
+    Bi[idx & 31][idx >> 5] = uv[q].y;
   }
   __syncthreads();
   v4d accP[2][4], accQ[2][4];
@@ -681,7 +697,6 @@ __global__ __launch_bounds__(256, 2) void k_lu_update(i64 mr, i64 ncols, const d
       }
     }
   }
-  const int g = lane >> 4;
 #pragma unroll
   for (int r2 = 0; r2 < 2; ++r2)
 #pragma unroll
@@ -695,18 +710,16 @@ __global__ __launch_bounds__(256, 2) void k_lu_update(i64 mr, i64 ncols, const d
         qo[r] = __shfl_xor(q[r], 16, 64);
       }
       if (col >= ncols) continue;
-      // lanes with even g write rows r = 0, 1, odd g rows r = 2, 3 of the pair
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const bool odd = (g & 1) != 0;
-        const i64 mrow = m0 + ((32 * wave + 16 * r2 + (g & ~1) + 4 * (odd ? 2 + h : h)) >> 1);
+        const i64 mrow = row_at(r2, h);
         if (mrow >= mr) continue;
         // even g: (p, q) are the real row's, (po, qo) the imaginary row's
         const double pre = odd ? po[2 + h] : p[h], pim = odd ? p[2 + h] : po[h];
         const double qre = odd ? qo[2 + h] : q[h], qim = odd ? q[2 + h] : qo[h];
-        double2* o = T + mrow + col * ldt;
-        const double2 e = *o;
-        *o = make_double2(e.x - (pre - qim), e.y - (qre + pim));
+        const double2 e = ev[r2][cb][h];
+        T[mrow + col * ldt] = make_double2(e.x - (pre - qim), e.y - (qre + pim));
       }
     }
 }
