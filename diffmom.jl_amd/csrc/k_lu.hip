@@ -9,7 +9,7 @@
 // Right-hand sides are carried as further columns of the matrix, so the
 // factorization leaves L^-1 P B in them and only U x = y remains
 // (k_lu_back: every workgroup solves its own columns).  n = 1976 with 64
-// right-hand sides: 9.0 + 0.64 ms; with a memory-resident panel and the
+// right-hand sides: 8.2 + 0.61 ms; with a memory-resident panel and the
 // solves column by column it took 25 + 64 x 3.4 ms.
 // Pivots: the largest |a|^2 in the column, the smallest row among equal ones.
 #include <hip/hip_runtime.h>
@@ -109,8 +109,9 @@ __device__ inline int exchange_map(int w, const int* piv, int lane, int& pos, in
   pos = lane < w ? lane : -1;
   src = pos;
   int cnt = w;
+  const int pv = piv[min(lane, w - 1)];  // lane j: exchange j
   for (int j = 0; j < w; ++j) {
-    const int p = __builtin_amdgcn_readfirstlane(piv[j]);
+    const int p = __builtin_amdgcn_readlane(pv, j);
     const unsigned long long hit = __ballot(pos == p);
     int b;
     if (hit) {
@@ -486,8 +487,9 @@ __global__ __launch_bounds__(1024) void k_lu_panel_mem(i64 n, i64 ld, int k0, in
 // own columns skipped, or a block of right-hand sides, own = 0).  64 columns
 // per workgroup; L11^-1 is formed in LDS by every workgroup (diagonal blocks of
 // 8, then two doublings) while the columns load, and multiplied on the FP64
-// matrix cores.  8-25 us a launch, most of it the block inversions' LDS
-// latency.  (One thread per column substituting through L11 waited ~100 cycles
+// matrix cores.  13 us a launch, most of it the block inversions' LDS
+// latency (17 with L11 read after the exchange map, the map's exchanges read
+// from LDS one by one and the exchanged rows kept in scratch).  (One thread per column substituting through L11 waited ~100 cycles
 // for each LDS read: 47 us.)
 __global__ __launch_bounds__(256) void k_lu_top(i64 ld, int k0, int w, const double2* __restrict__ A,
                                                 const int* __restrict__ ipiv, double2* __restrict__ T, i64 ldt,
@@ -501,6 +503,14 @@ __global__ __launch_bounds__(256) void k_lu_top(i64 ld, int k0, int w, const dou
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const i64 c0 = blockIdx.x * (i64)64;
   const bool solves = c0 + 64 > solve_from;
+  // L11 is on its way while the first wave turns the exchanges into a gather
+  double2 l11[kLuW * kLuW / 256];
+  if (solves)
+#pragma unroll
+    for (int q = 0; q < kLuW * kLuW / 256; ++q) {
+      const int e = tid + 256 * q;
+      l11[q] = A[k0 + min(e % kLuW, w - 1) + (i64)(k0 + min(e / kLuW, w - 1)) * ld];
+    }
   if (wave == 0) {
     int pos = lane, src = lane, cnt = w;
     if (swap) {
@@ -513,9 +523,10 @@ __global__ __launch_bounds__(256) void k_lu_top(i64 ld, int k0, int w, const dou
     if (lane == 0) xcnt = cnt;
   }
   if (solves)
-    for (int e = tid; e < kLuW * kLuW; e += 256) {
-      const int c = e / kLuW, r = e % kLuW;
-      L[r][c] = (c < w && r < w && r > c) ? A[k0 + r + (i64)(k0 + c) * ld] : make_double2(0.0, 0.0);
+#pragma unroll
+    for (int q = 0; q < kLuW * kLuW / 256; ++q) {
+      const int e = tid + 256 * q, c = e / kLuW, r = e % kLuW;
+      L[r][c] = (c < w && r < w && r > c) ? l11[q] : make_double2(0.0, 0.0);
       V[r][c] = make_double2(r == c ? 1.0 : 0.0, 0.0);
     }
   __syncthreads();
@@ -618,10 +629,11 @@ __global__ __launch_bounds__(256) void k_lu_top(i64 ld, int k0, int w, const dou
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
     const i64 col = c0 + v0 + 8 * q;
-    if (!valid(col)) continue;
-    double2* t = T + k0 + col * ldt;
-    if (i < w) t[i] = make_double2(Br[i][v0 + 8 * q], Bi[i][v0 + 8 * q]);
-    if (w + i < cnt) t[xpos[w + i]] = y[q];
+    const bool ok = valid(col);
+    double2* t = T + k0 + min(col, ncols - 1) * ldt;
+    const double2 ex = y[q];
+    if (ok && i < w) t[i] = make_double2(Br[i][v0 + 8 * q], Bi[i][v0 + 8 * q]);
+    if (ok && w + i < cnt) t[xpos[w + i]] = ex;
   }
 }
 
