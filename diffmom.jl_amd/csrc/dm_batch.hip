@@ -136,7 +136,7 @@ void gmres_batch(dm_ctx* ctx, i64 n, int R, DevOp& A, DevPrec* M, const double* 
     // the device, so only the Z X of a fully converged batch is wasted).  The
     // round trip costs about 25 us, the steps wasted 1.5 of some 60 on average:
     // from steps of about 1 ms on (n^2 R = 2e10) the flags are read every step
-    // (30720 unknowns, 128 columns: 721 -> 706 ms).  The relaxation still
+    // (30720 unknowns, 128 columns: 15 ms of 720).  The relaxation still
     // follows the estimates of every fourth.
     const bool every = (double)n * (double)n * R >= 2e10;
     for (int j = 0; j < mcap && total < maxiter; ++j) {
