@@ -1014,8 +1014,12 @@ int dm_apply(dm_ctx* ctx, const dm_zmat* z, int form, int adjoint, const double*
         // one permutation launch per direction for all columns (64 columns of
         // 7680: two launches a column took 0.3 ms)
         launch_permute_cols(n, R, ext, xe.p, n, xi.p, n, 1, adjoint != 0, s);
-        op->apply_batch(xi.p, yi.p, R, ws.p, s);
-        launch_permute_cols(n, R, ext, yi.p, n, xe.p, n, 0, adjoint != 0, s);
+        int j = 0;  // packed forms: the product's reduction writes caller order itself
+        while (j < R && op->apply_placed(xi.p + 2 * n * j, xe.p + 2 * n * j, ext, adjoint != 0, s)) ++j;
+        if (j == 0) {
+          op->apply_batch(xi.p, yi.p, R, ws.p, s);
+          launch_permute_cols(n, R, ext, yi.p, n, xe.p, n, 0, adjoint != 0, s);
+        }
       }
       HIP_OK(hipMemcpy2DAsync(Y + 2 * ldy * j0, 16 * ldy, out, 16 * n, 16 * n, R, hipMemcpyDeviceToHost, s));
       HIP_OK(hipStreamSynchronize(s));

@@ -46,6 +46,11 @@ struct DevOp {
   virtual void apply(const double* x, double* y, hipStream_t s) = 0;
   virtual void apply_batch(const double* X, double* Y, int R, void* ws, hipStream_t s) = 0;
   virtual size_t batch_ws(int R) const = 0;
+  // y[place[i]] = (A x)[i], conjugated if conj, where the operator's last kernel
+  // can write that (false: it cannot, nothing is done)
+  virtual bool apply_placed(const double* /*x*/, double* /*y*/, const int* /*place*/, bool /*conj*/, hipStream_t) {
+    return false;
+  }
 };
 struct OpZ64 : DevOp {
   const dm_zmat* z;
@@ -167,6 +172,12 @@ struct OpPacked : DevOp {
     if (!shape) shape = dmt::symv_shape(z->ctx, z, form, ws.p, s);
     ProfScope p(z->ctx, tag, s);
     dml::symv_packed(z->n, z->ref(form), x, y, ws.p, shape, s);
+  }
+  bool apply_placed(const double* x, double* y, const int* place, bool conj, hipStream_t s) override {
+    if (!shape) shape = dmt::symv_shape(z->ctx, z, form, ws.p, s);
+    ProfScope p(z->ctx, tag, s);
+    dml::symv_packed(z->n, z->ref(form), x, y, ws.p, shape, s, place, conj);
+    return true;
   }
   void apply_batch(const double* X, double* Y, int R, void*, hipStream_t s) override {
     for (int j = 0; j < R; ++j) apply(X + 2 * z->n * j, Y + 2 * z->n * j, s);

@@ -60,7 +60,9 @@ size_t symv_workspace_bytes(i64 n);
 // shape: 2..64 = LDS-staged form with that many tiles per workgroup segment;
 // 1000 + t (t = 1..1024) = wave form with t stored tiles per wave (chosen by
 // the tuner)
-void symv_packed(i64 n, const ZRef& z, const double* x, double* y, void* ws, int shape, hipStream_t s);
+// place: entry i of the product goes to y[place[i]]; conj: conjugated
+void symv_packed(i64 n, const ZRef& z, const double* x, double* y, void* ws, int shape, hipStream_t s,
+                 const int* place = nullptr, bool conj = false);
 // launch shapes worth timing for this size and precision
 std::vector<int> symv_shapes(i64 n, bool f32);
 // Compressed packed complex64 form: the cross approximation of the

@@ -220,8 +220,10 @@ __global__ __launch_bounds__(256) void k_symv(i64 n, int nb, int seg, const void
 }
 
 // y[R kPT + r] = sum_{J >= R} rowpart[tile (R, J)][r] + sum_{segments s of column R} colpart[s][r]
+// (entry g at place[g] where given, its imaginary part times sgn)
 __global__ void k_symv_reduce(i64 n, int nb, int seg, const double2* __restrict__ rowpart,
-                              const double2* __restrict__ colpart, double2* __restrict__ y) {
+                              const double2* __restrict__ colpart, double2* __restrict__ y,
+                              const int* __restrict__ place, double sgn) {
   const i64 g = blockIdx.x * (i64)blockDim.x + threadIdx.x;
   if (g >= n) return;
   const int R = (int)(g / kPT), r = (int)(g % kPT);
@@ -243,13 +245,14 @@ __global__ void k_symv_reduce(i64 n, int nb, int seg, const double2* __restrict_
     sr += v.x;
     si += v.y;
   }
+  const i64 to = place ? place[g] : g;
   const i64 sb = seg_base(R, seg);
   for (int s = 0; s <= R / seg; ++s) {
     double2 v = colpart[(sb + s) * kPT + r];
     sr += v.x;
     si += v.y;
   }
-  y[g] = make_double2(sr, si);
+  y[to] = make_double2(sr, sgn * si);
 }
 
 // ---------------------------------------------------------------- wave form
@@ -765,11 +768,13 @@ __global__ __launch_bounds__(256, 2) void k_symv_h(i64 n, int nb, int W, const i
 // y[R kPT + r] = sum_{J >= R} rowpart[tile (R, J)][r]
 //              + sum over the column runs of tile column R of their colpart
 // (a run ends at tile t = R (R + 1) / 2 + I when t + 1 is a multiple of tpw
-// or I = R); fixed order, deterministic.
+// or I = R); fixed order, deterministic.  Entry g goes to place[g] where given,
+// its imaginary part times sgn.
 template <typename P>
 __global__ __launch_bounds__(256) void k_symv_w_reduce(i64 n, int nb, int tpw, const unsigned char* __restrict__ rend,
                                                        int lanemajor, const P* __restrict__ rowpart,
-                                                       const P* __restrict__ colpart, double2* __restrict__ y) {
+                                                       const P* __restrict__ colpart, double2* __restrict__ y,
+                                                       const int* __restrict__ place, double sgn) {
   // 32 rows per block, 8 groups sharing the tiles of a row block round robin;
   // the groups' sums are added in a fixed order
   const int rl = threadIdx.x & 31, grp = threadIdx.x >> 5;
@@ -777,6 +782,7 @@ __global__ __launch_bounds__(256) void k_symv_w_reduce(i64 n, int nb, int tpw, c
   const int R = (int)min((i64)(nb - 1), (blockIdx.x * (i64)32) / kPT);
   // partial of row r: at r, or at 64 (r & 1) + (r >> 1) in the lane-major layout
   const int r = lanemajor ? (int)(((g & 1) << 6) + ((g % kPT) >> 1)) : (int)(g % kPT);
+  const i64 to = place ? place[min(g, n - 1)] : g;
   double sr = 0, si = 0;
   if (g < n) {
     int J = R + grp;
@@ -841,7 +847,7 @@ __global__ __launch_bounds__(256) void k_symv_w_reduce(i64 n, int nb, int tpw, c
       acc.x += part[q][rl].x;
       acc.y += part[q][rl].y;
     }
-    y[g] = acc;
+    y[to] = make_double2(acc.x, sgn * acc.y);
   }
 }
 
@@ -1042,7 +1048,7 @@ static void symv_hier_launch(i64 n, const float* z32p, const int* rank, const fl
                                                reinterpret_cast<const float2*>(fac), rmax,
                                                reinterpret_cast<const double2*>(x), rowpart, colpart);
   k_symv_w_reduce<P><<<(unsigned)((n + 31) / 32), 256, 0, s>>>(n, (int)nb, 1, hr.rend, 1, rowpart, colpart,
-                                                               reinterpret_cast<double2*>(y));
+                                                               reinterpret_cast<double2*>(y), nullptr, 1.0);
   HIP_OK(hipGetLastError());
 }
 
@@ -1078,7 +1084,8 @@ size_t symv_workspace_bytes(i64 n) {
   return (size_t)std::max(lds_form, wave_form) * kPT * sizeof(double2);
 }
 
-void symv_packed(i64 n, const ZRef& z, const double* x, double* y, void* ws, int shape, hipStream_t s) {
+void symv_packed(i64 n, const ZRef& z, const double* x, double* y, void* ws, int shape, hipStream_t s, const int* place,
+                 bool conj) {
   DM_REQUIRE(z.packed, DM_ERR_ARGUMENT, "symmetric product needs packed storage");
   const i64 nb = (n + kPT - 1) / kPT;
   if (shape >= kWaveShape) {
@@ -1096,7 +1103,7 @@ void symv_packed(i64 n, const ZRef& z, const double* x, double* y, void* ws, int
     else
       k_symv_w<0><<<(unsigned)blocks, 256, 0, s>>>(n, (int)nb, tpw, z.p, xv, rowpart, colpart);
     k_symv_w_reduce<double2><<<(unsigned)((n + 31) / 32), 256, 0, s>>>(n, (int)nb, tpw, nullptr, 0, rowpart, colpart,
-                                                              reinterpret_cast<double2*>(y));
+                                                              reinterpret_cast<double2*>(y), place, conj ? -1.0 : 1.0);
     HIP_OK(hipGetLastError());
     return;
   }
@@ -1112,7 +1119,7 @@ void symv_packed(i64 n, const ZRef& z, const double* x, double* y, void* ws, int
   else
     k_symv<0><<<(unsigned)nseg, 256, 0, s>>>(n, (int)nb, seg, z.p, xv, rowpart, colpart);
   k_symv_reduce<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, (int)nb, seg, rowpart, colpart,
-                                                              reinterpret_cast<double2*>(y));
+                                                              reinterpret_cast<double2*>(y), place, conj ? -1.0 : 1.0);
   HIP_OK(hipGetLastError());
 }
 
