@@ -19,6 +19,10 @@ namespace dmt {
 // must leave the same results whichever candidate it is given.
 int tune_choice(dm_ctx* ctx, const std::string& key, const std::vector<int>& cands, int fallback,
                 const std::function<void(int)>& run, hipStream_t s);
+// The same for a choice that changes the rounding of the results, which a timer
+// must not make: a loaded value (dm_tune_set) if it is one of cands, else value,
+// recorded under key as a timed choice would be.
+int fixed_choice(dm_ctx* ctx, const std::string& key, const std::vector<int>& cands, int value);
 }  // namespace dmt
 
 namespace dms {
@@ -95,10 +99,13 @@ struct OpZ32 : DevOp {
       planes.alloc(dml::zx_bf16_planes_elems(z->ld, z->n) * 2);
       dml::zx_bf16_split(z->n, z->ld, z->z32.p, planes.p, s);
     }
-    // FP32 accumulation chunk: key zx/c64/<n>/<R>
-    const int kc = dmt::tune_choice(
-        z->ctx, "zx/c64/" + std::to_string(z->n) + "/" + std::to_string(R), dml::zx_bf16_chunks(), 4096,
-        [&](int c) { dml::zx_bf16(z->n, z->ld, planes.p, X, z->n, R, Y, z->n, ws, s, c); }, s);
+    // FP32 accumulation chunk: key zx/c64/<n>/<R>.  4096 columns on every matrix:
+    // a chunk of 8192 is another order of the FP32 sums (9e-8 in the product, up to
+    // 1e-6 in the currents of a lockstep solve), and not faster by more than the
+    // timings scatter: 64 columns of 4143 unknowns 216 / 216 us, 7680: 254 / 430,
+    // 12542: 634 / 595, 30720: 2832 / 2911.
+    const int kc = dmt::fixed_choice(z->ctx, "zx/c64/" + std::to_string(z->n) + "/" + std::to_string(R),
+                                     dml::zx_bf16_chunks(), 4096);
     ProfScope p(z->ctx, nterms == 3 ? "zx_z32_relaxed" : "zx_z32", s);
     dml::zx_bf16(z->n, z->ld, planes.p, X, z->n, R, Y, z->n, ws, s, kc, nterms);
   }

@@ -67,6 +67,17 @@ int tune_choice(dm_ctx* ctx, const std::string& key, const std::vector<int>& can
   return best;
 }
 
+int fixed_choice(dm_ctx* ctx, const std::string& key, const std::vector<int>& cands, int value) {
+  auto it = ctx->tune.find(key);
+  if (it == ctx->tune.end()) {
+    if (tuning_enabled()) ctx->tune[key] = value;
+    return value;
+  }
+  DM_REQUIRE(std::find(cands.begin(), cands.end(), it->second) != cands.end(), DM_ERR_ARGUMENT,
+             "tuned value out of range for " + key);
+  return it->second;
+}
+
 namespace {
 std::string symv_key(const dm_zmat* z, int form) {
   return std::string("symv/") + (form == DM_Z32P ? "c64/" : "c128/") + std::to_string(z->n);
