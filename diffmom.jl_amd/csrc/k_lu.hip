@@ -314,16 +314,17 @@ __global__ __launch_bounds__(NT) void k_lu_panel(i64 n, i64 ld, int k0, int w, d
           else if (pos[r] == pv)
             pos[r] = lc;
         }
+        if (elim && mine) {
+#pragma unroll
+          for (int r = 0; r < RPT; ++r)
+            if (r == br) {
+#pragma unroll
+              for (int c = 0; c < W; ++c) prow[c] = a[r][c];
+            }
+        }
+        // also without a pivot: the next column's candidates overwrite these
+        __syncthreads();
         if (elim) {
-          if (mine) {
-#pragma unroll
-            for (int r = 0; r < RPT; ++r)
-              if (r == br) {
-#pragma unroll
-                for (int c = 0; c < W; ++c) prow[c] = a[r][c];
-              }
-          }
-          __syncthreads();
           // one LDS read for the whole row, its entries broadcast by lane
           // reads; columns already done (rotated to the end) are not updated
           const double2 pl = prow[lane & (W - 1)];
