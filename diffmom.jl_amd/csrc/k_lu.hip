@@ -34,14 +34,24 @@ __device__ inline double2 cfms(double2 c, double2 a, double2 b) {
   c.y = fma(-a.y, b.x, c.y);
   return c;
 }
+// 1 / d.  Where |d|^2 and its reciprocal are normal numbers, by |d|^2; else
+// (|d| beyond 2^-511 or 2^511) the same for d scaled by a power of two.
+__device__ inline bool plain_range(double dn) { return dn >= 0x1p-1022 && dn <= 0x1p1022; }
+__device__ inline double2 crecip_scaled(double2 d) {
+  const int e = ilogb(fmax(fabs(d.x), fabs(d.y)));
+  d = make_double2(scalbn(d.x, -e), scalbn(d.y, -e));
+  const double dn = d.x * d.x + d.y * d.y;
+  return make_double2(scalbn(d.x / dn, -e), scalbn(-d.y / dn, -e));
+}
 __device__ inline double2 crecip(double2 d) {
   const double dn = d.x * d.x + d.y * d.y;
+  if (!plain_range(dn)) return crecip_scaled(d);
   return make_double2(d.x / dn, -d.y / dn);
 }
-
-// 1 / d by one reciprocal of |d|^2 (hardware estimate, two Newton steps)
+// the same by one reciprocal of |d|^2 (hardware estimate, two Newton steps)
 __device__ inline double2 crecip_fast(double2 d) {
   const double dn = fma(d.x, d.x, d.y * d.y);
+  if (!plain_range(dn)) return crecip_scaled(d);
   double r = __builtin_amdgcn_rcp(dn);
   r = fma(fma(-dn, r, 1.0), r, r);
   r = fma(fma(-dn, r, 1.0), r, r);
