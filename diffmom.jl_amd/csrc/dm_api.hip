@@ -396,13 +396,30 @@ void solve_columns(dm_ctx* ctx, const dm_solve_opts& o, const dm_rwg& r, DevOp* 
   }
 }
 
-// Dense LU of z's complex128 matrix and the solution of the nrhs columns of Bd
-// (device, internal basis order, n x nrhs) into host X (caller order).  Up to
-// kLuRhs right-hand sides are carried through the factorization as further
-// columns; more take a forward substitution of their own per block.
+// Host right-hand sides (caller order, ldb) into Bd (internal order, n x nrhs),
+// kCols columns at a time in caller order on the device.
+void stage_rhs(dm_ctx* ctx, const dm_rwg& r, const double* B, i64 ldb, i64 nrhs, bool conj, double* Bd) {
+  constexpr i64 kCols = 64;
+  hipStream_t s = ctx->stream;
+  const i64 n = r.n;
+  DBuf<double> be;
+  be.alloc((size_t)2 * n * std::max<i64>(std::min(nrhs, kCols), 1));
+  for (i64 j = 0; j < nrhs; j += kCols) {
+    const i64 c = std::min(kCols, nrhs - j);
+    HIP_OK(hipMemcpy2DAsync(be.p, 16 * n, B + 2 * ldb * j, 16 * ldb, 16 * n, c, hipMemcpyHostToDevice, s));
+    launch_permute_cols(n, c, r.d_ext.p, be.p, n, Bd + 2 * n * j, n, 1, conj, s);
+  }
+}
+
+// Dense LU of z's complex128 matrix and the solution of nrhs columns into host
+// X (caller order).  rhs(j, R) gives columns j .. j + R - 1 (R <= kLuRhs) on the
+// device in internal order, n x R, valid until its next call.  Up to kLuRhs
+// right-hand sides are carried through the factorization as further columns;
+// more take a forward substitution of their own per block.
 constexpr i64 kLuRhs = 1024;
-void solve_direct(dm_ctx* ctx, const dm_rwg& r, const dm_zmat* z, const double* Bd, i64 nrhs, bool conj_out,
-                  double* X, i64 ldx, bool name_pivot, double t0, dm_solve_stats& st, double& worst) {
+void solve_direct(dm_ctx* ctx, const dm_rwg& r, const dm_zmat* z,
+                  const std::function<const double*(i64, i64)>& rhs, i64 nrhs, bool conj_out, double* X, i64 ldx,
+                  bool name_pivot, double t0, dm_solve_stats& st, double& worst) {
   hipStream_t s = ctx->stream;
   const i64 n = z->n, ld = z->ld, R0 = std::min(nrhs, kLuRhs);
   DBuf<double> A, x, xe, tmp, nr;
@@ -411,9 +428,11 @@ void solve_direct(dm_ctx* ctx, const dm_rwg& r, const dm_zmat* z, const double* 
   A.alloc((size_t)2 * ld * (n + R0));
   HIP_OK(hipMemcpyAsync(A.p, z->z64.p, (size_t)16 * ld * n, hipMemcpyDeviceToDevice, s));
   double* Y = A.p + (size_t)2 * ld * n;
+  const double* Bd = nullptr;  // the block's right-hand sides
   auto put_rhs = [&](i64 j0, i64 R) {
-    if (R > 0)
-      HIP_OK(hipMemcpy2DAsync(Y, 16 * ld, Bd + 2 * n * j0, 16 * n, 16 * n, R, hipMemcpyDeviceToDevice, s));
+    if (R <= 0) return;
+    Bd = rhs(j0, R);
+    HIP_OK(hipMemcpy2DAsync(Y, 16 * ld, Bd, 16 * n, 16 * n, R, hipMemcpyDeviceToDevice, s));
   };
   put_rhs(0, R0);
   ipiv.alloc(n);
@@ -447,7 +466,7 @@ void solve_direct(dm_ctx* ctx, const dm_rwg& r, const dm_zmat* z, const double* 
     // relative true residuals of the block, column by column
     for (i64 q = 0; q < R; q += RB) {
       const int w = (int)std::min(RB, R - q);
-      const double* b = Bd + 2 * n * (j0 + q);
+      const double* b = Bd + 2 * n * q;
       op.apply_batch(x.p + 2 * n * q, tmp.p, w, ws.p, s);
       dml::axpby(n * w, 1, 0, b, -1, 0, tmp.p, s);
       dmb::norm2(n, w, tmp.p, nullptr, nr.p, s);
@@ -1472,7 +1491,7 @@ int dm_solve_scattering_pw(dm_ctx* ctx, const dm_rwg* rwg_c, double k_re, double
     double worst = 0;
     bool all_ok = true;
     if (o.method == DM_METHOD_LU) {
-      solve_direct(ctx, r, z.get(), V.p, nrhs, false, X, n, false, t1, st, worst);
+      solve_direct(ctx, r, z.get(), [&](i64 j, i64) { return V.p + 2 * n * j; }, nrhs, false, X, n, false, t1, st, worst);
     } else {
       auto M = build_precond(z.get(), pick_form(z.get(), o.method == DM_METHOD_MIXED, batched), o, s);
       HIP_OK(hipStreamSynchronize(s));
@@ -1522,15 +1541,14 @@ int dm_solve(dm_ctx* ctx, const dm_zmat* z, const double* B, int64_t ldb, int64_
     double t0 = now();
     if (o.method == DM_METHOD_LU) {
       DM_REQUIRE(z->forms & DM_Z64, DM_ERR_ARGUMENT, "dense LU needs the complex128 matrix");
-      DBuf<double> Bx, Bd;
-      Bx.alloc((size_t)2 * n * nrhs);
-      Bd.alloc((size_t)2 * n * nrhs);
-      if (nrhs > 0) {
-        HIP_OK(hipMemcpy2DAsync(Bx.p, 16 * n, B, 16 * ldb, 16 * n, nrhs, hipMemcpyHostToDevice, s));
-        launch_permute_cols(n, nrhs, r.d_ext.p, Bx.p, n, Bd.p, n, 1, o.adjoint != 0, s);
-      }
+      DBuf<double> Bd;
+      Bd.alloc((size_t)2 * n * std::min(nrhs, kLuRhs));
+      auto rhs = [&](i64 j, i64 R) {
+        stage_rhs(ctx, r, B + 2 * ldb * j, ldb, R, o.adjoint != 0, Bd.p);
+        return Bd.p;
+      };
       double worst = 0;
-      solve_direct(ctx, r, z, Bd.p, nrhs, o.adjoint != 0, X, ldx, true, t0, st, worst);
+      solve_direct(ctx, r, z, rhs, nrhs, o.adjoint != 0, X, ldx, true, t0, st, worst);
       st.solved = 1;
       st.residual = worst;
       st.solve_time_s = now() - t0 - st.precond_time_s;
@@ -1551,15 +1569,9 @@ int dm_solve(dm_ctx* ctx, const dm_zmat* z, const double* B, int64_t ldb, int64_
     if (f32) A32 = make_op(z, o.method == DM_METHOD_MIXED ? op_form(z, batched) : f32);
     bool all_ok = true;
     double worst = 0;
-    DBuf<double> be, Bd;
-    constexpr i64 kCols = 64;  // columns staged in caller order per launch
-    be.alloc((size_t)2 * n * std::max<i64>(std::min(nrhs, kCols), 1));
+    DBuf<double> Bd;
     Bd.alloc((size_t)2 * n * std::max<i64>(nrhs, 1));
-    for (i64 j = 0; j < nrhs; j += kCols) {
-      const i64 c = std::min(kCols, nrhs - j);
-      HIP_OK(hipMemcpy2DAsync(be.p, 16 * n, B + 2 * ldb * j, 16 * ldb, 16 * n, c, hipMemcpyHostToDevice, s));
-      launch_permute_cols(n, c, r.d_ext.p, be.p, n, Bd.p + 2 * n * j, n, 1, o.adjoint != 0, s);
-    }
+    stage_rhs(ctx, r, B, ldb, nrhs, o.adjoint != 0, Bd.p);
     solve_columns(ctx, o, r, A64.get(), A32.get(), M.get(), Bd.p, n, nrhs, X, ldx, st, worst, all_ok, nullptr,
                   o.adjoint != 0);
     st.solved = all_ok ? 1 : 0;
