@@ -526,18 +526,22 @@ int dm_create(int device, dm_ctx** out) {
 int dm_destroy(dm_ctx* ctx) {
   return guard([&] {
     if (!ctx) return;
-    (void)hipSetDevice(ctx->device);
-    (void)hipStreamSynchronize(ctx->stream);
-    (void)hipStreamSynchronize(ctx->stream2);
-    ctx->cache.clear();
-    for (auto& r : ctx->recs) {
-      (void)hipEventDestroy(r.a);
-      (void)hipEventDestroy(r.b);
+    {
+      std::lock_guard<std::mutex> lk(ctx->mu);
+      (void)hipSetDevice(ctx->device);
+      (void)hipStreamSynchronize(ctx->stream);
+      (void)hipStreamSynchronize(ctx->stream2);
+      ctx->cache.clear();
+      for (auto& r : ctx->recs) {
+        (void)hipEventDestroy(r.a);
+        (void)hipEventDestroy(r.b);
+      }
+      for (hipEvent_t e : ctx->ev_free) (void)hipEventDestroy(e);
+      (void)hipStreamDestroy(ctx->stream);
+      (void)hipStreamDestroy(ctx->stream2);
+      ctx->closed = true;
     }
-    for (hipEvent_t e : ctx->ev_free) (void)hipEventDestroy(e);
-    (void)hipStreamDestroy(ctx->stream);
-    (void)hipStreamDestroy(ctx->stream2);
-    delete ctx;
+    if (--ctx->refs == 0) delete ctx;  // else the last handle does
   });
 }
 
@@ -1066,6 +1070,7 @@ int dm_apply_noalloc(dm_ctx* ctx, const dm_zmat* z, int form, int adjoint, const
                                          " bytes of scratch for this form, more than its " +
                                          std::to_string(kScratchBytes) + " bytes");
     std::lock_guard<std::mutex> lk(ctx->mu);
+    DM_REQUIRE(!ctx->closed, DM_ERR_ARGUMENT, "the context of this handle was destroyed");
     HIP_OK(hipSetDevice(ctx->device));
     unsigned char* base = static_cast<unsigned char*>(scratch_of(ctx->device));
     DM_REQUIRE(base != nullptr, DM_ERR_DEVICE, "scratch of this device was not set up (dm_create)");

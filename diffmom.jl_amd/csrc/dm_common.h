@@ -7,6 +7,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <atomic>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -137,6 +138,8 @@ struct dm_ctx {
   hipStream_t stream = nullptr;   // main stream: every public call runs here
   hipStream_t stream2 = nullptr;  // second stream for overlapped work
   std::mutex mu;
+  std::atomic<int> refs{1};       // dm_destroy's own and one per live handle (CtxRef)
+  bool closed = false;            // dm_destroy has run: no streams, no cache (under mu)
   int cu_count = 256;
   int prof = 0;  // HIP events around tracked launches: 0 none, 1 all, 2 operator products only
   std::vector<ProfRec> recs;
@@ -153,6 +156,30 @@ struct dm_ctx {
     ev_free.pop_back();
     return e;
   }
+};
+
+// A handle's hold on its context: handles may be freed after dm_destroy (a
+// program's garbage collector frees them in any order), so the last one deletes
+// the record.
+struct CtxRef {
+  dm_ctx* p = nullptr;
+  CtxRef() = default;
+  explicit CtxRef(dm_ctx* c) { *this = c; }
+  CtxRef(const CtxRef&) = delete;
+  CtxRef& operator=(const CtxRef& o) { return *this = o.p; }
+  CtxRef& operator=(dm_ctx* c) {
+    if (c) ++c->refs;
+    release();
+    p = c;
+    return *this;
+  }
+  ~CtxRef() { release(); }
+  void release() {
+    if (p && --p->refs == 0) delete p;
+    p = nullptr;
+  }
+  operator dm_ctx*() const { return p; }
+  dm_ctx* operator->() const { return p; }
 };
 
 // Brackets one tracked launch with HIP events on its stream when profiling is on.
@@ -185,6 +212,7 @@ struct CtxScope {
   dm_ctx* c;
   DevCache* prev;
   explicit CtxScope(dm_ctx* c_) : lk(c_->mu), c(c_), prev(tl_cache) {
+    DM_REQUIRE(!c->closed, DM_ERR_ARGUMENT, "the context of this handle was destroyed");
     HIP_OK(hipSetDevice(c->device));
     c->cache.promote(c->stream, c->stream2);
     tl_cache = &c->cache;
@@ -195,17 +223,33 @@ struct CtxScope {
   }
 };
 // The same for freeing a handle of the context: small blocks stay in the cache.
+// After dm_destroy they go back to the device.
 struct FreeScope {
-  CtxScope sc;
-  explicit FreeScope(dm_ctx* c) : sc(c) { c->cache.freeing = true; }
-  ~FreeScope() { sc.c->cache.freeing = false; }
+  CtxRef keep;  // the handle's own hold ends inside the scope
+  std::lock_guard<std::mutex> lk;
+  DevCache* prev;
+  explicit FreeScope(dm_ctx* c) : keep(c), lk(c->mu), prev(tl_cache) {
+    (void)hipSetDevice(c->device);
+    tl_cache = nullptr;
+    if (c->closed) return;
+    c->cache.promote(c->stream, c->stream2);
+    c->cache.freeing = true;
+    tl_cache = &c->cache;
+  }
+  ~FreeScope() {
+    if (!keep->closed) {
+      keep->cache.freeing = false;
+      keep->cache.promote(keep->stream, keep->stream2);
+    }
+    tl_cache = prev;
+  }
 };
 
 // Message returned by dm_last_error() for the calling thread.
 void dm_set_error(const std::string& msg);
 
 struct dm_mesh {
-  dm_ctx* ctx = nullptr;
+  CtxRef ctx;
   i64 nv = 0, nt = 0;
   std::vector<double> xyz;  // 3 x nv
   std::vector<i64> tri;     // 3 x nt, 1-based
@@ -241,7 +285,7 @@ struct SpaiPattern {
 struct dm_zmat;
 struct dm_rwg {
   const dm_mesh* mesh = nullptr;
-  dm_ctx* ctx = nullptr;
+  CtxRef ctx;
   i64 n = 0;
   // caller-order arrays (1-based triangle / vertex ids)
   std::vector<i64> tplus, tminus, evert, vplus_opp, vminus_opp;
@@ -328,7 +372,7 @@ __device__ inline double2 zat(const ZRef& z, i64 r, i64 c) {
 }
 
 struct dm_zmat {
-  dm_ctx* ctx = nullptr;
+  CtxRef ctx;
   const dm_rwg* rwg = nullptr;
   i64 n = 0, ld = 0;
   int forms = 0;
@@ -362,7 +406,7 @@ struct dm_zmat {
 };
 
 struct dm_mfop {
-  dm_ctx* ctx = nullptr;
+  CtxRef ctx;
   const dm_rwg* rwg = nullptr;
   double k_re = 0, k_im = 0, eta0 = 0;
   int quad_order = 3;

@@ -20,14 +20,14 @@
 #include "k_mpnn.h"
 
 struct dm_mpnn {
-  dm_ctx* ctx = nullptr;
+  CtxRef ctx;
   DBuf<float> p, m, v, g;  // FP32 master parameters, Adam moments, gradient
   DBuf<uint16_t> pb;       // bfloat16 copy used by the kernels
   int step = 0;
 };
 
 struct dm_mpnn_data {
-  dm_ctx* ctx = nullptr;
+  CtxRef ctx;
   i64 nnode = 0;
   int ns = 0;
   std::vector<int64_t> ptr;  // host copy of the sample offsets

@@ -68,7 +68,8 @@ typedef struct dm_mfop dm_mfop;
 /* A context keeps device blocks released by its calls for reuse by later
  * calls of the same size (at most min(64 GB, a quarter of the device)), and
  * blocks of freed handles of up to 128 MiB each (2 GiB in all); dm_destroy
- * frees them. */
+ * frees them.  Handles may be freed after their context was destroyed (any
+ * other use of them is refused then). */
 int dm_create(int device, dm_ctx** out);
 int dm_destroy(dm_ctx* ctx);
 const char* dm_last_error(void);
