@@ -40,6 +40,11 @@ double time_ms(Launch&& run, hipStream_t s) {
   HIP_OK(hipEventElapsedTime(&ms, a, b));
   (void)hipEventDestroy(a);
   (void)hipEventDestroy(b);
+  // The runtime drops timed launches' holds on their buffers in its callback
+  // thread, some 0.1 ms later; a block freed before that is returned to the
+  // device by that thread, after hipFree.  A host function waits its turn there.
+  HIP_OK(hipLaunchHostFunc(s, [](void*) {}, nullptr));
+  HIP_OK(hipStreamSynchronize(s));
   return ms / 3.0;
 }
 
