@@ -299,13 +299,12 @@ __global__ void k_scatter(i64 n, i64 gnode0, const int* __restrict__ nbr, const 
   gh_out[idx] += acc;
 }
 
-// part[b][a * KB1 + c] = sum over this workgroup's nodes of A'[i][a] B[i][c],
-// A' = A (1 - T^2) when T is given, B column KB (bias) = 1 when bias.
+// part[b][a * KB + c] = sum over this workgroup's nodes of A[i][a] B[i][c]
 template <int LA, int KB>
-__global__ __launch_bounds__(256) void k_outer(i64 n, const float* __restrict__ A, const float* __restrict__ T,
-                                               const float* __restrict__ B, int bias, float* __restrict__ part) {
-  constexpr int KB1 = KB + 1;
-  constexpr int O = LA * KB1;
+__global__ __launch_bounds__(256) void k_outer(i64 n, const float* __restrict__ A, const float* __restrict__ B,
+                                               float* __restrict__ part) {
+  constexpr int KB1 = KB + 1;  // padded rows
+  constexpr int O = LA * KB;
   constexpr int PER = (O + 255) / 256;
   __shared__ float As[NT * LA];
   __shared__ float Bs[NT * KB1];
@@ -320,32 +319,22 @@ __global__ __launch_bounds__(256) void k_outer(i64 n, const float* __restrict__ 
     for (int e = tid; e < NT * LA; e += 256) {
       int nd = e / LA, a = e % LA;
       i64 gi = i0 + nd;
-      float v = 0.f;
-      if (gi < n) {
-        v = A[gi * LA + a];
-        if (T) {
-          float tt = T[gi * LA + a];
-          v *= 1.f - tt * tt;
-        }
-      }
-      As[nd * LA + a] = v;
+      As[nd * LA + a] = gi < n ? A[gi * LA + a] : 0.f;
     }
-    for (int e = tid; e < NT * KB1; e += 256) {
-      int nd = e / KB1, c = e % KB1;
+    for (int e = tid; e < NT * KB; e += 256) {
+      int nd = e / KB, c = e % KB;
       i64 gi = i0 + nd;
-      Bs[nd * KB1 + c] = gi < n ? (c < KB ? B[gi * KB + c] : 1.f) : 0.f;
+      Bs[nd * KB1 + c] = gi < n ? B[gi * KB + c] : 0.f;
     }
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int o = tid + 256 * j;
       if (o < O) {
-        const int a = o / KB1, c = o % KB1;
-        if (c < KB || bias) {
-          float s = 0.f;
-          for (int nd = 0; nd < NT; ++nd) s += As[nd * LA + a] * Bs[nd * KB1 + c];
-          acc[j] += s;
-        }
+        const int a = o / KB, c = o % KB;
+        float s = 0.f;
+        for (int nd = 0; nd < NT; ++nd) s += As[nd * LA + a] * Bs[nd * KB1 + c];
+        acc[j] += s;
       }
     }
   }
@@ -439,12 +428,14 @@ __global__ __launch_bounds__(256) void k_outer_pair(i64 n, const float* __restri
 }
 
 // grad[woff + a * KB + c] (c < KB), grad[boff + a] (c == KB, bias) from G
-// partials: the four waves of a workgroup take the partials b = wave mod 4 of
-// 64 sums, then their FP64 sums are added in order.
-__global__ __launch_bounds__(256) void k_outer_reduce(int G, int LA, int KB, int bias, const float* __restrict__ part,
-                                                      float* __restrict__ grad, int woff, int boff) {
+// partials of LA rows of KB1 values (KB, or KB + 1 with a bias column): the four
+// waves of a workgroup take the partials b = wave mod 4 of 64 sums, then their
+// FP64 sums are added in order.
+__global__ __launch_bounds__(256) void k_outer_reduce(int G, int LA, int KB, int KB1, int bias,
+                                                      const float* __restrict__ part, float* __restrict__ grad,
+                                                      int woff, int boff) {
   __shared__ double red[4][64];
-  const int KB1 = KB + 1, O = LA * KB1;
+  const int O = LA * KB1;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int o = blockIdx.x * 64 + lane;
   double s = 0;
@@ -667,12 +658,10 @@ void acols_adj(i64 n, int k, const float* A, const float2* x, double* out, hipSt
 }
 
 template <int LA, int KB>
-void outer(i64 n, const float* A, const float* T, const float* B, int bias, float* part, float* grad, int woff,
-           int boff, hipStream_t s) {
+void outer(i64 n, const float* A, const float* B, float* part, float* grad, int woff, hipStream_t s) {
   const int G = (int)std::min<i64>(OUTER_G, std::max<i64>(1, (n + NT - 1) / NT));
-  k_outer<LA, KB><<<G, 256, 0, s>>>(n, A, T, B, bias, part);
-  const int O = LA * (KB + 1);
-  k_outer_reduce<<<(O + 63) / 64, 256, 0, s>>>(G, LA, KB, bias, part, grad, woff, boff);
+  k_outer<LA, KB><<<G, 256, 0, s>>>(n, A, B, part);
+  k_outer_reduce<<<(LA * KB + 63) / 64, 256, 0, s>>>(G, LA, KB, KB, 0, part, grad, woff, 0);
 }
 
 // weight and bias gradients of one layer: left factor gh (1 - t^2), right
@@ -682,8 +671,8 @@ void outer_layer(i64 n, const float* gh, const float* t, const float* hin, const
   const int G = (int)std::min<i64>(OUTER_G, std::max<i64>(1, (n + NT - 1) / NT));
   constexpr int O = H * (H + 1);
   k_outer_pair<<<G, 256, 0, s>>>(n, gh, t, hin, ml, part);
-  k_outer_reduce<<<(O + 63) / 64, 256, 0, s>>>(G, H, H, 1, part, grad, ws, bo);
-  k_outer_reduce<<<(O + 63) / 64, 256, 0, s>>>(G, H, H, 0, part + (size_t)G * O, grad, wn, 0);
+  k_outer_reduce<<<(O + 63) / 64, 256, 0, s>>>(G, H, H, H + 1, 1, part, grad, ws, bo);
+  k_outer_reduce<<<(O + 63) / 64, 256, 0, s>>>(G, H, H, H + 1, 0, part + (size_t)G * O, grad, wn, 0);
 }
 
 }  // namespace
@@ -736,7 +725,7 @@ void backward(const Graph& g, i64 gnode0, const uint16_t* prm, const Cache& c, c
   float* gh = work;
   float* gh2 = work + n * H;
   float* gm = work + 2 * n * H;
-  outer<2, H>(n, gy, nullptr, c.h + (i64)L * n * H, 0, part, grad, OFF_WD, 0, s);
+  outer<2, H>(n, gy, c.h + (i64)L * n * H, part, grad, OFF_WD, s);
   k_decode_back<<<nb256(n * H), 256, 0, s>>>(n, reinterpret_cast<const float2*>(gy), prm + OFF_WD, gh);
   const unsigned gl = (unsigned)((n + NT - 1) / NT);
   for (int l = L - 1; l >= 0; --l) {
@@ -748,7 +737,7 @@ void backward(const Graph& g, i64 gnode0, const uint16_t* prm, const Cache& c, c
     k_scatter<<<nb256(n * H), 256, 0, s>>>(n, gnode0, g.nbr, g.sgn, gm, gh2);
     std::swap(gh, gh2);
   }
-  outer<H, FIN>(n, gh, nullptr, c.u, 0, part, grad, OFF_WE, 0, s);
+  outer<H, FIN>(n, gh, c.u, part, grad, OFF_WE, s);
   HIP_OK(hipGetLastError());
 }
 
