@@ -816,8 +816,9 @@ __device__ inline void tile_body(const AsmArgs& a, int cap, AccT* __restrict__ z
       }
       if (l == 0 && go < a.n) {
         const double ln = a.len[go];
-        atomicAdd(y + 2 * go, (Pr * accr - Pi * acci) * ln);
-        atomicAdd(y + 2 * go + 1, (Pr * acci + Pi * accr) * ln);
+        // (real k: Pr = 0, and 0 times an infinite sum is no number)
+        atomicAdd(y + 2 * go, (Pr == 0.0 ? -(Pi * acci) : Pr * accr - Pi * acci) * ln);
+        atomicAdd(y + 2 * go + 1, (Pr == 0.0 ? Pi * accr : Pr * acci + Pi * accr) * ln);
       }
     }
   }
