@@ -1024,8 +1024,8 @@ int dm_apply(dm_ctx* ctx, const dm_zmat* z, int form, int adjoint, const double*
       const int* ext = z->rwg->d_ext.p;
       const double* out = xe.p;
       if (R < kMfmaMinRhs && gemv_small_fits(n) && (form == DM_Z64 || form == DM_Z32)) {
-        ProfScope p(ctx, form == DM_Z64 ? "gemv_z64" : "gemv_z32", s);
         for (int j = 0; j < R; ++j) {
+          ProfScope p(ctx, form == DM_Z64 ? "gemv_z64" : "gemv_z32", s);
           const i64 at = 2 * n * j;
           if (form == DM_Z64)
             launch_gemv_small_z64(n, z->ld, z->z64.p, ext, xe.p + at, yi.p + at, adjoint != 0, s);
@@ -1037,9 +1037,10 @@ int dm_apply(dm_ctx* ctx, const dm_zmat* z, int form, int adjoint, const double*
         // one permutation launch per direction for all columns (64 columns of
         // 7680: two launches a column took 0.3 ms)
         launch_permute_cols(n, R, ext, xe.p, n, xi.p, n, 1, adjoint != 0, s);
-        int j = 0;  // packed forms: the product's reduction writes caller order itself
-        while (j < R && op->apply_placed(xi.p + 2 * n * j, xe.p + 2 * n * j, ext, adjoint != 0, s)) ++j;
-        if (j == 0) {
+        bool placed = true;  // packed forms: the product's reduction writes caller order itself
+        for (int j = 0; placed && j < R; ++j)
+          placed = op->apply_placed(xi.p + 2 * n * j, xe.p + 2 * n * j, ext, adjoint != 0, s);
+        if (!placed) {
           op->apply_batch(xi.p, yi.p, R, ws.p, s);
           launch_permute_cols(n, R, ext, yi.p, n, xe.p, n, 0, adjoint != 0, s);
         }
