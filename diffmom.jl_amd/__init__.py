@@ -1045,11 +1045,15 @@ class ScatteringResult:
 def mesh_resolution_report(mesh, freq_hz, points_per_wavelength=10.0, c0=C0_DEFAULT):
     """src/geometry/Mesh.jl:3418-3471"""
     lam = c0 / freq_hz
-    t = mesh.tri - 1
+    t = np.asarray(mesh.tri).astype(np.int64) - 1
+    nv = len(mesh.xyz)
     a = np.concatenate([t[:, 0], t[:, 1], t[:, 2]])
     b = np.concatenate([t[:, 1], t[:, 2], t[:, 0]])
-    key = np.unique(np.minimum(a, b) * mesh.nv + np.maximum(a, b))  # one integer per edge
-    e = np.stack([key // mesh.nv, key % mesh.nv], axis=1)
+    if t.size and 0 <= t.min() and t.max() < nv:
+        key = np.unique(np.minimum(a, b) * nv + np.maximum(a, b))  # one integer per edge
+        e = np.stack([key // nv, key % nv], axis=1)
+    else:  # indexing decides
+        e = np.unique(np.sort(np.stack([a, b], axis=1), axis=1), axis=0)
     lens = np.sort(np.linalg.norm(mesh.xyz[e[:, 0]] - mesh.xyz[e[:, 1]], axis=1))
     target = lam / points_per_wavelength
     return dict(wavelength_m=lam, target_max_edge_m=target, edge_min_m=lens[0], edge_max_m=lens[-1],
