@@ -89,6 +89,13 @@ void DevCache::trim() {
   }
   free_blocks.clear();
 }
+void DevCache::reclaim() {
+  // (released blocks may still be in use by queued kernels, as hipFree assumes)
+  (void)hipDeviceSynchronize();
+  for (auto& e : pending) free_blocks.emplace(e.first, e.second);
+  pending.clear();
+  trim();
+}
 void DevCache::clear() {
   trim();
   for (auto& e : pending) (void)hipFree(e.second);

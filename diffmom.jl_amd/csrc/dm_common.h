@@ -47,8 +47,8 @@ struct DmError : std::runtime_error {
 // out again for requests of exactly the same size.  A released block first
 // waits in `pending`: it becomes reusable only once both of the context's
 // streams have been seen idle, so no queued kernel can still touch it.
-// dm_destroy frees everything kept; a failed hipMalloc frees the reusable
-// blocks and retries.
+// dm_destroy frees everything kept; a failed hipMalloc waits for the device,
+// frees all of it and retries.
 // Handles that a caller frees give their memory back to the device, except
 // blocks of up to kFreedBlock bytes, of which kFreedTotal in all are kept (a
 // hipFree costs ~0.2 ms and waits for the device: programs that make and free
@@ -66,6 +66,7 @@ struct DevCache {
   bool give(void* p, size_t b);
   void promote(hipStream_t a, hipStream_t b);  // pending -> reusable when both streams are idle
   void trim();                                 // free the reusable blocks
+  void reclaim();                              // wait for the device, free everything kept
   void clear();                                // free everything
   void forget(void* p, size_t b);              // a kept block leaves the cache
 };
@@ -111,7 +112,7 @@ struct DBuf {
       hipError_t e = hipMalloc(&p, b);
       if (e == hipErrorOutOfMemory && tl_cache) {
         (void)hipGetLastError();
-        tl_cache->trim();
+        tl_cache->reclaim();
         e = hipMalloc(&p, b);
       }
       HIP_OK(e);
