@@ -115,6 +115,7 @@ struct DBuf {
         tl_cache->reclaim();
         e = hipMalloc(&p, b);
       }
+      if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch's check
       HIP_OK(e);
       HIP_OK(hipGetDevice(&dev));
     }
