@@ -1233,7 +1233,8 @@ int dm_farfield(dm_ctx* ctx, const dm_rwg* rwg, const double* rhat, int64_t nome
     const i64 n = r.n;
     DBuf<double> dr, dg, di, de, ws, part;
     dr.upload(rhat, 3 * nomega, s);
-    if (dmf::farfield_direct(ncur)) {
+    const dmf::FfRoute route = dmf::farfield_route(n, nomega, ncur);
+    if (route == dmf::FfRoute::direct) {
       // few currents: straight from the quadrature points
       const i64 chunk = std::min<i64>(nomega, 1 << 16);
       di.alloc((size_t)2 * n * ncur);
@@ -1252,11 +1253,14 @@ int dm_farfield(dm_ctx* ctx, const dm_rwg* rwg, const double* rhat, int64_t nome
       HIP_OK(hipStreamSynchronize(s));
       return;
     }
-    // transverse radiation vectors of a chunk of directions (<= ~1 GiB), then
-    // E = G I on the matrix cores, column by column of currents in blocks of 1024
-    const i64 chunk = std::max<i64>(1, std::min<i64>(std::min<i64>(nomega, 1 << 18), (1LL << 30) / (32 * std::max<i64>(n, 1))));
+    // radiation vectors of a chunk of directions (<= ~1 GiB), all three components
+    // or the transverse two, then E = G I on the matrix cores, column by column of
+    // currents in blocks of 1024
+    const bool full = route == dmf::FfRoute::full;
+    const i64 chunk = std::max<i64>(
+        1, std::min<i64>(std::min<i64>(nomega, 1 << 18), (1LL << 30) / ((full ? 48 : 32) * std::max<i64>(n, 1))));
     const int RB = (int)std::min<i64>(ncur, 1024);
-    dg.alloc((size_t)2 * 2 * chunk * n);
+    dg.alloc((size_t)2 * (full ? 3 : 2) * chunk * n);
     di.alloc((size_t)2 * n * RB);
     de.alloc((size_t)2 * 3 * chunk * RB);
     ws.alloc(dml::gemm_c128_workspace_bytes(n, RB) / sizeof(double));
@@ -1267,9 +1271,15 @@ int dm_farfield(dm_ctx* ctx, const dm_rwg* rwg, const double* rhat, int64_t nome
         const i64 nq = std::min(chunk, nomega - q0);
         {
           ProfScope p(ctx, "radiation", s);
-          dmf::radiation_uv(r, T, dr.p + 3 * q0, nq, k, eta0, dg.p, s);
+          if (full)
+            dmf::radiation_vectors(r, T, dr.p + 3 * q0, nq, k, eta0, dg.p, s);
+          else
+            dmf::radiation_uv(r, T, dr.p + 3 * q0, nq, k, eta0, dg.p, s);
         }
-        {
+        if (full) {
+          ProfScope p(ctx, "farfield_gemm", s);
+          dml::gemm_c128(3 * nq, n, dg.p, 3 * nq, di.p, n, R, de.p, 3 * nq, ws.p, s);
+        } else {
           ProfScope p(ctx, "farfield_gemm", s);
           const int nk = dml::gemm_c128_split(2 * nq, n, R);
           if (part.n < (size_t)2 * nk * 2 * nq * R) part.alloc((size_t)2 * nk * 2 * nq * R);

@@ -256,9 +256,10 @@ __global__ __launch_bounds__(256) void k_ff_join(i64 nomega, int R, int nk, cons
     E[3 * d + c + col * lde] = make_double2(u[c] * a.x + v[c] * b.x, u[c] * a.y + v[c] * b.y);
 }
 
-// Few currents (up to eight): G is never formed; the matrix path costs the same
-// for 1 and for 64 currents (0.77 ms at 7680 bases x 2592 directions).  F[p][r] = the currents' (unnormalised)
-// vector at quadrature point p of every triangle, 3 complex, times its weight;
+// Few currents (up to eight): G is never formed; forming and multiplying it costs
+// the same for 1 and for 64 currents (0.77 ms at 7680 bases x 2592 directions).
+// F[p][r] = the currents' (unnormalised) vector at quadrature point p of every
+// triangle, 3 complex, times its weight;
 // E(r^) = -i k eta0 / (4 pi) (1 - r^ r^) sum_p F[p] exp(i k r^.r_p).
 constexpr int FF_R = dmf::kFfCurrents;  // currents per pass
 constexpr int FF_ROW = 6 * FF_R;  // doubles per point: [current][x, y, z][re, im]
@@ -365,7 +366,27 @@ void launch_rad_uv(const FfArgs& a, int nblk, size_t smem, double* G, hipStream_
 
 namespace dmf {
 
-bool farfield_direct(i64 ncur) { return ncur <= 2 * FF_R; }
+// The lines between the routes, whole calls in us, full / transverse / direct
+// (n x directions):
+//   4 currents   96 x 648 125 / 132 / 146, 280 x 648 159 / 164 / 152,
+//                408 x 32 163 / 169 / 145, 1160 x 648 - / 182 / 175,
+//                2640 x 468 535 / 195 / 205, 4720 x 162 - / 191 / 233,
+//                7701 x 468 1343 / 315 / 288, 7701 x 2592 - / 971 / 418
+//   8 currents   96 x 32 175 / 183 / 263, 736 x 576 306 / 253 / 323,
+//                1160 x 648 - / 263 / 354, 7701 x 1200 1577 / 636 / 636,
+//                4720 x 2160 1159 / 646 / 595, 7701 x 2592 - / 1093 / 848
+//   16 currents  176 x 648 358 / 363 / -, 736 x 432 446 / 394 / -,
+//                7701 x 2592 - / 1322 / 1618
+// Directly, a pass of four currents costs the phases of all points, in waves of 64
+// directions that walk 1/256 of the points each: it pays for one pass unless many
+// points meet few directions, for two only where the phases dominate.  Up to 512
+// bases the product is a single part and the third row costs less than the join.
+FfRoute farfield_route(i64 n, i64 nomega, i64 ncur) {
+  const double pairs = (double)n * (double)nomega;
+  if (ncur <= FF_R && n >= 256 && (n <= 1200 || (nomega >= 256 && pairs >= 1.5e6))) return FfRoute::direct;
+  if (ncur <= 2 * FF_R && nomega >= 1024 && pairs >= 1e7) return FfRoute::direct;
+  return n < 512 ? FfRoute::full : FfRoute::transverse;
+}
 
 // Chunks of points: enough one-wave workgroups to fill the chip (4096), at
 // least 32 points each.

@@ -124,13 +124,15 @@ namespace dmf {
 // written at row out_idx[i] (identity or caller order).
 void planewave(const dm_rwg& r, const TriTables& t, const double* kvec, const double* pol, const double* E0, int M,
                const int* out_idx, double* V, i64 ldv, hipStream_t s);
-// Far fields E = G I (3 nomega x R) of currents in caller order.  Few currents
-// (farfield_direct): directly from the quadrature points, kFfCurrents at a time;
-// more: radiation_uv forms the transverse components of G (2 nomega x n, caller
-// basis order), gemm_c128_parts multiplies, farfield_join adds the partial
-// products and restores x, y, z.
+// Far fields E = G I (3 nomega x R) of currents in caller order, by one of
+//   full         radiation_vectors, then gemm_c128;
+//   transverse   radiation_uv forms the transverse components of G (2 nomega x n,
+//                caller basis order), gemm_c128_parts multiplies, farfield_join adds
+//                the partial products and restores x, y, z;
+//   direct       farfield_few, from the quadrature points, kFfCurrents at a time.
+enum class FfRoute { full, transverse, direct };
 constexpr int kFfCurrents = 4;
-bool farfield_direct(i64 ncur);
+FfRoute farfield_route(i64 n, i64 nomega, i64 ncur);
 size_t farfield_direct_ws(const dm_rwg& r, const TriTables& t, i64 nomega);
 void farfield_few(const dm_rwg& r, const TriTables& t, const double* rhat, i64 nomega, double k, double eta0,
                   const double* I, i64 ldi, int R, double* E, i64 lde, double* ws, hipStream_t s);
