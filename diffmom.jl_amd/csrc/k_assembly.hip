@@ -609,7 +609,7 @@ __device__ inline void tile_coords(int nblk, int& bi, int& bj, bool& valid) {
 //     (triangle of m, triangle of n), which is the order of the pairs themselves
 //     whatever the number of threads.  FP32, where the barriers are hidden by the
 //     CU's other workgroups and plain additions replace the FP32 LDS atomics'
-//     loops (30720 unknowns: 20.8 -> 11.0 ms), and FP64 blocks whose two sums
+//     loops (30720 unknowns: 20.9 -> 10.8 ms), and FP64 blocks whose two sums
 //     do not fit the LDS (20 % slower than PL = 2).
 //   PL = 0: LDS atomics in any order.  The four- and the seven-point rule, whose
 //     two sums do not fit (phases: 7680 unknowns 1.03 -> 1.36 ms and 2.4 -> 2.9),
