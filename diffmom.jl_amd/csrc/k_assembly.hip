@@ -335,7 +335,7 @@ struct TileSide {
   int* nb;      // cap*3 edge neighbours
 };
 
-constexpr int kLater = 128;  // 2 TB: a row's second sum stands kLater rows after its first
+constexpr int kLater = 256;  // > TB
 
 // Rounds p up to 16 bytes as an offset from the 16-byte aligned LDS base:
 // pointer arithmetic keeps the LDS address space visible to the compiler
@@ -603,8 +603,8 @@ __device__ inline void tile_coords(int nblk, int& bi, int& bj, bool& valid) {
 // every time, but for rules where that costs a fifth and more:
 //   PL = 2: two sums per entry, one per triangle of m.  Each gets two terms, added
 //     to zero by LDS atomics in any order (a + b = b + a); the entry is the first
-//     sum plus the second.  30720 unknowns, packed, with the rounding: 12.0 to 12.9 ms
-//     (12.0 to 12.7 with one sum in any order).
+//     sum plus the second.  30720 unknowns, packed, with the rounding: 12.6 ms (12.2
+//     with one sum in any order); 64 plates 1.01 ms (0.99).
 //   PL = 1: every round of pairs adds in phases with a barrier between, by
 //     (triangle of m, triangle of n), which is the order of the pairs themselves
 //     whatever the number of threads.  FP32, where the barriers are hidden by the
@@ -727,7 +727,7 @@ __device__ inline void tile_body(const AsmArgs& a, int cap, AccT* __restrict__ z
       for (int pidx = tid; pidx < npairs; pidx += NTHR) {
         const int i = pidx / nJ;
         pair(lossy, i, pidx - i * nJ, [&](int, int rs, int cs, AccT re, AccT im) {
-          AccT* z = zt + cell(PL == 2 ? rs : rs & (kLater - 1), cs & (kLater - 1));
+          AccT* z = zt + cell(rs & (kLater - 1), cs & (kLater - 1)) + (PL == 2 && rs >= kLater ? 2 * plane : 0);
           atomicAdd(z, re);
           atomicAdd(z + plane, im);
         });
@@ -987,7 +987,7 @@ template <typename T, typename AccT, int MODE, int NTHR>
 void launch_tile_n(const AsmArgs& a, int cap, AccT* z, const double* x, double* y, hipStream_t s) {
   const int pl = tile_planes<T, AccT, MODE>(a.nq, a.TB, cap);
   size_t smem = tile_smem<T, AccT>(a.nq, a.TB, cap, pl == 2 ? 2 : 1);
-  DM_REQUIRE(smem <= kLdsMax && 2 * a.TB == kLater, DM_ERR_ARGUMENT, "tile working set exceeds LDS");
+  DM_REQUIRE(smem <= kLdsMax && a.TB < kLater, DM_ERR_ARGUMENT, "tile working set exceeds LDS");
   i64 T_ = (i64)a.nblk * (a.nblk + 1) / 2;
   i64 grid = ((T_ + 7) / 8) * 8;
   DM_REQUIRE(grid < (1LL << 31), DM_ERR_ARGUMENT, "tile grid too large");
@@ -1008,9 +1008,8 @@ void launch_tile_n(const AsmArgs& a, int cap, AccT* z, const double* x, double* 
   HIP_OK(hipGetLastError());
 }
 
-// FP64: 1024 threads (16 waves, <= 128 VGPRs each) fill the CU that a tile's LDS
-// (90 to 100 KB with one sum per entry, 155 to 160 with two) limits to one
-// workgroup; 512 is the tuner's other candidate.
+// FP64: 1024 threads (16 waves, <= 128 VGPRs each) fill the CU that the ~98 KB
+// of LDS per tile limits to one workgroup; 512 is the tuner's other candidate.
 // FP32: 512.
 template <typename T, typename AccT, int MODE>
 void launch_tile(const AsmArgs& a, int cap, AccT* z, const double* x, double* y, hipStream_t s, int nthr = 0) {
@@ -1034,7 +1033,7 @@ void launch_tile_group(const std::vector<AsmArgs>& args, const std::vector<AccT*
     cap = std::max(cap, args[m].side_cap);
   }
   const size_t smem = tile_smem<T, AccT>(nq, args[0].TB, cap, pl == 2 ? 2 : 1);
-  DM_REQUIRE(smem <= kLdsMax && 2 * args[0].TB == kLater, DM_ERR_ARGUMENT, "tile working set exceeds LDS");
+  DM_REQUIRE(smem <= kLdsMax && args[0].TB < kLater, DM_ERR_ARGUMENT, "tile working set exceeds LDS");
   DM_REQUIRE(cum[nmesh] < (1LL << 31), DM_ERR_ARGUMENT, "too many tiles for one launch");
   DBuf<AsmArgs> dargs;
   DBuf<AccT*> dz;
