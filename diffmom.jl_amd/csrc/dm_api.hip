@@ -166,7 +166,6 @@ AsmArgs make_args_into(dm_rwg& r, const TriTables& T, double kr, double ki, doub
   a.blk_tri = r.d_blk_tri.p;
   a.hrwg = r.d_hrwg.p;
   a.hsig = r.d_hsig.p;
-  a.hlater = r.d_hlater.p;
   a.nb = r.d_nb.p;
   a.ext = r.d_ext.p;
   a.len = r.d_len.p;
@@ -819,6 +818,7 @@ int dm_assemble_z_multi(dm_ctx* ctx, int64_t nmesh, const dm_rwg* const* rwgs, d
     hipStream_t s = ctx->stream;
     std::vector<std::unique_ptr<dm_zmat>> zs(nmesh);
     std::vector<AsmArgs> args(nmesh);
+    int cap = 0;
     // near-field tables of all meshes in one pair of buffers, one overflow flag
     std::vector<i64> toff(nmesh + 1, 0);
     for (i64 m = 0; m < nmesh; ++m) toff[m + 1] = toff[m] + rwgs[m]->mesh->nt;
@@ -847,6 +847,7 @@ int dm_assemble_z_multi(dm_ctx* ctx, int64_t nmesh, const dm_rwg* const* rwgs, d
         args[m] = make_args_into(r, T, k_re, k_im, eta0, z->ld, nt.jself.p + 18 * toff[m], nt.jadj.p + 54 * toff[m],
                                  nt.flag.p, false);
         tabs[m] = &T;
+        cap = std::max(cap, r.max_blk_tris);
         zs[m] = std::move(z);
       }
       // every mesh's near-field tables in one launch per kind
@@ -858,6 +859,31 @@ int dm_assemble_z_multi(dm_ctx* ctx, int64_t nmesh, const dm_rwg* const* rwgs, d
     std::stable_sort(order.begin(), order.end(), [&](i64 a, i64 b) { return args[a].nblk > args[b].nblk; });
     std::vector<AsmArgs> oargs(nmesh);
     for (i64 q = 0; q < nmesh; ++q) oargs[q] = args[order[q]];
+    // the persistent kernel lays out LDS for the largest block; meshes with
+    // smaller blocks get side images built for that layout (kept on the RWG
+    // set per quadrature order and layout, like its own-layout images)
+    for (i64 q = 0; q < nmesh; ++q) {
+      AsmArgs& a = oargs[q];
+      if (a.side_cap == cap) continue;
+      dm_rwg& r = const_cast<dm_rwg&>(*rwgs[order[q]]);
+      std::lock_guard<std::mutex> lk(r.tab_mu);
+      for (int f = 0; f < 2; ++f) {
+        const size_t stride = side_image_bytes(a.nq, f == 1, cap);
+        DBuf<char>& img = r.side_img_cap[{quad_order * 2 + f, cap}];
+        if (!img.p) {
+          img.alloc(stride * a.nblk);
+          launch_build_sides(a, cap, f == 1, img.p, s);
+        }
+        if (f == 1) {
+          a.side_img64 = img.p;
+          a.side_stride64 = (i64)stride;
+        } else {
+          a.side_img32 = img.p;
+          a.side_stride32 = (i64)stride;
+        }
+      }
+      a.side_cap = cap;
+    }
     for (int form : {DM_Z64, DM_Z32, DM_Z64P, DM_Z32P}) {
       if (!(forms & form)) continue;
       std::vector<void*> ptrs(nmesh);
@@ -881,7 +907,7 @@ int dm_assemble_z_multi(dm_ctx* ctx, int64_t nmesh, const dm_rwg* const* rwgs, d
         }
       }
       ProfScope p(ctx, "assemble_multi", s);
-      launch_assemble_multi(oargs, ptrs, form, s);
+      launch_assemble_multi(oargs, ptrs, form, cap, s);
     }
     check_flag(nt, s);
     for (i64 m = 0; m < nmesh; ++m) outs[m] = zs[m].release();

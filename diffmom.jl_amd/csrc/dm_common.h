@@ -310,7 +310,6 @@ struct dm_rwg {
   DBuf<double> d_len;       // n (internal order)
   DBuf<int> d_hrwg;         // nt*3 internal RWG of half (t, e), -1 if none
   DBuf<double> d_hsig;      // nt*3 sign/coefficient of half (t, e)
-  DBuf<char> d_hlater;      // nt*3: t comes after the basis's other triangle in its block's blk_tri
   DBuf<int> d_nb;           // nt*3
   DBuf<int> d_blk_off, d_blk_tri;
   DBuf<int> d_tplus_i, d_tminus_i, d_eplus_i, d_eminus_i;  // internal order, 0-based
@@ -321,6 +320,9 @@ struct dm_rwg {
   std::shared_ptr<SpaiPattern> spai;  // latest pattern; preconditioners keep their own reference
   // tile-side images per quadrature order and precision (built lazily)
   DBuf<char> side_img[8][2];
+  // side images for another mesh's block layout (many-mesh launches), keyed by
+  // (2 x quadrature order + FP64 flag, triangles per block of the layout)
+  std::map<std::pair<int, int>, DBuf<char>> side_img_cap;
   // the matrix buffers of the last dm_solve_scattering_pw that did not hand
   // its matrix to the caller, kept for the next solve on this handle (same
   // sizes: no allocation, no free at the end of the solve); freed with the
@@ -448,7 +450,6 @@ struct AsmArgs {
   const int* blk_tri;
   const int* hrwg;
   const double* hsig;
-  const char* hlater;  // half: its triangle is the basis's second one in blk_tri
   const int* nb;
   const int* ext;
   const double* len;
@@ -495,7 +496,8 @@ void launch_assemble_z32p(const AsmArgs& a, float* z, int max_tris, hipStream_t 
 void zero_packed_padding(i64 n, void* z, size_t scalar_bytes, hipStream_t s);
 // Several meshes' matrices (one stored form) in one persistent launch;
 // packed forms need zeroed buffers.  Synchronises the stream on return.
-void launch_assemble_multi(const std::vector<AsmArgs>& args, const std::vector<void*>& z, int form, hipStream_t s);
+void launch_assemble_multi(const std::vector<AsmArgs>& args, const std::vector<void*>& z, int form, int max_tris,
+                           hipStream_t s);
 // matrix-free y += Z x in internal order (FP64), x and y complex128
 void launch_mf_apply(const AsmArgs& a, const double* x, double* y, int max_tris, hipStream_t s);
 

@@ -412,21 +412,15 @@ void finalize_rwg(dm_rwg& r) {
   r.blk_off.assign(r.nblk + 1, 0);
   r.blk_tri.clear();
   r.max_blk_tris = 0;
-  std::vector<int> mark(nt, -1), place(nt, 0);
-  std::vector<char> hlater(nt * 3, 0);
+  std::vector<int> mark(nt, -1);
   for (int b = 0; b < r.nblk; ++b) {
     i64 i0 = (i64)b * r.TB, i1 = std::min<i64>(n, i0 + r.TB);
     for (i64 i = i0; i < i1; ++i) {
       int e = r.ext_of_int[i];
       for (int s = 0; s < 2; ++s) {
         int t = (int)((s ? r.tminus[e] : r.tplus[e]) - 1);
-        if (mark[t] != b) { mark[t] = b; place[t] = (int)r.blk_tri.size(); r.blk_tri.push_back(t); }
+        if (mark[t] != b) { mark[t] = b; r.blk_tri.push_back(t); }
       }
-    }
-    for (i64 i = i0; i < i1; ++i) {
-      const int e = r.ext_of_int[i];
-      const i64 t0 = r.tplus[e] - 1, t1 = r.tminus[e] - 1;
-      hlater[place[t0] > place[t1] ? 3 * t0 + r.eplus[e] : 3 * t1 + r.eminus[e]] = 1;
     }
     r.blk_off[b + 1] = (int)r.blk_tri.size();
     r.max_blk_tris = std::max(r.max_blk_tris, r.blk_off[b + 1] - r.blk_off[b]);
@@ -462,7 +456,6 @@ void finalize_rwg(dm_rwg& r) {
   pk.add(r.d_len, len_i);
   pk.add(r.d_hrwg, hrwg);
   pk.add(r.d_hsig, hsig);
-  pk.add(r.d_hlater, hlater);
   pk.add(r.d_nb, r.nb);
   pk.add(r.d_blk_off, r.blk_off);
   pk.add(r.d_blk_tri, r.blk_tri);

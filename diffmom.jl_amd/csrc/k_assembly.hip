@@ -330,12 +330,10 @@ struct TileSide {
   T* u;         // cap*NQ*3 quad points - centroid
   T* av;        // cap*9 vertices - centroid
   double* sig;  // cap*3 half sign (0 when the half's basis is outside this block)
-  short* slot;  // cap*3 local basis index in this block (+ kLater on the basis's second triangle of the block), or -1
+  int* slot;    // cap*3 local basis index in this block or -1
   int* gid;     // cap
   int* nb;      // cap*3 edge neighbours
 };
-
-constexpr int kLater = 256;  // > TB
 
 // Rounds p up to 16 bytes as an offset from the 16-byte aligned LDS base:
 // pointer arithmetic keeps the LDS address space visible to the compiler
@@ -351,9 +349,9 @@ __device__ inline char* carve_side(char* base, char* p, int cap, TileSide<T, NQ>
   s.u = reinterpret_cast<T*>(p); p += sizeof(T) * cap * NQ * 3;
   s.av = reinterpret_cast<T*>(p); p += sizeof(T) * cap * 9;
   p = lds_align16(base, p);
+  s.slot = reinterpret_cast<int*>(p); p += sizeof(int) * cap * 3;
   s.gid = reinterpret_cast<int*>(p); p += sizeof(int) * cap;
   s.nb = reinterpret_cast<int*>(p); p += sizeof(int) * cap * 3;
-  s.slot = reinterpret_cast<short*>(p); p += sizeof(short) * cap * 3;
   return lds_align16(base, p);
 }
 
@@ -361,7 +359,7 @@ template <typename T, int NQ>
 __host__ __device__ inline size_t side_bytes(int cap) {
   size_t b = sizeof(double) * cap * 6 + sizeof(T) * cap * (NQ * 3 + 9);
   b = (b + 15) & ~size_t(15);
-  b += (sizeof(int) * 4 + sizeof(short) * 3) * cap;
+  b += sizeof(int) * cap * 7;
   b = (b + 15) & ~size_t(15);
   return b;
 }
@@ -383,7 +381,7 @@ __device__ inline void load_side(const AsmArgs& a, int blk, int nt_side, TileSid
     for (int e = 0; e < 3; ++e) {
       int r = a.hrwg[3 * (i64)g + e];
       int loc = (r >= lo && r < lo + a.TB) ? r - lo : -1;
-      s.slot[3 * i + e] = (short)(loc >= 0 && a.hlater[3 * (i64)g + e] ? loc + kLater : loc);
+      s.slot[3 * i + e] = loc;
       s.sig[3 * i + e] = loc >= 0 ? a.hsig[3 * (i64)g + e] : 0.0;
       s.nb[3 * i + e] = a.nb[3 * (i64)g + e];
     }
@@ -594,50 +592,29 @@ __device__ inline void tile_coords(int nblk, int& bi, int& bj, bool& valid) {
   bi = (int)(l - b * (b + 1) / 2);
 }
 
-// MODE 0: write Z (AccT = storage scalar), MODE 1: matrix-free y += Z x, MODE 2:
-// packed storage.  One tile (bi <= bj) of one mesh: the whole workgroup's work.
-//
-// An entry (m, n) gets four terms, one per triangle of m and triangle of n.  A
-// solve on the complex64 rounding of Z carries a difference in an entry's last
-// bit into the currents at its tolerance, so a stored matrix comes out the same
-// every time, but for rules where that costs a fifth and more:
-//   PL = 2: two sums per entry, one per triangle of m.  Each gets two terms, added
-//     to zero by LDS atomics in any order (a + b = b + a); the entry is the first
-//     sum plus the second.  30720 unknowns, packed, with the rounding: 12.6 ms (12.2
-//     with one sum in any order); 64 plates 1.01 ms (0.99).
-//   PL = 1: every round of pairs adds in phases with a barrier between, by
-//     (triangle of m, triangle of n), which is the order of the pairs themselves
-//     whatever the number of threads.  FP32, where the barriers are hidden by the
-//     CU's other workgroups and plain additions replace the FP32 LDS atomics'
-//     loops (30720 unknowns: 20.9 -> 10.8 ms), and FP64 blocks whose two sums
-//     do not fit the LDS (20 % slower than PL = 2).
-//   PL = 0: LDS atomics in any order.  The four- and the seven-point rule, whose
-//     two sums do not fit (phases: 7680 unknowns 1.03 -> 1.36 ms and 2.4 -> 2.9),
-//     and MODE 1, whose tiles meet in global atomics anyway.
-template <typename T, typename AccT, int NQ, int NTHR, int MODE, int PL>
+// MODE 0: write Z (AccT = storage scalar), MODE 1: matrix-free y += Z x.
+// One tile (bi <= bj) of one mesh: the whole workgroup's work.
+template <typename T, typename AccT, int NQ, int NTHR, int MODE>
 __device__ inline void tile_body(const AsmArgs& a, int cap, AccT* __restrict__ zout, const double* __restrict__ x,
                                  double* __restrict__ y, int bi, int bj) {
   extern __shared__ __align__(16) char smem[];
   const int TB = a.TB;
-  // one element of padding per row, or (to fit the LDS) columns turned by the row,
-  // keeps a wave's reads down a column on all banks
-  const int ldt = PL == 2 ? TB : TB + 1;
-  auto cell = [&](int r, int c) { return r * ldt + (PL == 2 ? c ^ (r & 31) : c); };
+  const int ldt = TB + 1;
   AccT* zt = reinterpret_cast<AccT*>(smem);
-  const int plane = TB * ldt;  // real parts, imaginary parts, the same of the second set
-  char* p = smem + sizeof(AccT) * (PL == 2 ? 4 : 2) * plane;
+  char* p = smem + sizeof(AccT) * 2 * TB * ldt;
   p = lds_align16(smem, p);
   TileSide<T, NQ> R, C;
   p = carve_side<T, NQ>(smem, p, cap, R);
   p = carve_side<T, NQ>(smem, p, cap, C);
-  T* ww = reinterpret_cast<T*>(p);
+  int* extr = reinterpret_cast<int*>(p);
+  int* extc = extr + TB;
+  T* ww = reinterpret_cast<T*>(extc + TB + 2);
   // FP64 phase table (cos, sin of 2 pi j / 256), used by the FP64 far pairs
-  double2* ptab = reinterpret_cast<double2*>(lds_align16(smem, reinterpret_cast<char*>(ww + NQ * NQ)));
+  double2* ptab = reinterpret_cast<double2*>(lds_align16(smem, reinterpret_cast<char*>(ww + 49)));
   const int tid = threadIdx.x;
   const int nI = a.blk_off[bi + 1] - a.blk_off[bi];
   const int nJ = a.blk_off[bj + 1] - a.blk_off[bj];
-  const int zero16 = (int)((sizeof(AccT) * (PL == 2 ? 4 : 2) * plane + 15) / 16);
-  for (int k = tid; k < zero16; k += NTHR) reinterpret_cast<int4*>(smem)[k] = make_int4(0, 0, 0, 0);
+  for (int k = tid; k < 2 * TB * ldt; k += NTHR) zt[k] = (AccT)0;
   {
     // both sides' images are contiguous in LDS (R then C): 16-byte copies
     const i64 stride = sizeof(T) == 8 ? a.side_stride64 : a.side_stride32;
@@ -651,6 +628,11 @@ __device__ inline void tile_body(const AsmArgs& a, int cap, AccT* __restrict__ z
       dr[k] = sr[k];
       dc[k] = sc[k];
     }
+  }
+  for (int k = tid; k < TB; k += NTHR) {
+    i64 gi = (i64)bi * TB + k, gj = (i64)bj * TB + k;
+    extr[k] = gi < a.n ? a.ext[gi] : 0x7fffffff;
+    extc[k] = gj < a.n ? a.ext[gj] : 0x7fffffff;
   }
   if (tid < NQ * NQ) ww[tid] = (T)(a.w[tid / NQ] * a.w[tid % NQ] * INV4PI);
   if constexpr (sizeof(T) == 8) {
@@ -672,113 +654,56 @@ __device__ inline void tile_body(const AsmArgs& a, int cap, AccT* __restrict__ z
   const c2* jadj = reinterpret_cast<const c2*>(a.jadj);
 
   const int npairs = nI * nJ;
-  const int *extr = a.ext + (i64)bi * TB, *extc = a.ext + (i64)bj * TB;
-  // put(3 e + f, row slot, column slot, term) for the pair's terms in this tile
-  auto pair = [&](auto lossy, int i, int j, auto&& put) {
-    const int gi = R.gid[i], gj = C.gid[j];
-    int jn = -1;
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-      if (R.nb[3 * i + k] == gj) jn = k;
-    if (gi == gj || jn >= 0) {
-      // self / edge-adjacent: FP64 table lookup with the caller-order rule
-      int jn2 = 0;
+  auto pair_loop = [&](auto lossy) {
+    for (int pidx = tid; pidx < npairs; pidx += NTHR) {
+      const int i = pidx / nJ;
+      const int j = pidx - i * nJ;
+      const int gi = R.gid[i], gj = C.gid[j];
+      int jn = -1;
 #pragma unroll
       for (int k = 0; k < 3; ++k)
-        if (C.nb[3 * j + k] == gi) jn2 = k;
+        if (R.nb[3 * i + k] == gj) jn = k;
+      if (gi == gj || jn >= 0) {
+        // self / edge-adjacent: FP64 table lookup with the caller-order rule
+        int jn2 = 0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          if (C.nb[3 * j + k] == gi) jn2 = k;
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+          int rs = R.slot[3 * i + e];
+          if (rs < 0) continue;
+#pragma unroll
+          for (int f = 0; f < 3; ++f) {
+            int cs = C.slot[3 * j + f];
+            if (cs < 0) continue;
+            bool fwd = extr[rs] <= extc[cs];
+            c2 v;
+            if (gi == gj)
+              v = fwd ? jself[(i64)gi * 9 + 3 * e + f] : jself[(i64)gi * 9 + 3 * f + e];
+            else
+              v = fwd ? jadj[((i64)gi * 3 + jn) * 9 + 3 * e + f] : jadj[((i64)gj * 3 + jn2) * 9 + 3 * f + e];
+            double s = R.sig[3 * i + e] * C.sig[3 * j + f];
+            atomicAdd(zt + rs * ldt + cs, (AccT)(v.re * s));
+            atomicAdd(zt + TB * ldt + rs * ldt + cs, (AccT)(v.im * s));
+          }
+        }
+        continue;
+      }
+      T Jr[9], Ji[9];
+      far_block<T, NQ, decltype(lossy)::value>(R, i, C, j, ww, ptab, kr, ki, (T)f4r, (T)f4i, Jr, Ji);
 #pragma unroll
       for (int e = 0; e < 3; ++e) {
         int rs = R.slot[3 * i + e];
         if (rs < 0) continue;
+        T sr = (T)R.sig[3 * i + e];
 #pragma unroll
         for (int f = 0; f < 3; ++f) {
           int cs = C.slot[3 * j + f];
           if (cs < 0) continue;
-          bool fwd = extr[rs & (kLater - 1)] <= extc[cs & (kLater - 1)];
-          c2 v;
-          if (gi == gj)
-            v = fwd ? jself[(i64)gi * 9 + 3 * e + f] : jself[(i64)gi * 9 + 3 * f + e];
-          else
-            v = fwd ? jadj[((i64)gi * 3 + jn) * 9 + 3 * e + f] : jadj[((i64)gj * 3 + jn2) * 9 + 3 * f + e];
-          double s = R.sig[3 * i + e] * C.sig[3 * j + f];
-          put(3 * e + f, rs, cs, (AccT)(v.re * s), (AccT)(v.im * s));
-        }
-      }
-      return;
-    }
-    T Jr[9], Ji[9];
-    far_block<T, NQ, decltype(lossy)::value>(R, i, C, j, ww, ptab, kr, ki, (T)f4r, (T)f4i, Jr, Ji);
-#pragma unroll
-    for (int e = 0; e < 3; ++e) {
-      int rs = R.slot[3 * i + e];
-      if (rs < 0) continue;
-      T sr = (T)R.sig[3 * i + e];
-#pragma unroll
-      for (int f = 0; f < 3; ++f) {
-        int cs = C.slot[3 * j + f];
-        if (cs < 0) continue;
-        T s = sr * (T)C.sig[3 * j + f];
-        put(3 * e + f, rs, cs, (AccT)(Jr[3 * e + f] * s), (AccT)(Ji[3 * e + f] * s));
-      }
-    }
-  };
-  auto pair_loop = [&](auto lossy) {
-    if constexpr (PL != 1) {
-      for (int pidx = tid; pidx < npairs; pidx += NTHR) {
-        const int i = pidx / nJ;
-        pair(lossy, i, pidx - i * nJ, [&](int, int rs, int cs, AccT re, AccT im) {
-          AccT* z = zt + cell(rs & (kLater - 1), cs & (kLater - 1)) + (PL == 2 && rs >= kLater ? 2 * plane : 0);
-          atomicAdd(z, re);
-          atomicAdd(z + plane, im);
-        });
-      }
-    } else {
-      constexpr bool fold = sizeof(AccT) == 8;  // (FP32 LDS atomics are loops)
-      for (int p0 = 0; p0 < npairs; p0 += NTHR) {
-        int rs[3], cs[3];
-        AccT wr[9], wi[9];
-        const bool in = p0 + tid < npairs;
-        if (in) {
-          const int i = (p0 + tid) / nJ, j = p0 + tid - i * nJ;
-          pair(lossy, i, j, [&](int ef, int, int, AccT re, AccT im) {
-            wr[ef] = re;
-            wi[ef] = im;
-          });
-#pragma unroll
-          for (int e = 0; e < 3; ++e) {
-            rs[e] = R.slot[3 * i + e];
-            cs[e] = C.slot[3 * j + e];
-          }
-        }
-        auto each = [&](auto&& f9) {
-          if (!in) return;
-#pragma unroll
-          for (int e = 0; e < 3; ++e)
-#pragma unroll
-            for (int f = 0; f < 3; ++f)
-              if (rs[e] >= 0 && cs[f] >= 0)
-                f9((rs[e] >= kLater ? 2 : 0) + (cs[f] >= kLater ? 1 : 0),
-                   zt + cell(rs[e] & (kLater - 1), cs[f] & (kLater - 1)), wr[3 * e + f], wi[3 * e + f]);
-        };
-        each([&](int at, AccT* z, AccT re, AccT im) {
-          if (fold ? at < 2 : at == 0) {
-            if constexpr (fold) {
-              atomicAdd(z, re);
-              atomicAdd(z + plane, im);
-            } else {
-              z[0] += re;
-              z[plane] += im;
-            }
-          }
-        });
-        for (int ph = fold ? 2 : 1; ph < 4; ++ph) {
-          __syncthreads();
-          each([&](int at, AccT* z, AccT re, AccT im) {
-            if (at == ph) {
-              z[0] += re;
-              z[plane] += im;
-            }
-          });
+          T s = sr * (T)C.sig[3 * j + f];
+          atomicAdd(zt + rs * ldt + cs, (AccT)(Jr[3 * e + f] * s));
+          atomicAdd(zt + TB * ldt + rs * ldt + cs, (AccT)(Ji[3 * e + f] * s));
         }
       }
     }
@@ -787,8 +712,6 @@ __device__ inline void tile_body(const AsmArgs& a, int cap, AccT* __restrict__ z
     pair_loop(std::true_type{});
   else
     pair_loop(std::false_type{});
-  // an entry's sum
-  auto entry = [&](int at) { return (double)(PL == 2 ? zt[at] + zt[at + 2 * plane] : zt[at]); };
   const i64 r0 = (i64)bi * TB, c0 = (i64)bj * TB;
   // MODE 1: entry tid of x times its length, rows' then columns' (loaded while
   // the last pairs of other waves are formed)
@@ -811,7 +734,7 @@ __device__ inline void tile_body(const AsmArgs& a, int cap, AccT* __restrict__ z
       if (gr >= a.n || gc >= a.n) continue;
       int rr = r, cc = c;
       if (diag && r > c) { rr = c; cc = r; }
-      double tr = entry(cell(rr, cc)), ti = entry(plane + cell(rr, cc));
+      double tr = (double)zt[rr * ldt + cc], ti = (double)zt[TB * ldt + rr * ldt + cc];
       double l2 = a.len[gr] * a.len[gc];
       double vr = (Pr * tr - Pi * ti) * l2, vi = (Pr * ti + Pi * tr) * l2;
       bad |= !isfinite(vr) || !isfinite(vi);
@@ -824,7 +747,7 @@ __device__ inline void tile_body(const AsmArgs& a, int cap, AccT* __restrict__ z
         int c = k % TB, r = k / TB;
         i64 gr = r0 + r, gc = c0 + c;
         if (gr >= a.n || gc >= a.n) continue;
-        double tr = entry(cell(r, c)), ti = entry(plane + cell(r, c));
+        double tr = (double)zt[r * ldt + c], ti = (double)zt[TB * ldt + r * ldt + c];
         double l2 = a.len[gr] * a.len[gc];
         double vr = (Pr * tr - Pi * ti) * l2, vi = (Pr * ti + Pi * tr) * l2;
         const i64 at = gc + gr * a.ld;
@@ -848,7 +771,7 @@ __device__ inline void tile_body(const AsmArgs& a, int cap, AccT* __restrict__ z
       if (gr >= a.n || gc >= a.n) continue;
       int rr = r, cc = c;
       if (diag && r > c) { rr = c; cc = r; }
-      double tr = entry(cell(rr, cc)), ti = entry(plane + cell(rr, cc));
+      double tr = (double)zt[rr * ldt + cc], ti = (double)zt[TB * ldt + rr * ldt + cc];
       double l2 = a.len[gr] * a.len[gc];
       double vr = (Pr * tr - Pi * ti) * l2, vi = (Pr * ti + Pi * tr) * l2;
       bad |= !isfinite(vr) || !isfinite(vi);
@@ -868,7 +791,7 @@ __device__ inline void tile_body(const AsmArgs& a, int cap, AccT* __restrict__ z
     // lane: the 64 lanes' reads fall on all banks); x in the place of the
     // sides' images.  7680 unknowns: 777 us; one thread per entry, reading x
     // and the lengths term by term: 1048.
-    double2* xs = reinterpret_cast<double2*>(lds_align16(smem, smem + sizeof(AccT) * 2 * plane));
+    double2* xs = reinterpret_cast<double2*>(lds_align16(smem, smem + sizeof(AccT) * 2 * TB * ldt));
     if (tid < 2 * TB) xs[tid] = xl;
     __syncthreads();
     const int l = tid & 7, per = TB / 8;
@@ -881,7 +804,7 @@ __device__ inline void tile_body(const AsmArgs& a, int cap, AccT* __restrict__ z
         const int c = per * l + t;
         int rr = rows ? o : c, cc = rows ? c : o;
         if (diag && rr > cc) { int t2 = rr; rr = cc; cc = t2; }
-        const double tr = entry(cell(rr, cc)), ti = entry(plane + cell(rr, cc));
+        const double tr = (double)zt[rr * ldt + cc], ti = (double)zt[TB * ldt + rr * ldt + cc];
         const double2 xv = xs[rows ? TB + c : c];
         accr += tr * xv.x - ti * xv.y;
         acci += tr * xv.y + ti * xv.x;
@@ -901,23 +824,23 @@ __device__ inline void tile_body(const AsmArgs& a, int cap, AccT* __restrict__ z
   }
 }
 
-template <typename T, typename AccT, int NQ, int NTHR, int MODE, int PL>
+template <typename T, typename AccT, int NQ, int NTHR, int MODE>
 __global__ __launch_bounds__(NTHR) void k_tile(AsmArgs a, int cap, AccT* __restrict__ zout,
                                                 const double* __restrict__ x, double* __restrict__ y) {
   int bi, bj;
   bool valid;
   tile_coords(a.nblk, bi, bj, valid);
   if (!valid) return;
-  tile_body<T, AccT, NQ, NTHR, MODE, PL>(a, cap, zout, x, y, bi, bj);
+  tile_body<T, AccT, NQ, NTHR, MODE>(a, cap, zout, x, y, bi, bj);
 }
 
 // Persistent assembly of several meshes in one launch: workgroup g starts with
 // tile g and takes the next ones from a global counter (which starts at the
 // grid's size) over the concatenated tile lists (meshes in the caller's order,
 // largest first for balance) until all cum[nmesh] tiles are done.
-template <typename T, typename AccT, int NQ, int NTHR, int MODE, int PL>
+template <typename T, typename AccT, int NQ, int NTHR, int MODE>
 __global__ __launch_bounds__(NTHR) void k_tile_multi(const AsmArgs* __restrict__ args, AccT* const* __restrict__ zouts,
-                                                      const i64* __restrict__ cum, int nmesh,
+                                                      const i64* __restrict__ cum, int nmesh, int cap,
                                                       int* __restrict__ counter) {
   __shared__ int item;
   const i64 total = cum[nmesh];
@@ -932,7 +855,7 @@ __global__ __launch_bounds__(NTHR) void k_tile_multi(const AsmArgs* __restrict__
     while (b * (b + 1) / 2 > l) --b;
     while ((b + 1) * (b + 2) / 2 <= l) ++b;
     const AsmArgs& a = args[m];  // read in place: a private copy would live in scratch
-    tile_body<T, AccT, NQ, NTHR, MODE, PL>(a, a.side_cap, zouts[m], nullptr, nullptr, (int)(l - b * (b + 1) / 2), (int)b);
+    tile_body<T, AccT, NQ, NTHR, MODE>(a, cap, zouts[m], nullptr, nullptr, (int)(l - b * (b + 1) / 2), (int)b);
     if (threadIdx.x == 0) item = next;
     __syncthreads();
     w = item;
@@ -954,8 +877,8 @@ __global__ void k_build_sides(AsmArgs a, int cap, char* img, i64 stride) {
 }
 
 template <typename T, typename AccT>
-size_t tile_smem(int nq, int TB, int cap, int planes) {
-  size_t b = sizeof(AccT) * 2 * planes * TB * (planes == 2 ? TB : TB + 1);
+size_t tile_smem(int nq, int TB, int cap) {
+  size_t b = sizeof(AccT) * 2 * TB * (TB + 1);
   b = (b + 15) & ~size_t(15);
   size_t sb = 0;
   switch (nq) {
@@ -965,43 +888,30 @@ size_t tile_smem(int nq, int TB, int cap, int planes) {
     default: sb = side_bytes<T, 7>(cap); break;
   }
   b += 2 * sb;
-  b += sizeof(T) * nq * nq;
+  b += sizeof(int) * (2 * TB + 2) + sizeof(T) * 49;
   if (sizeof(T) == 8) b = ((b + 15) & ~size_t(15)) + sizeof(double) * 2 * 256;  // phase table
   return b;
 }
 
-constexpr size_t kLdsMax = 160 * 1024;
-
-// PL of the tile kernel (see tile_body).  Two sums of the three-point rule fit
-// blocks that touch up to 66 triangles: those of spheres and of square-celled plates
-// touch at most 57, those of plates with long cells up to 66.
-template <typename T, typename AccT, int MODE>
-int tile_planes(int nq, int TB, int cap) {
-  if (MODE == 1) return 0;
-  if (sizeof(T) == 4) return 1;
-  if (nq > 3) return 0;
-  return tile_smem<T, AccT>(nq, TB, cap, 2) + 16 <= kLdsMax ? 2 : 1;  // 16: k_tile_multi's counter
-}
-
 template <typename T, typename AccT, int MODE, int NTHR>
 void launch_tile_n(const AsmArgs& a, int cap, AccT* z, const double* x, double* y, hipStream_t s) {
-  const int pl = tile_planes<T, AccT, MODE>(a.nq, a.TB, cap);
-  size_t smem = tile_smem<T, AccT>(a.nq, a.TB, cap, pl == 2 ? 2 : 1);
-  DM_REQUIRE(smem <= kLdsMax && a.TB < kLater, DM_ERR_ARGUMENT, "tile working set exceeds LDS");
+  size_t smem = tile_smem<T, AccT>(a.nq, a.TB, cap);
+  DM_REQUIRE(smem <= 160 * 1024, DM_ERR_ARGUMENT, "tile working set exceeds LDS");
   i64 T_ = (i64)a.nblk * (a.nblk + 1) / 2;
   i64 grid = ((T_ + 7) / 8) * 8;
   DM_REQUIRE(grid < (1LL << 31), DM_ERR_ARGUMENT, "tile grid too large");
-  auto go = [&](auto kfn) {
-    HIP_OK(hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-    kfn<<<dim3((unsigned)grid), dim3(NTHR), smem, s>>>(a, cap, z, x, y);
-  };
-  constexpr bool f64 = sizeof(T) == 8 && MODE != 1;
-  constexpr int one = MODE == 1 ? 0 : 1, two = f64 ? 2 : one, high = f64 ? 0 : one;  // forms tile_planes gives
   switch (a.nq) {
-    case 1: pl == 2 ? go(k_tile<T, AccT, 1, NTHR, MODE, two>) : go(k_tile<T, AccT, 1, NTHR, MODE, one>); break;
-    case 3: pl == 2 ? go(k_tile<T, AccT, 3, NTHR, MODE, two>) : go(k_tile<T, AccT, 3, NTHR, MODE, one>); break;
-    case 4: go(k_tile<T, AccT, 4, NTHR, MODE, high>); break;
-    case 7: go(k_tile<T, AccT, 7, NTHR, MODE, high>); break;
+#define DM_CASE(NQ)                                                                              \
+  case NQ:                                                                                       \
+    HIP_OK(hipFuncSetAttribute((const void*)k_tile<T, AccT, NQ, NTHR, MODE>,                     \
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));          \
+    k_tile<T, AccT, NQ, NTHR, MODE><<<dim3((unsigned)grid), dim3(NTHR), smem, s>>>(a, cap, z, x, y); \
+    break;
+    DM_CASE(1)
+    DM_CASE(3)
+    DM_CASE(4)
+    DM_CASE(7)
+#undef DM_CASE
     default:
       dm_throw(DM_ERR_ARGUMENT, "unsupported quadrature size");
   }
@@ -1022,18 +932,19 @@ void launch_tile(const AsmArgs& a, int cap, AccT* z, const double* x, double* y,
   }
 }
 
-// Meshes whose tiles take one form of sums (PL) in one launch.
-template <typename T, typename AccT, int MODE, int NTHR>
-void launch_tile_group(const std::vector<AsmArgs>& args, const std::vector<AccT*>& zouts, int pl, int ncu, hipStream_t s) {
-  const int nmesh = (int)args.size(), nq = args[0].nq;
+template <typename T, typename AccT, int MODE>
+void launch_tile_multi(const std::vector<AsmArgs>& args, const std::vector<AccT*>& zouts, int cap, hipStream_t s) {
+  // as in launch_tile; 64 plates, 9262 tiles: 1.37 ms with 512 threads, 1.18 with 1024
+  // (1.11 with the next tile's number fetched ahead)
+  constexpr int NTHR = sizeof(T) == 8 ? 1024 : 512;
+  const int nmesh = (int)args.size();
+  DM_REQUIRE(nmesh >= 1, DM_ERR_ARGUMENT, "no meshes");
+  const int nq = args[0].nq;
+  for (const auto& a : args) DM_REQUIRE(a.nq == nq && a.TB == args[0].TB, DM_ERR_ARGUMENT, "meshes differ in quadrature");
+  size_t smem = tile_smem<T, AccT>(nq, args[0].TB, cap);
+  DM_REQUIRE(smem <= 160 * 1024, DM_ERR_ARGUMENT, "tile working set exceeds LDS");
   std::vector<i64> cum(nmesh + 1, 0);
-  int cap = 0;
-  for (int m = 0; m < nmesh; ++m) {
-    cum[m + 1] = cum[m] + (i64)args[m].nblk * (args[m].nblk + 1) / 2;
-    cap = std::max(cap, args[m].side_cap);
-  }
-  const size_t smem = tile_smem<T, AccT>(nq, args[0].TB, cap, pl == 2 ? 2 : 1);
-  DM_REQUIRE(smem <= kLdsMax && args[0].TB < kLater, DM_ERR_ARGUMENT, "tile working set exceeds LDS");
+  for (int m = 0; m < nmesh; ++m) cum[m + 1] = cum[m] + (i64)args[m].nblk * (args[m].nblk + 1) / 2;
   DM_REQUIRE(cum[nmesh] < (1LL << 31), DM_ERR_ARGUMENT, "too many tiles for one launch");
   DBuf<AsmArgs> dargs;
   DBuf<AccT*> dz;
@@ -1043,60 +954,31 @@ void launch_tile_group(const std::vector<AsmArgs>& args, const std::vector<AccT*
   dz.upload(zouts, s);
   dcum.upload(cum, s);
   counter.alloc(1);
-  auto go = [&](auto kfn) {
-    HIP_OK(hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-    int per_cu = 0;
-    HIP_OK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, NTHR, smem));
-    i64 grid = std::min<i64>(cum[nmesh], (i64)std::max(per_cu, 1) * ncu);
-    k_fill_int<<<1, 1, 0, s>>>(counter.p, (int)grid);
-    kfn<<<dim3((unsigned)grid), dim3(NTHR), smem, s>>>(dargs.p, dz.p, dcum.p, nmesh, counter.p);
-  };
-  // forms tile_planes gives: FP64 two or none with 1024 threads and, of the rules
-  // with few points, phases with 512; FP32 phases with 512
-  constexpr int few = NTHR == 1024 ? 2 : 1, high = NTHR == 1024 ? 0 : 1;
-  constexpr bool all = NTHR == 1024 || sizeof(T) == 4;
-  DM_REQUIRE(all || nq <= 3, DM_ERR_ARGUMENT, "unsupported quadrature size");
+  int dev = 0, ncu = 0;
+  HIP_OK(hipGetDevice(&dev));
+  HIP_OK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   switch (nq) {
-    case 1: go(k_tile_multi<T, AccT, 1, NTHR, MODE, few>); break;
-    case 3: go(k_tile_multi<T, AccT, 3, NTHR, MODE, few>); break;
-    case 4: if constexpr (all) go(k_tile_multi<T, AccT, 4, NTHR, MODE, high>); break;
-    case 7: if constexpr (all) go(k_tile_multi<T, AccT, 7, NTHR, MODE, high>); break;
+#define DM_CASE(NQ)                                                                                        \
+  case NQ: {                                                                                               \
+    auto kfn = k_tile_multi<T, AccT, NQ, NTHR, MODE>;                                                      \
+    HIP_OK(hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem)); \
+    int per_cu = 0;                                                                                        \
+    HIP_OK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, NTHR, smem));                        \
+    i64 grid = std::min<i64>(cum[nmesh], (i64)std::max(per_cu, 1) * ncu);                                  \
+    k_fill_int<<<1, 1, 0, s>>>(counter.p, (int)grid);                                                      \
+    kfn<<<dim3((unsigned)grid), dim3(NTHR), smem, s>>>(dargs.p, dz.p, dcum.p, nmesh, cap, counter.p);      \
+    break;                                                                                                 \
+  }
+    DM_CASE(1)
+    DM_CASE(3)
+    DM_CASE(4)
+    DM_CASE(7)
+#undef DM_CASE
     default:
       dm_throw(DM_ERR_ARGUMENT, "unsupported quadrature size");
   }
   HIP_OK(hipGetLastError());
   HIP_OK(hipStreamSynchronize(s));  // the argument tables are freed on return
-}
-
-template <typename T, typename AccT, int MODE>
-void launch_tile_multi(const std::vector<AsmArgs>& args, const std::vector<AccT*>& zouts, hipStream_t s) {
-  const int nmesh = (int)args.size();
-  DM_REQUIRE(nmesh >= 1, DM_ERR_ARGUMENT, "no meshes");
-  for (const auto& a : args)
-    DM_REQUIRE(a.nq == args[0].nq && a.TB == args[0].TB, DM_ERR_ARGUMENT, "meshes differ in quadrature");
-  int dev = 0, ncu = 0;
-  HIP_OK(hipGetDevice(&dev));
-  HIP_OK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  // a mesh's entries are summed as where it is assembled alone
-  for (int pl : {2, 1, 0}) {
-    std::vector<AsmArgs> ga;
-    std::vector<AccT*> gz;
-    for (int m = 0; m < nmesh; ++m)
-      if (tile_planes<T, AccT, MODE>(args[m].nq, args[m].TB, args[m].side_cap) == pl) {
-        ga.push_back(args[m]);
-        gz.push_back(zouts[m]);
-      }
-    if (ga.empty()) continue;
-    // 64 plates, 9262 tiles: 1.37 ms with 512 threads, 1.18 with 1024 (1.11 with the
-    // next tile's number fetched ahead); the phases' registers spill with 1024
-    if constexpr (sizeof(T) == 8) {
-      if (pl != 1) {
-        launch_tile_group<T, AccT, MODE, 1024>(ga, gz, pl, ncu, s);
-        continue;
-      }
-    }
-    launch_tile_group<T, AccT, MODE, 512>(ga, gz, pl, ncu, s);
-  }
 }
 
 }  // namespace
@@ -1177,21 +1059,22 @@ void launch_mf_apply(const AsmArgs& a, const double* x, double* y, int cap, hipS
   launch_tile<double, double, 1>(a, cap, nullptr, x, y, s);
 }
 
-void launch_assemble_multi(const std::vector<AsmArgs>& args, const std::vector<void*>& z, int form, hipStream_t s) {
+void launch_assemble_multi(const std::vector<AsmArgs>& args, const std::vector<void*>& z, int form, int max_tris,
+                           hipStream_t s) {
   if (form == DM_Z64 || form == DM_Z64P) {
     std::vector<double*> zz;
     for (void* p : z) zz.push_back(static_cast<double*>(p));
     if (form == DM_Z64)
-      launch_tile_multi<double, double, 0>(args, zz, s);
+      launch_tile_multi<double, double, 0>(args, zz, max_tris, s);
     else
-      launch_tile_multi<double, double, 2>(args, zz, s);
+      launch_tile_multi<double, double, 2>(args, zz, max_tris, s);
   } else {
     std::vector<float*> zz;
     for (void* p : z) zz.push_back(static_cast<float*>(p));
     if (form == DM_Z32)
-      launch_tile_multi<float, float, 0>(args, zz, s);
+      launch_tile_multi<float, float, 0>(args, zz, max_tris, s);
     else
-      launch_tile_multi<float, float, 2>(args, zz, s);
+      launch_tile_multi<float, float, 2>(args, zz, max_tris, s);
   }
 }
 
