@@ -135,9 +135,12 @@ void gmres_batch(dm_ctx* ctx, i64 n, int R, DevOp& A, DevPrec* M, const double* 
     // flags every 4 steps (columns that converge in between are masked on
     // the device, so only the Z X of a fully converged batch is wasted).  The
     // round trip costs about 25 us, the steps wasted 1.5 of some 60 on average:
-    // from steps of about 1 ms on (n^2 R = 2e10) the flags are read every step
-    // (30720 unknowns, 128 columns: 15 ms of 720).  The relaxation still
-    // follows the estimates of every fourth.
+    // from steps of about 1 ms on (n^2 R = 2e10) the flags are read every step.
+    // A whole solve in ms, read every step / every fourth (unknowns x columns, n^2 R):
+    //   7680 x 64 (4e9) 38.3 / 37.0, x 128 (8e9) 59.5 / 57.8, x 256 (1.5e10) 109.8 / 107.8,
+    //   12936 x 64 (1.1e10) 70.9 / 71.0, 24120 x 64 (3.7e10) 178 / 180,
+    //   30720 x 128 (1.2e11) 743 / 751.
+    // The relaxation still follows the estimates of every fourth.
     const bool every = (double)n * (double)n * R >= 2e10;
     for (int j = 0; j < mcap && total < maxiter; ++j) {
       double* vj = vblk(K.V.p, j);
