@@ -99,13 +99,19 @@ struct OpZ32 : DevOp {
       planes.alloc(dml::zx_bf16_planes_elems(z->ld, z->n) * 2);
       dml::zx_bf16_split(z->n, z->ld, z->z32.p, planes.p, s);
     }
-    // FP32 accumulation chunk: key zx/c64/<n>/<R>.  4096 columns on every matrix:
-    // a chunk of 8192 is another order of the FP32 sums (9e-8 in the product, up to
-    // 1e-6 in the currents of a lockstep solve), and not faster by more than the
-    // timings scatter: 64 columns of 4143 unknowns 216 / 216 us, 7680: 254 / 430,
-    // 12542: 634 / 595, 30720: 2832 / 2911.
+    // FP32 accumulation chunk: key zx/c64/<n>/<R>.  Another chunk is another order of
+    // the FP32 sums (9e-8 in the product, 2e-6 in the currents of a lockstep solve at
+    // 30720 unknowns, where two runs differ by 1e-6), so no timer chooses it: 4096
+    // columns, 8192 where the products are large.  Eight products in ms, 4096 / 8192
+    // (unknowns x columns, n^2 R):
+    //   9296 x 64 3.1 / 4.0, 10680 x 128 (1.5e10) 4.7 / 5.2, 12545 x 128 (2.0e10) 6.9 / 7.2,
+    //   19040 x 16 7.9 / 9.9, x 64 (2.3e10) 8.6 / 10.4;
+    //   15408 x 128 (3.0e10) 9.6 / 9.7, 24120 x 64 (3.7e10) 14.2 / 15.5,
+    //   19040 x 128 (4.6e10) 15.4 / 15.5, 24120 x 128 25.7 / 26.0, 30720 x 64 22.7 / 23.3.
+    // From 3e10 on a timer took 8192 nearly always, when one chose, and the rule keeps
+    // those results.
     const int kc = dmt::fixed_choice(z->ctx, "zx/c64/" + std::to_string(z->n) + "/" + std::to_string(R),
-                                     dml::zx_bf16_chunks(), 4096);
+                                     dml::zx_bf16_chunks(), (double)z->n * z->n * R >= 3e10 ? 8192 : 4096);
     ProfScope p(z->ctx, nterms == 3 ? "zx_z32_relaxed" : "zx_z32", s);
     dml::zx_bf16(z->n, z->ld, planes.p, X, z->n, R, Y, z->n, ws, s, kc, nterms);
   }
